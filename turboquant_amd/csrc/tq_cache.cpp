@@ -245,9 +245,15 @@ class KvCache {
   // compute_logit_bias (tq.rs:185-253): q [num_q_heads][q_len][head_dim],
   // bias [num_q_heads][q_len][seq_len] in q's dtype
   int logit_bias(int l, const void *q, int q_dtype, int num_q_heads, int q_len, void *bias, hipStream_t stream) {
+    const LayerBuffers &L = storage_.layer(l);
+    if (reinterpret_cast<uintptr_t>(q) % 16 == 0) {  // 16-byte loads of the query rows
+      int rc = sign_matrix(stream);
+      if (rc) return rc;
+      return tqh::query_logit_bias(q, q_dtype, static_cast<const uint32_t *>(rmat_), num_q_heads, q_len, L.signs,
+                                   L.norms, heads_, (int)L.seq, (long long)L.cap, head_dim_, bias, stream);
+    }
     int rc = project(q, q_dtype, (size_t)num_q_heads * q_len, stream);
     if (rc) return rc;
-    const LayerBuffers &L = storage_.layer(l);
     return tq_qjl_logit_bias(static_cast<const float *>(rq_), num_q_heads, q_len, L.signs, L.norms, heads_,
                              (int)L.seq, (long long)L.cap, head_dim_, bias, q_dtype, stream);
   }

@@ -70,6 +70,14 @@ int decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, const
                      long long kv_head_stride, long long seq_stride, float softmax_scale, void *out, int out_dtype,
                      void *workspace, size_t workspace_bytes, hipStream_t stream, const uint32_t *rmat = nullptr);
 
+// compute_logit_bias (tq.rs:185-253) of query rows q [num_q_heads][q_len]
+// [head_dim]: tq_qjl_project and tq_qjl_logit_bias (output in q's type) in one
+// launch, the projection on the matrix cores from exact products.  q on a
+// 16-byte boundary.
+int query_logit_bias(const void *q, int q_dtype, const uint32_t *sign_matrix, int num_q_heads, int q_len,
+                     const uint8_t *signs, const uint16_t *norms, int num_kv_heads, int kv_len, long long head_stride,
+                     int head_dim, void *out, hipStream_t stream);
+
 // fl(1 / fl(sqrt(dim))): the QJL projection's scale (1 / sqrt(d), qjl.rs),
 // each step rounded to f32.
 float inv_sqrt_dim(int dim);

@@ -658,50 +658,6 @@ __global__ __launch_bounds__(kBlock) void qjl_project_kernel(const void *__restr
   for (int m = 0; m < E; m++) rq[row * D + 64 * m + lane] = p[m];
 }
 
-// compute_logit_bias (tq.rs:185-253): bias[h][i][t] = (sum_j rq[h][i][j]
-// (2 b_tj - 1)) * (|r_t| * sf), sf = f32(sqrt(pi/2)) / sqrt(d), for query
-// head h over KV head h / (H / H_kv).  Lane = token; per workgroup QB
-// queries of one head, their +-rq nibble sums in LDS.
-template <int D, int QB>
-__global__ __launch_bounds__(kBlock) void qjl_logit_bias_kernel(const float *__restrict__ rq, int q_len,
-                                                                const uint32_t *__restrict__ signs,
-                                                                const uint16_t *__restrict__ norms, int kv_len,
-                                                                long long head_stride, int n_rep, float sf,
-                                                                void *__restrict__ out, int out_dtype) {
-  constexpr int CT = (D / 4) * 16;
-  __shared__ float s_tab[QB * CT];
-  const int h = blockIdx.z;
-  const int i0 = blockIdx.y * QB;
-  const int nql = min(QB, q_len - i0);
-  for (int e = threadIdx.x; e < nql * CT; e += kBlock) {
-    const int ql = e / CT, rr = e % CT, c = rr / 16, m = rr % 16;
-    const float *rp = rq + (((long long)h * q_len + i0 + ql) * D) + 4 * c;
-    float val = -0.0f;
-#pragma unroll
-    for (int b = 0; b < 4; b++) val = val + (((m >> b) & 1) ? rp[b] : -rp[b]);
-    s_tab[e] = val;
-  }
-  __syncthreads();
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= kv_len) return;
-  const long long rec = (long long)(h / n_rep) * head_stride + t;
-  uint32_t sgn[D / 32];
-#pragma unroll
-  for (int w = 0; w < D / 32; w++) sgn[w] = signs[rec * (D / 32) + w];
-  const float c = f16_to_f32(norms[rec]) * sf;
-  for (int ql = 0; ql < nql; ql++) {
-    const float *tb = s_tab + ql * CT;
-    float raw = 0.0f;
-#pragma unroll
-    for (int cc = 0; cc < D / 4; cc++) raw += tb[cc * 16 + ((sgn[cc >> 3] >> ((cc & 7) * 4)) & 15u)];
-    const float val = raw * c;
-    const long long oi = ((long long)h * q_len + i0 + ql) * kv_len + t;
-    if (out_dtype == kF32) static_cast<float *>(out)[oi] = val;
-    else if (out_dtype == kBF16) static_cast<uint16_t *>(out)[oi] = f32_to_bf16(val);
-    else static_cast<uint16_t *>(out)[oi] = f32_to_f16(val);
-  }
-}
-
 int qjl_consts(int polar_bits, int dim, uint64_t rot_seed, uint64_t qjl_seed, QjlConsts &k) {
   if (dim != 32 && dim != 64 && dim != 128)
     return tqh::fail(TQ_ERR_INVALID_DIMENSION, "QJL kernels take dim 32, 64 or 128 (got %d)", dim);
@@ -953,40 +909,6 @@ extern "C" int tq_qjl_project(const void *q, int q_dtype, const uint32_t *sign_m
     else
       hipLaunchKernelGGL((qjl_project_kernel<D, kF16>), dim3(grid), dim3(kBlock), 0, stream, q, sign_matrix, rq, n, inv);
     return tqh::check_launch("qjl_project_kernel");
-  });
-}
-
-extern "C" float tq_qjl_bias_scale(int head_dim) {
-  // tq.rs:213-214: f32(sqrt(pi / 2)) / sqrt(head_dim as f32)
-  volatile float sp = (float)std::sqrt(3.14159265358979323846 / 2.0);
-  volatile float fd = (float)head_dim;
-  volatile float sq = sqrtf(fd);
-  return sp / sq;
-}
-
-extern "C" int tq_qjl_logit_bias(const float *rq, int num_q_heads, int q_len, const uint8_t *signs_cache,
-                                 const uint16_t *norms_cache, int num_kv_heads, int kv_len,
-                                 long long cache_head_stride, int head_dim, void *out, int out_dtype,
-                                 hipStream_t stream) {
-  int rc = check_sketch_dim(head_dim);
-  if (rc) return rc;
-  if (!tqh::valid_dtype(out_dtype)) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "unknown dtype %d", out_dtype);
-  if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0)
-    return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "num_q_heads (%d) must be a multiple of num_kv_heads (%d)", num_q_heads,
-                     num_kv_heads);
-  if (q_len < 0 || kv_len < 0 || cache_head_stride < kv_len) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "bad shape");
-  if (q_len == 0 || kv_len == 0) return TQ_OK;
-  if (!rq || !signs_cache || !norms_cache || !out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
-  const float sf = tq_qjl_bias_scale(head_dim);
-  const int n_rep = num_q_heads / num_kv_heads;
-  return by_cache_dim(head_dim, [&](auto d) {
-    constexpr int D = decltype(d)::value;
-    constexpr int QB = 8;
-    const dim3 grid((unsigned)((kv_len + kBlock - 1) / kBlock), (unsigned)((q_len + QB - 1) / QB), (unsigned)num_q_heads);
-    hipLaunchKernelGGL((qjl_logit_bias_kernel<D, QB>), grid, dim3(kBlock), 0, stream, rq, q_len,
-                       reinterpret_cast<const uint32_t *>(signs_cache), norms_cache, kv_len, cache_head_stride, n_rep,
-                       sf, out, out_dtype);
-    return tqh::check_launch("qjl_logit_bias_kernel");
   });
 }
 

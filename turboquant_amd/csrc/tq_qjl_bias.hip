@@ -1,0 +1,378 @@
+// tq_qjl_bias.hip -- the TQ cache's logit bias (compute_logit_bias, reference
+// src/cache/tq.rs:185-253) on the matrix cores, with the query projection
+// R q formed in the launch or given by the caller.
+//
+// bias[h][i][t] = (sum_j rq[h][i][j] (2 b_tj - 1)) * (|r_t| * sf), query head
+// h over KV head h / n_rep.  The n_rep q_len query rows that read one KV head
+// are consecutive, so per KV head this is one product of [rows][D] with
+// [D][kv_len], whose right operand is +-1.
+//
+// What bounds it: the output (2 or 4 bytes per row and token against 128
+// useful multiply-adds), so the product has to stay below the store rate.
+// One workgroup makes 64 rows x 512 tokens: the rows are staged once in LDS
+// as two f16 parts (hi = x rounded to f16, lo = the rest rounded to f16, 22
+// to 23 significant bits together, on a power-of-two scale per row), each of
+// its 8 waves expands the sign bits of its 64 tokens once into registers
+// (f16 +-1) and keeps them for all rows.  Both part products are exact in
+// the f32 accumulator.  A lane holds 4 tokens that follow each other for
+// each of its rows, so a wave's store is 128 bytes (16-bit outputs) per row;
+// rows of a kv_len that is no multiple of 4 are stored unaligned (513 x 1537
+// 17.9 us, x 1536 13.3 us, 16 heads).  512 tokens a workgroup instead of 256
+// halve the projection's work per row: 25.2 -> 16.1 us at 16 x 1024 x 1024.
+//
+// Mean of 16 heads x 1024 x 1024 and 16 x 513 x 1537 over 8 KV heads, d =
+// 128, bf16: 49.2 us with one lane per token adding LDS table entries, plus
+// 18.7 us for the projection's own launch, against 18.8 us for both.  Error
+// against f64, f32 output: 2.0e-7 before, 1.1e-7 now (rq's own sum included).
+#include "tq_common.h"
+#include "tq_mfma.h"
+
+#include <cmath>
+
+namespace {
+
+using namespace tqd;
+using namespace tqm;
+
+constexpr int kRows = 64, kThreads = 512, kTokens = kThreads;
+
+// Where the staged rows come from: rq as given (f32), or R q of bf16, f16 or
+// f32 query rows.
+enum Source : int { kGiven = 0, kFromBF16 = 1, kFromF16 = 2, kFromF32 = 3 };
+
+struct BiasArgs {
+  const void *src;        // rq or q, [num_kv_heads][rows][D]
+  const uint32_t *rbits;  // sign bits of R (bit set: -1), for a query source
+  float inv;              // fl(1 / fl(sqrt(D)))
+  int rows;               // query rows per KV head
+  const uint32_t *signs;
+  const uint16_t *norms;
+  int kv_len;
+  long long head_stride;
+  float sf;
+  void *out;
+  int token_blocks;
+};
+
+// The scale 2^-E that brings a row's largest magnitude m into [2^13, 2^14),
+// as the exponent E (m = 0 and tiny rows: clamped; an infinite m takes 114,
+// which keeps every finite element of the row finite in f16).
+__device__ __forceinline__ int row_exponent(float m) {
+  const int e = (int)((f2u(m) >> 23) & 0xffu) - 126;
+  return min(max(e, -100), 128) - 14;
+}
+// x 2^-E as two f16 parts.  An infinity is its own upper part.
+__device__ __forceinline__ void split2(float x, float sc, uint16_t &hi, uint16_t &lo) {
+  const float v = x * sc;
+  hi = f32_to_f16(v);
+  const float h = f16_to_f32(hi);
+  lo = f32_to_f16(h == v ? 0.f : v - h);
+}
+__device__ __forceinline__ uint32_t pair(uint16_t a, uint16_t b) { return (uint32_t)a | ((uint32_t)b << 16); }
+
+// Four values as consecutive elements of type OUT.  Rows of kv_len elements
+// start anywhere, so the store is of unaligned bytes.
+template <int OUT>
+__device__ __forceinline__ void store4(char *p, const float (&v)[4]) {
+  if constexpr (OUT == kF32) {
+    __builtin_memcpy(p, v, 16);
+  } else {
+    const uint2 w = OUT == kBF16 ? make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]))
+                                 : make_uint2(pair(f32_to_f16(v[0]), f32_to_f16(v[1])),
+                                              pair(f32_to_f16(v[2]), f32_to_f16(v[3])));
+    __builtin_memcpy(p, &w, 8);
+  }
+}
+template <int OUT>
+__device__ __forceinline__ void store1(char *p, float v) {
+  if constexpr (OUT == kF32) *reinterpret_cast<float *>(p) = v;
+  else *reinterpret_cast<uint16_t *>(p) = OUT == kBF16 ? f32_to_bf16(v) : f32_to_f16(v);
+}
+
+template <int D, int SRC, int OUT>
+__global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_kernel(BiasArgs a) {
+  constexpr int NS = D / 32, JH = D / 32, TT = 4, OB = OUT == kF32 ? 4 : 2;
+  constexpr int RS = D + 8;  // halves per staged row: 16-byte chunks of 16 rows in different banks
+  __shared__ uint2 s_nib[16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_hi[kRows * RS], s_lo[kRows * RS];
+  __shared__ __attribute__((aligned(16))) float s_scale[kRows];
+  __shared__ float s_max[2][kRows];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int g = blockIdx.z;
+  const int rblk = (int)(blockIdx.x / (unsigned)a.token_blocks), tblk = (int)(blockIdx.x % (unsigned)a.token_blocks);
+  const int r0 = rblk * kRows, nrows = min(kRows, a.rows - r0);
+  const long long row0 = (long long)g * a.rows + r0;
+
+  // the wave's tokens: column l16 of tile T is token t0 + 4 l16 + T
+  const int t0 = tblk * kTokens + wave * 64;
+  uint32_t sw[TT][NS];
+  float c[TT];
+#pragma unroll
+  for (int T = 0; T < TT; T++) {
+    const long long rec = (long long)g * a.head_stride + min(t0 + 4 * l16 + T, a.kv_len - 1);
+#pragma unroll
+    for (int s = 0; s < NS; s++) sw[T][s] = a.signs[rec * NS + s];
+    c[T] = f16_to_f32(a.norms[rec]) * a.sf;
+  }
+  // +-1 in f16 for the four sign bits of a nibble, LSB first (bit set: +1)
+  if (tid < 16) {
+    auto pm1 = [&](int bit) { return ((tid >> bit) & 1) ? 0x3C00u : 0xBC00u; };
+    s_nib[tid] = make_uint2(pm1(0) | (pm1(1) << 16), pm1(2) | (pm1(3) << 16));
+  }
+
+  if constexpr (SRC == kGiven) {
+    // wave w stages rows 8 w .. + 7, D / 4 lanes of 4 elements per row
+    constexpr int LPR = D / 4, RPS = 64 / LPR;
+#pragma unroll
+    for (int step = 0; step < 8 / RPS; step++) {
+      const int row = 8 * wave + step * RPS + lane / LPR, e0 = 4 * (lane % LPR);
+      float x[4] = {0.f, 0.f, 0.f, 0.f};
+      if (row < nrows) {
+        const float *p = static_cast<const float *>(a.src) + (row0 + row) * D + e0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = p[i];
+      }
+      float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+#pragma unroll
+      for (int o = 1; o < LPR; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+      const int e = row_exponent(m);
+      const float sc = exp2i(-e);
+      uint16_t hi[4], lo[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) split2(x[i], sc, hi[i], lo[i]);
+      *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pair(hi[0], hi[1]), pair(hi[2], hi[3]));
+      *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pair(lo[0], lo[1]), pair(lo[2], lo[3]));
+      if (lane % LPR == 0) s_scale[row] = exp2i(e);
+    }
+  } else {
+    // Waves w and w + 4 project rows 16 w .. + 15, each for half of R's
+    // rows j: D[j][row] over 16-row tiles of R as the left operand (+-1,
+    // exact) and the query rows as the right one: a bf16 or f16 query as it
+    // is, an f32 query cut into three bf16 parts that sum to it exactly, so
+    // every product is exact and only the f32 accumulation order differs
+    // from the serial sum of precompute_query_projections (qjl.rs:196-208).
+    constexpr int PARTS = SRC == kFromF32 ? 3 : 1;
+    const int row = 16 * (wave & 3) + l16, jh = wave >> 2;
+    const bool live = 16 * (wave & 3) < nrows;  // uniform
+    f32x4 rq[JH];
+    uint32_t rw[JH][NS];  // R's sign words of row 16 (JH jh + jt) + l16
+    u32x4 q[NS][PARTS];
+    if (live) {
+#pragma unroll
+      for (int jt = 0; jt < JH; jt++)
+#pragma unroll
+        for (int s = 0; s < NS; s++) rw[jt][s] = a.rbits[(16 * (JH * jh + jt) + l16) * NS + s];
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        const long long xi = (row0 + row) * D + 32 * s + 8 * lg;
+        if constexpr (SRC == kFromF32) {
+          float v[8] = {};
+          if (row < nrows) {
+            const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(a.src) + xi);
+            const float4 v0 = p[0], v1 = p[1];
+            v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
+            v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
+          }
+#pragma unroll
+          for (int p = 0; p < 3; p++) {
+            uint32_t cut[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+              cut[j] = f2u(v[j]) & 0xffff0000u;  // the leading 8 significand bits
+              v[j] -= u2f(cut[j]);               // exact: the rest
+            }
+            q[s][p] = u32x4{__builtin_amdgcn_perm(cut[1], cut[0], 0x07060302u),
+                            __builtin_amdgcn_perm(cut[3], cut[2], 0x07060302u),
+                            __builtin_amdgcn_perm(cut[5], cut[4], 0x07060302u),
+                            __builtin_amdgcn_perm(cut[7], cut[6], 0x07060302u)};
+          }
+        } else {
+          q[s][0] = u32x4{0u, 0u, 0u, 0u};
+          if (row < nrows) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(a.src) + xi);
+            q[s][0] = u32x4{v.x, v.y, v.z, v.w};
+          }
+        }
+      }
+    }
+    __syncthreads();  // the nibble table
+    if (live) {
+      float m = 0.f;
+#pragma unroll
+      for (int jt = 0; jt < JH; jt++) {
+        rq[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          const uint32_t byte = (rw[jt][s] >> (8 * lg)) & 0xffu;
+          const uint2 n0 = s_nib[byte & 15u], n1 = s_nib[byte >> 4];
+          // f16 +-1 to bf16 +-1 flips the exponent bits 0x0380
+          constexpr uint32_t F = SRC == kFromF16 ? 0u : 0x03800380u;
+          const u32x4 am = {n0.x ^ F, n0.y ^ F, n1.x ^ F, n1.y ^ F};
+#pragma unroll
+          for (int p = 0; p < PARTS; p++)
+            rq[jt] = SRC == kFromF16 ? mfma(am, q[s][p], rq[jt]) : mfma_bf16(am, q[s][p], rq[jt]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          rq[jt][i] = -rq[jt][i] * a.inv;  // R's set bits are -1, the table's +1
+          m = fmaxf(m, fabsf(rq[jt][i]));
+        }
+      }
+      m = max_xor32(max_xor16(m));
+      if (lg == 0) s_max[jh][row] = m;
+    }
+    __syncthreads();
+    if (live) {
+      const int e = row_exponent(fmaxf(s_max[0][row], s_max[1][row]));
+      const float sc = exp2i(-e);
+#pragma unroll
+      for (int jt = 0; jt < JH; jt++) {
+        uint16_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) split2(rq[jt][i], sc, hi[i], lo[i]);
+        const int at = row * RS + 16 * (JH * jh + jt) + 4 * lg;
+        *reinterpret_cast<uint2 *>(s_hi + at) = make_uint2(pair(hi[0], hi[1]), pair(hi[2], hi[3]));
+        *reinterpret_cast<uint2 *>(s_lo + at) = make_uint2(pair(lo[0], lo[1]), pair(lo[2], lo[3]));
+      }
+      if (jh == 0 && lg == 0) s_scale[row] = exp2i(e);
+    }
+  }
+  __syncthreads();
+  if (t0 >= a.kv_len) return;
+
+  // the tokens' signs as the right operand of every slice
+  u32x4 b[TT][NS];
+#pragma unroll
+  for (int T = 0; T < TT; T++)
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const uint32_t byte = (sw[T][s] >> (8 * lg)) & 0xffu;
+      const uint2 n0 = s_nib[byte & 15u], n1 = s_nib[byte >> 4];
+      b[T][s] = u32x4{n0.x, n0.y, n1.x, n1.y};
+    }
+
+  const int t = t0 + 4 * l16;
+  const long long pitch = (long long)a.kv_len * OB;  // bytes of an output row
+  char *base = static_cast<char *>(a.out) + row0 * pitch;
+  const long long at = 4 * lg * pitch + (long long)t * OB;  // the lane's first row, first token
+#pragma unroll 1
+  for (int rt = 0; 16 * rt < nrows; rt++, base += 16 * pitch) {
+    f32x4 acc[TT];
+#pragma unroll
+    for (int T = 0; T < TT; T++) acc[T] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint16_t *ph = s_hi + (16 * rt + l16) * RS + 8 * lg, *pl = s_lo + (16 * rt + l16) * RS + 8 * lg;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const u32x4 lo = *reinterpret_cast<const u32x4 *>(pl + 32 * s);
+#pragma unroll
+      for (int T = 0; T < TT; T++) acc[T] = mfma(lo, b[T][s], acc[T]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const u32x4 hi = *reinterpret_cast<const u32x4 *>(ph + 32 * s);
+#pragma unroll
+      for (int T = 0; T < TT; T++) acc[T] = mfma(hi, b[T][s], acc[T]);
+    }
+    const float4 s4 = *reinterpret_cast<const float4 *>(s_scale + 16 * rt + 4 * lg);
+    const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
+    const int left = nrows - 16 * rt - 4 * lg;  // rows of this tile that the lane still has
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float v[TT];
+#pragma unroll
+      for (int T = 0; T < TT; T++) v[T] = (acc[T][i] * sc[i]) * c[T];
+      char *p = base + i * pitch + at;
+      if (i < left) {
+        if (t + 4 <= a.kv_len) {
+          store4<OUT>(p, v);
+        } else {
+#pragma unroll
+          for (int T = 0; T < TT; T++)
+            if (t + T < a.kv_len) store1<OUT>(p + T * OB, v[T]);
+        }
+      }
+    }
+  }
+}
+
+template <int D, int SRC, int OUT>
+int launch_one(const BiasArgs &a, dim3 grid, hipStream_t st) {
+  hipLaunchKernelGGL((qjl_logit_bias_kernel<D, SRC, OUT>), grid, dim3(kThreads), 0, st, a);
+  return tqh::check_launch("qjl_logit_bias_kernel");
+}
+
+// Query sources write their own type; rows that were given any.
+template <int D>
+int launch_bias(const BiasArgs &a, int source, int out_dtype, dim3 grid, hipStream_t st) {
+  if (source == kFromF32) return launch_one<D, kFromF32, kF32>(a, grid, st);
+  if (source == kFromBF16) return launch_one<D, kFromBF16, kBF16>(a, grid, st);
+  if (source == kFromF16) return launch_one<D, kFromF16, kF16>(a, grid, st);
+  if (out_dtype == kF32) return launch_one<D, kGiven, kF32>(a, grid, st);
+  if (out_dtype == kBF16) return launch_one<D, kGiven, kBF16>(a, grid, st);
+  return launch_one<D, kGiven, kF16>(a, grid, st);
+}
+
+int bias(const void *src, int source, const uint32_t *rbits, int num_q_heads, int q_len, const uint8_t *signs,
+         const uint16_t *norms, int num_kv_heads, int kv_len, long long head_stride, int head_dim, void *out,
+         int out_dtype, hipStream_t stream) {
+  if (head_dim != 64 && head_dim != 128 && head_dim != 256)
+    return tqh::fail(TQ_ERR_INVALID_DIMENSION, "cache QJL kernels take head_dim 64, 128 or 256 (got %d)", head_dim);
+  if (!tqh::valid_dtype(out_dtype)) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "unknown dtype %d", out_dtype);
+  if (num_kv_heads <= 0 || num_q_heads <= 0 || num_q_heads % num_kv_heads != 0)
+    return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "num_q_heads (%d) must be a multiple of num_kv_heads (%d)", num_q_heads,
+                     num_kv_heads);
+  if (q_len < 0 || kv_len < 0 || head_stride < kv_len) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "bad shape");
+  if (q_len == 0 || kv_len == 0) return TQ_OK;
+  if (!src || !signs || !norms || !out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
+  const long long rows = (long long)(num_q_heads / num_kv_heads) * q_len;
+  const long long tblocks = ((long long)kv_len + kTokens - 1) / kTokens, rblocks = (rows + kRows - 1) / kRows;
+  if (rows > 0x7fffffffll || tblocks * rblocks > 0x7fffffffll)
+    return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many query rows (%lld) for %d tokens", rows, kv_len);
+  BiasArgs a{};
+  a.src = src;
+  a.rbits = rbits;
+  a.inv = tqh::inv_sqrt_dim(head_dim);
+  a.rows = (int)rows;
+  a.signs = reinterpret_cast<const uint32_t *>(signs);
+  a.norms = norms;
+  a.kv_len = kv_len;
+  a.head_stride = head_stride;
+  a.sf = tq_qjl_bias_scale(head_dim);
+  a.out = out;
+  a.token_blocks = (int)tblocks;
+  const dim3 grid((unsigned)(tblocks * rblocks), 1, (unsigned)num_kv_heads);
+  if (head_dim == 64) return launch_bias<64>(a, source, out_dtype, grid, stream);
+  if (head_dim == 128) return launch_bias<128>(a, source, out_dtype, grid, stream);
+  return launch_bias<256>(a, source, out_dtype, grid, stream);
+}
+
+}  // namespace
+
+extern "C" float tq_qjl_bias_scale(int head_dim) {
+  // tq.rs:213-214: f32(sqrt(pi / 2)) / sqrt(head_dim as f32)
+  volatile float sp = (float)std::sqrt(3.14159265358979323846 / 2.0);
+  volatile float fd = (float)head_dim;
+  volatile float sq = sqrtf(fd);
+  return sp / sq;
+}
+
+extern "C" int tq_qjl_logit_bias(const float *rq, int num_q_heads, int q_len, const uint8_t *signs_cache,
+                                 const uint16_t *norms_cache, int num_kv_heads, int kv_len,
+                                 long long cache_head_stride, int head_dim, void *out, int out_dtype,
+                                 hipStream_t stream) {
+  return bias(rq, kGiven, nullptr, num_q_heads, q_len, signs_cache, norms_cache, num_kv_heads, kv_len,
+              cache_head_stride, head_dim, out, out_dtype, stream);
+}
+
+namespace tqh {
+
+int query_logit_bias(const void *q, int q_dtype, const uint32_t *sign_matrix, int num_q_heads, int q_len,
+                     const uint8_t *signs, const uint16_t *norms, int num_kv_heads, int kv_len, long long head_stride,
+                     int head_dim, void *out, hipStream_t stream) {
+  const int source = q_dtype == TQ_DTYPE_F32 ? kFromF32 : q_dtype == TQ_DTYPE_BF16 ? kFromBF16 : kFromF16;
+  return bias(q, source, sign_matrix, num_q_heads, q_len, signs, norms, num_kv_heads, kv_len, head_stride, head_dim,
+              out, q_dtype, stream);
+}
+
+}  // namespace tqh
