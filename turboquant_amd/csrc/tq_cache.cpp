@@ -22,7 +22,9 @@
 
 namespace {
 
+// A layer's buffers: parts of one allocation, each on a 256-byte boundary.
 struct LayerBuffers {
+  void *block = nullptr;
   uint8_t *k_idx = nullptr, *v_idx = nullptr;
   uint16_t *k_sc = nullptr, *v_sc = nullptr;
   uint8_t *signs = nullptr;     // QJL only
@@ -71,44 +73,37 @@ class CompressedStorage {
     if (L.cap >= needed) return TQ_OK;
     const size_t grow = needed / 4 > 128 ? needed / 4 : 128;
     const size_t cap = needed + grow;
-    const size_t ib = (size_t)heads_ * cap * packed_dim(), sb = (size_t)heads_ * cap * num_blocks() * 2;
-    const size_t gb = (size_t)heads_ * cap * sign_bytes(), nb = (size_t)heads_ * cap * 2;
     LayerBuffers N;
     N.cap = cap;
     N.seq = L.seq;
     N.active = L.active;
-    // stream-ordered allocation and release (the device's memory pool): the
-    // old buffers go back to the pool after the work queued before them, so
-    // growth never waits on the host
-    bool ok = pool_alloc(&N.k_idx, ib, stream) && pool_alloc(&N.v_idx, ib, stream) && pool_alloc(&N.k_sc, sb, stream) &&
-              pool_alloc(&N.v_sc, sb, stream);
-    if (ok && qjl_) ok = pool_alloc(&N.signs, gb, stream) && pool_alloc(&N.norms, nb, stream);
-    if (!ok) {
-      free_layer(N, stream);
+    GrowPart part[tqh::kGrowParts];
+    const int np = parts(L, N, part);
+    size_t bytes = 0, at[tqh::kGrowParts];
+    for (int i = 0; i < np; i++) {
+      at[i] = bytes;
+      bytes += ((size_t)heads_ * cap * part[i].rec_bytes + 255) & ~(size_t)255;
+    }
+    // stream-ordered allocation and release (the device's memory pool), one
+    // block per layer (a release costs the host about 12 us): the old block
+    // goes back to the pool after the work queued before it, so growth never
+    // waits on the host
+    if (!pool_alloc(&N.block, bytes, stream))
       return tqh::fail(TQ_ERR_DEVICE, "cache allocation of %zu records per head failed", cap);
+    N.k_idx = static_cast<uint8_t *>(N.block) + at[0];
+    N.v_idx = static_cast<uint8_t *>(N.block) + at[1];
+    N.k_sc = reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(N.block) + at[2]);
+    N.v_sc = reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(N.block) + at[3]);
+    if (qjl_) {
+      N.signs = static_cast<uint8_t *>(N.block) + at[4];
+      N.norms = reinterpret_cast<uint16_t *>(static_cast<uint8_t *>(N.block) + at[5]);
     }
-    // new capacity starts zeroed, as Tensor::zeros
-    ok = hipMemsetAsync(N.k_idx, 0, ib, stream) == hipSuccess && hipMemsetAsync(N.v_idx, 0, ib, stream) == hipSuccess &&
-         hipMemsetAsync(N.k_sc, 0, sb, stream) == hipSuccess && hipMemsetAsync(N.v_sc, 0, sb, stream) == hipSuccess;
-    if (ok && qjl_)
-      ok = hipMemsetAsync(N.signs, 0, gb, stream) == hipSuccess && hipMemsetAsync(N.norms, 0, nb, stream) == hipSuccess;
-    if (!ok) {
+    parts(L, N, part);
+    // the stored rows copied, the new capacity zeroed, as Tensor::zeros
+    const int rc = tqh::grow_layer(part, np, heads_, (long long)L.cap, (long long)cap, (long long)L.seq, stream);
+    if (rc) {
       free_layer(N, stream);
-      return tqh::fail(TQ_ERR_DEVICE, "cache clear failed");
-    }
-    if (L.seq > 0) {
-      auto copy = [&](void *dst, const void *src, size_t rec_bytes) {
-        return hipMemcpy2DAsync(dst, cap * rec_bytes, src, L.cap * rec_bytes, L.seq * rec_bytes, heads_,
-                                hipMemcpyDeviceToDevice, stream) == hipSuccess;
-      };
-      const size_t pi = packed_dim(), ps = (size_t)num_blocks() * 2;
-      ok = copy(N.k_idx, L.k_idx, pi) && copy(N.v_idx, L.v_idx, pi) && copy(N.k_sc, L.k_sc, ps) &&
-           copy(N.v_sc, L.v_sc, ps);
-      if (ok && qjl_) ok = copy(N.signs, L.signs, sign_bytes()) && copy(N.norms, L.norms, 2);
-      if (!ok) {
-        free_layer(N, stream);
-        return tqh::fail(TQ_ERR_DEVICE, "cache growth copy failed");
-      }
+      return rc;
     }
     // queued work may still read the old buffers: they return to the pool in
     // stream order, after it
@@ -140,9 +135,21 @@ class CompressedStorage {
   }
 
  private:
+  using GrowPart = tqh::GrowPart;
+  // the buffers of a layer on growth from `from` to `to`
+  int parts(const LayerBuffers &from, const LayerBuffers &to, GrowPart (&p)[tqh::kGrowParts]) const {
+    const int pi = packed_dim(), ps = num_blocks() * 2;
+    p[0] = {from.k_idx, to.k_idx, pi};
+    p[1] = {from.v_idx, to.v_idx, pi};
+    p[2] = {from.k_sc, to.k_sc, ps};
+    p[3] = {from.v_sc, to.v_sc, ps};
+    if (!qjl_) return 4;
+    p[4] = {from.signs, to.signs, sign_bytes()};
+    p[5] = {from.norms, to.norms, 2};
+    return 6;
+  }
   static void free_layer(LayerBuffers &L, hipStream_t stream) {
-    for (void *p : {(void *)L.k_idx, (void *)L.v_idx, (void *)L.k_sc, (void *)L.v_sc, (void *)L.signs, (void *)L.norms})
-      pool_free(p, stream);
+    pool_free(L.block, stream);
     L = LayerBuffers{};
   }
   void release_all(hipStream_t stream) {

@@ -70,6 +70,19 @@ int decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, const
                      long long kv_head_stride, long long seq_stride, float softmax_scale, void *out, int out_dtype,
                      void *workspace, size_t workspace_bytes, hipStream_t stream, const uint32_t *rmat = nullptr);
 
+// One buffer of a cache layer that grows: [heads][capacity] records of
+// rec_bytes (even), from src (null when nothing is stored) to dst.
+constexpr int kGrowParts = 6;
+struct GrowPart {
+  const void *src = nullptr;
+  void *dst = nullptr;
+  int rec_bytes = 0;
+};
+// Copies the first `rows` records of every head into the new buffers and
+// zeroes the others, one launch for all parts.
+int grow_layer(const GrowPart *parts, int num_parts, int heads, long long old_cap, long long new_cap, long long rows,
+               hipStream_t stream);
+
 // compute_logit_bias (tq.rs:185-253) of query rows q [num_q_heads][q_len]
 // [head_dim]: tq_qjl_project and tq_qjl_logit_bias (output in q's type) in one
 // launch, the projection on the matrix cores from exact products.  q on a
