@@ -195,12 +195,6 @@ class KvCache {
     int rc = storage_.ensure_capacity(l, old + tokens, stream);
     if (rc) return rc;
     const LayerBuffers &L = storage_.layer(l);
-    rc = tq_polar_quantize_to_cache(k, dtype, heads_, tokens, L.k_idx, L.k_sc, (long long)L.cap, (long long)old,
-                                    head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode, stream);
-    if (rc) return rc;
-    rc = tq_polar_quantize_to_cache(v, dtype, heads_, tokens, L.v_idx, L.v_sc, (long long)L.cap, (long long)old,
-                                    head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode, stream);
-    if (rc) return rc;
     if (mode_.qjl) {
       rc = sign_matrix(stream);
       if (rc) return rc;
@@ -208,12 +202,36 @@ class KvCache {
         rc = rq_scratch(num_q_rows, stream);
         if (rc) return rc;
       }
-      rc = tq_qjl_cache_sketch_project(k, dtype, heads_, tokens, L.k_idx, L.k_sc,
-                                       static_cast<const uint32_t *>(rmat_), L.signs, L.norms, (long long)L.cap,
-                                       (long long)old, head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode,
-                                       q, q_dtype, static_cast<float *>(rq_), num_q_rows, stream);
-      if (rc) return rc;
+      tqh::TqAppend a{};
+      a.k = k;
+      a.v = v;
+      a.dtype = dtype;
+      a.num_heads = heads_;
+      a.tokens = tokens;
+      a.k_idx = L.k_idx;
+      a.v_idx = L.v_idx;
+      a.k_sc = L.k_sc;
+      a.v_sc = L.v_sc;
+      a.signs = L.signs;
+      a.norms = L.norms;
+      a.head_stride = (long long)L.cap;
+      a.offset = (long long)old;
+      a.head_dim = head_dim_;
+      a.bits = mode_.bits;
+      a.norm_mode = mode_.norm_mode;
+      a.sign_matrix = static_cast<const uint32_t *>(rmat_);
+      a.q = q;
+      a.q_dtype = q_dtype;
+      a.rq = static_cast<float *>(rq_);
+      a.num_q_rows = num_q_rows;
+      rc = tqh::tq_append(a, stream);
+    } else {
+      if (!v) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
+      rc = tqh::polar_quantize_to_cache(k, v, dtype, heads_, tokens, L.k_idx, L.k_sc, L.v_idx, L.v_sc,
+                                        (long long)L.cap, (long long)old, head_dim_, mode_.bits, mode_.outlier_blocks,
+                                        mode_.norm_mode, stream);
     }
+    if (rc) return rc;
     storage_.set_seq(l, old + tokens);
     return TQ_OK;
   }

@@ -70,6 +70,34 @@ int decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, const
                      long long kv_head_stride, long long seq_stride, float softmax_scale, void *out, int out_dtype,
                      void *workspace, size_t workspace_bytes, hipStream_t stream, const uint32_t *rmat = nullptr);
 
+// tq_polar_quantize_to_cache of x and, unless null, of x2 (the same shape and
+// placement in its own buffers) in one launch per codebook.
+int polar_quantize_to_cache(const void *x, const void *x2, int x_dtype, int num_heads, int tokens, uint8_t *packed,
+                            uint16_t *scales, uint8_t *packed2, uint16_t *scales2, long long head_stride,
+                            long long offset, int head_dim, int bits, size_t outlier_blocks, int norm_mode,
+                            hipStream_t stream);
+
+// A TQ cache's append in one launch: k and v [num_heads][tokens][head_dim]
+// quantized into their records, the sketch of the keys' residuals
+// (tq_qjl_cache_sketch) and, for num_q_rows > 0, rq = R q (tq_qjl_project).
+// The standard codebook (outlier_blocks 0).
+struct TqAppend {
+  const void *k, *v;
+  int dtype, num_heads, tokens;
+  uint8_t *k_idx, *v_idx;
+  uint16_t *k_sc, *v_sc;
+  uint8_t *signs;
+  uint16_t *norms;
+  long long head_stride, offset;
+  int head_dim, bits, norm_mode;
+  const uint32_t *sign_matrix;
+  const void *q;
+  int q_dtype;
+  float *rq;
+  size_t num_q_rows;
+};
+int tq_append(const TqAppend &a, hipStream_t stream);
+
 // One buffer of a cache layer that grows: [heads][capacity] records of
 // rec_bytes (even), from src (null when nothing is stored) to dst.
 constexpr int kGrowParts = 6;
