@@ -1,7 +1,7 @@
 // tq_codec.hip -- core full-vector TurboQuant codec kernels (quantize_vec /
 // dequantize_vec / dequantize_rotated, reference src/quantize.rs:142-316),
-// batched on gfx950: one lane per vector (a lane pair for d = 256), see
-// tq_codec_dev.h.  A wave covers 64 (or 32) consecutive vectors.
+// batched on gfx950: d / 32 lanes per vector, see tq_codec_dev.h.  A wave
+// covers 2048 / d consecutive vectors.
 #include "tq_codec_dev.h"
 
 namespace {
@@ -10,63 +10,65 @@ using namespace tqd;
 
 constexpr int kBlock = 256;
 
-// quantize_vec (quantize.rs:142-157) for `n` vectors of D f32.
+// quantize_vec (quantize.rs:142-157) for `n` vectors of D f32.  Reads 4 D
+// bytes per vector and writes about a tenth of it; small batches are bound by
+// one lane's instructions, large ones by the reads.  10,000 vectors of 128 at
+// 3 bits: 14.3 us with a lane per vector, 5.0 us now.
 template <int D, int BITS>
 __global__ __launch_bounds__(kBlock) void codec_quant_kernel(const float *__restrict__ x, uint8_t *__restrict__ packed,
                                                              uint16_t *__restrict__ scales, long long n,
                                                              CodecConsts k) {
-  using G = Geo<D>;
-  constexpr int E = G::E, LPV = G::LPV;
-  constexpr int NW = E * BITS / 32;            // packed words per lane
-  constexpr int RB = D * BITS / 8;             // packed bytes per vector
-  constexpr int U = StoreUnit<E * BITS / 8>::value;
-  static_assert(RB % U == 0, "row alignment");
+  constexpr int LPV = Geo<D>::LPV;
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   const long long v = t / LPV;
-  const int half = (int)(t % LPV);
-  if (v >= n) return;  // LPV divides kBlock, so lane pairs exit together
-
-  float w[E];
-  {
-    const float4 *p = reinterpret_cast<const float4 *>(x + v * D + half * E);
-#pragma unroll
-    for (int q = 0; q < E / 4; q++) {
-      const float4 f = p[q];
-      w[4 * q] = f.x; w[4 * q + 1] = f.y; w[4 * q + 2] = f.z; w[4 * q + 3] = f.w;
-    }
-  }
-  uint32_t pk[NW];
-  const float norm = quantize_lane<E, LPV, BITS>(w, half, k, pk);
-  store_words<NW, U>(packed + v * RB + half * (E * BITS / 8), pk);
-  if (half == 0) scales[v] = f32_to_f16(norm < kMinNorm ? 0.0f : norm);  // select_scale, quantize.rs:123-126
+  const int q = (int)(t % LPV);
+  if (v >= n) return;  // LPV divides 64: a vector's lanes leave together
+  float w[32];
+  load_elements(x + t * 32, w);
+  uint32_t pk[BITS];
+  const float norm = quantize_lanes<LPV, BITS>(w, q, k, pk);
+  store_codes<BITS>(packed + t * (4 * BITS), pk);
+  if (q == 0) scales[v] = f32_to_f16(norm < kMinNorm ? 0.0f : norm);  // select_scale, quantize.rs:123-126
 }
 
 // dequantize_vec (quantize.rs:225-240) or, ROTATE = false, dequantize_rotated
-// (quantize.rs:306-316).
+// (quantize.rs:306-316).  A wave's 64 lanes make one run of 8 KB: staged
+// through LDS, each store instruction writes 1 KB of it.  10,000 vectors of
+// 128 at 3 bits: 9.9 us (rotated 7.3) with a lane per vector, 4.6 us (3.6) now.
 template <int D, int BITS, bool ROTATE>
 __global__ __launch_bounds__(kBlock) void codec_dequant_kernel(const uint8_t *__restrict__ packed,
                                                                const uint16_t *__restrict__ scales,
                                                                float *__restrict__ out, long long n, CodecConsts k) {
-  using G = Geo<D>;
-  constexpr int E = G::E, LPV = G::LPV;
-  constexpr int NW = E * BITS / 32;
-  constexpr int RB = D * BITS / 8;
-  constexpr int U = StoreUnit<E * BITS / 8>::value;
+  constexpr int LPV = Geo<D>::LPV, RS = 36;  // staged floats per lane, padded
   __shared__ float s_cent[16];
+  __shared__ __attribute__((aligned(16))) float s_out[kBlock / 64][64 * RS];
   if (threadIdx.x < 16) s_cent[threadIdx.x] = k.cent[threadIdx.x & ((1 << BITS) - 1)];
   __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
   const long long v = t / LPV;
-  const int half = (int)(t % LPV);
-  if (v >= n) return;
-
-  uint32_t pk[NW];
-  load_words<NW, U>(packed + v * RB + half * (E * BITS / 8), pk);
-  float w[E];
-  dequant_lane<E, LPV, BITS, ROTATE>(pk, f16_to_f32(scales[v]), half, s_cent, k, w);
-  float4 *o = reinterpret_cast<float4 *>(out + v * D + half * E);
+  const int q = (int)(t % LPV);
+  uint32_t pk[BITS] = {};
+  float sc = 0.f;
+  if (v < n) {  // the others still take part in the wave's staging
+    load_codes<BITS>(packed + t * (4 * BITS), pk);
+    sc = f16_to_f32(scales[v]);
+  }
+  float w[32];
+  dequant_lanes<LPV, BITS, ROTATE>(pk, sc, q, s_cent, k, w);
+  float4 *row = reinterpret_cast<float4 *>(s_out[wave] + lane * RS);
 #pragma unroll
-  for (int q = 0; q < E / 4; q++) o[q] = make_float4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
+  for (int i = 0; i < 8; i++) row[i] = make_float4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const long long t0 = t - lane;  // the wave's first run of 32
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const int f = 256 * i + 4 * lane, r = f / 32;
+    if (t0 + r < n * LPV)
+      *reinterpret_cast<float4 *>(out + t0 * 32 + f) = *reinterpret_cast<const float4 *>(s_out[wave] + r * RS + f % 32);
+  }
 }
 
 template <template <int, int> class Launch, typename A>
@@ -132,7 +134,7 @@ struct DequantLaunch {
   }
 };
 
-constexpr long long kMaxVectors = (1ll << 31) / 2;  // grid.x bound with two lanes per vector
+constexpr long long kMaxVectors = (1ll << 31) / 2;
 
 }  // namespace
 

@@ -1,11 +1,15 @@
 // tq_codec_dev.h -- lane-level core codec (quantize_vec / dequantize_vec,
 // reference src/quantize.rs:142-316) shared by the codec and QJL kernels.
 //
-// One lane owns one vector (a lane pair for d = 256, each holding a half), so
-// the reference's sequential parts stay sequential and bit-exact: the f32 sum
-// of squares runs in element order (quantize.rs:51-53) and the Walsh-Hadamard
-// butterflies run on registers in the reference's stage order
-// (rotation.rs:22-40); only the last stage of d = 256 crosses the pair.
+// A vector is spread over D / 32 neighbouring lanes, 32 elements each, so a
+// lane's straight-line work does not grow with D: with one lane per vector
+// (a pair for d = 256) a quantize of two 256-element vectors took 20.7 us,
+// nearly all of it one wave issuing the 128-element unrolled code.  The
+// reference's sequential parts stay sequential and bit-exact: the f32 sum of
+// squares runs in element order through the lanes (quantize.rs:51-53), and
+// the Walsh-Hadamard stages keep the reference's order (rotation.rs:22-40),
+// those that pair elements of one lane on registers, the last ones across
+// lanes.
 //
 // Bucketize: the reference compares (f64)v > B_k against f64 boundaries
 // (codebook/mod.rs:66-87).  For f32 v that is v >= T_k with T_k the smallest
@@ -16,8 +20,10 @@
 #include "tq_codebooks.h"
 #include "tq_common.h"
 #include "tq_device.h"
+#include "tq_mfma.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace tqd {
 
@@ -32,104 +38,146 @@ struct CodecConsts {
 
 template <int D>
 struct Geo {
-  static constexpr int LPV = D > 128 ? 2 : 1;  // lanes per vector
-  static constexpr int E = D / LPV;            // elements per lane
+  static constexpr int E = 32;       // elements per lane
+  static constexpr int LPV = D / E;  // lanes per vector
 };
 
-// lane ^ 1 (DPP quad_perm [1,0,3,2]).  A DPP read from a lane that is
-// switched off returns 0: call it only where both lanes of the pair are
-// active (never as one arm of a conditional).
-__device__ __forceinline__ float swap_pair(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
-}
-
-template <int BYTES>
-struct StoreUnit {  // widest aligned store unit for a run of BYTES at a BYTES-aligned row offset
-  static constexpr int value = (BYTES % 16 == 0) ? 16 : (BYTES % 8 == 0) ? 8 : 4;
-};
-
-template <int NW, int U>
-__device__ __forceinline__ void store_words(uint8_t *dst, const uint32_t (&w)[NW]) {
-  if constexpr (U == 16) {
-#pragma unroll
-    for (int k = 0; k < NW / 4; k++)
-      reinterpret_cast<uint4 *>(dst)[k] = make_uint4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
-  } else if constexpr (U == 8) {
-#pragma unroll
-    for (int k = 0; k < NW / 2; k++) reinterpret_cast<uint2 *>(dst)[k] = make_uint2(w[2 * k], w[2 * k + 1]);
+// #{t : U[t] <= x} for the 2^BITS - 1 ascending thresholds U: a binary search
+// whose probe at each level is picked from the candidates by the decisions
+// already made (a select tree), BITS compares per element instead of
+// 2^BITS - 1.
+template <int BITS>
+__device__ __forceinline__ uint32_t bucket_sorted(float x, const float (&U)[(1 << BITS) - 1]) {
+  if constexpr (BITS == 2) {
+    const bool b1 = x >= U[1];
+    const bool b0 = x >= (b1 ? U[2] : U[0]);
+    return (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
+  } else if constexpr (BITS == 3) {
+    const bool b2 = x >= U[3];
+    const bool b1 = x >= (b2 ? U[5] : U[1]);
+    const float lo = b1 ? U[2] : U[0], hi = b1 ? U[6] : U[4];
+    const bool b0 = x >= (b2 ? hi : lo);
+    return (b2 ? 4u : 0u) | (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
   } else {
-#pragma unroll
-    for (int k = 0; k < NW; k++) reinterpret_cast<uint32_t *>(dst)[k] = w[k];
+    const bool b3 = x >= U[7];
+    const bool b2 = x >= (b3 ? U[11] : U[3]);
+    const float l1 = b2 ? U[5] : U[1], h1 = b2 ? U[13] : U[9];
+    const bool b1 = x >= (b3 ? h1 : l1);
+    const float a0 = b1 ? U[2] : U[0], a1 = b1 ? U[6] : U[4], a2 = b1 ? U[10] : U[8], a3 = b1 ? U[14] : U[12];
+    const float l0 = b2 ? a1 : a0, h0 = b2 ? a3 : a2;
+    const bool b0 = x >= (b3 ? h0 : l0);
+    return (b3 ? 8u : 0u) | (b2 ? 4u : 0u) | (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
   }
 }
 
-template <int NW, int U>
-__device__ __forceinline__ void load_words(const uint8_t *src, uint32_t (&w)[NW]) {
-  if constexpr (U == 16) {
+// Value of the lane before, inside rows of 16 (DPP row_shr:1).
+__device__ __forceinline__ float lane_before(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x111, 0xF, 0xF, false));
+}
+
+// sum over the vector's elements of sq, in element order from `zero`: lane q
+// continues the sum of lane q - 1, so after LPV rounds the last lane's has
+// run over the whole vector; every lane gets it.  All lanes of a vector take
+// part.
+template <int LPV>
+__device__ __forceinline__ float ordered_sum(const float (&sq)[32], int q, float zero) {
+  float s = zero;
 #pragma unroll
-    for (int k = 0; k < NW / 4; k++) {
-      const uint4 v = reinterpret_cast<const uint4 *>(src)[k];
-      w[4 * k] = v.x; w[4 * k + 1] = v.y; w[4 * k + 2] = v.z; w[4 * k + 3] = v.w;
+  for (int round = 0; round < LPV; round++) {
+    if (round > 0) {
+      const float before = lane_before(s);  // evaluated by every lane
+      s = q == 0 ? zero : before;
     }
-  } else if constexpr (U == 8) {
 #pragma unroll
-    for (int k = 0; k < NW / 2; k++) {
-      const uint2 v = reinterpret_cast<const uint2 *>(src)[k];
-      w[2 * k] = v.x; w[2 * k + 1] = v.y;
+    for (int e = 0; e < 32; e++) s = s + sq[e];
+  }
+  if constexpr (LPV > 1) s = __shfl(s, (int)(threadIdx.x & 63) | (LPV - 1), 64);
+  return s;
+}
+
+// The unnormalized transform of a vector spread over LPV lanes (lane q holds
+// elements 32 q ..), stages in the order of butterfly<D>: h < 32 inside the
+// lanes, h = 32 X between lanes q and q ^ X (the lower takes x + y, the upper
+// x - y).
+template <int LPV>
+__device__ __forceinline__ void butterfly_lanes(float (&w)[32], int q) {
+  butterfly<32>(w);
+  auto cross = [&](auto xc) {
+    constexpr int X = decltype(xc)::value;
+    if constexpr (X < LPV) {
+      const bool upper = (q & X) != 0;
+#pragma unroll
+      for (int e = 0; e < 32; e++) {
+        const float o = tqm::lane_xor<X>(w[e]);
+        w[e] = upper ? o - w[e] : w[e] + o;
+      }
     }
+  };
+  cross(std::integral_constant<int, 1>{});
+  cross(std::integral_constant<int, 2>{});
+  cross(std::integral_constant<int, 4>{});
+}
+
+// A lane's packed words: 32 codes of BITS bits, on 4 BITS-byte boundaries.
+template <int BITS>
+__device__ __forceinline__ void store_codes(uint8_t *dst, const uint32_t (&w)[BITS]) {
+  uint32_t *p = reinterpret_cast<uint32_t *>(dst);
+  if constexpr (BITS == 4) *reinterpret_cast<uint4 *>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+  else if constexpr (BITS == 2) *reinterpret_cast<uint2 *>(p) = make_uint2(w[0], w[1]);
+  else p[0] = w[0], p[1] = w[1], p[2] = w[2];
+}
+template <int BITS>
+__device__ __forceinline__ void load_codes(const uint8_t *src, uint32_t (&w)[BITS]) {
+  const uint32_t *p = reinterpret_cast<const uint32_t *>(src);
+  if constexpr (BITS == 4) {
+    const uint4 v = *reinterpret_cast<const uint4 *>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  } else if constexpr (BITS == 2) {
+    const uint2 v = *reinterpret_cast<const uint2 *>(p);
+    w[0] = v.x; w[1] = v.y;
   } else {
+    w[0] = p[0]; w[1] = p[1]; w[2] = p[2];
+  }
+}
+__device__ __forceinline__ void load_elements(const float *src, float (&w)[32]) {
+  const float4 *p = reinterpret_cast<const float4 *>(src);
 #pragma unroll
-    for (int k = 0; k < NW; k++) w[k] = reinterpret_cast<const uint32_t *>(src)[k];
+  for (int i = 0; i < 8; i++) {
+    const float4 f = p[i];
+    w[4 * i] = f.x; w[4 * i + 1] = f.y; w[4 * i + 2] = f.z; w[4 * i + 3] = f.w;
   }
 }
 
-// Quantizes one lane's E elements of a vector (its half when LPV = 2) into
-// packed words; returns the vector's L2 norm.  `w` is overwritten.
-template <int E, int LPV, int BITS>
-__device__ __forceinline__ float quantize_lane(float (&w)[E], int half, const CodecConsts &k,
-                                               uint32_t (&pk)[E * BITS / 32]) {
-  constexpr int NB = (1 << BITS) - 1;
+// Quantizes lane q's 32 elements of a vector into packed words; returns the
+// vector's L2 norm.  `w` is overwritten.
+template <int LPV, int BITS>
+__device__ __forceinline__ float quantize_lanes(float (&w)[32], int q, const CodecConsts &k, uint32_t (&pk)[BITS]) {
   // l2_norm: f32 sum of squares in element order, from -0.0 (Rust's f32 sum)
-  float norm;
-  {
-    float s = -0.0f;
+  float sq[32];
 #pragma unroll
-    for (int e = 0; e < E; e++) s = s + w[e] * w[e];
-    if constexpr (LPV == 2) {
-      float s1 = swap_pair(s);  // the upper half continues from the lower half's sum
-#pragma unroll
-      for (int e = 0; e < E; e++) s1 = s1 + w[e] * w[e];
-      const float u = swap_pair(s1);  // evaluated by both lanes of the pair
-      s = half ? s1 : u;
-    }
-    norm = sqrtf(s);
-  }
+  for (int e = 0; e < 32; e++) sq[e] = w[e] * w[e];
+  const float norm = sqrtf(ordered_sum<LPV>(sq, q, -0.0f));
   // normalize_inplace (quantize.rs:60-71), then Forward rotation: sign, WHT
   if (norm < kMinNorm) {
 #pragma unroll
-    for (int e = 0; e < E; e++) w[e] = 0.0f;
+    for (int e = 0; e < 32; e++) w[e] = 0.0f;
   } else {
     const float inv = 1.0f / norm;
 #pragma unroll
-    for (int e = 0; e < E; e++) w[e] = w[e] * inv;
+    for (int e = 0; e < 32; e++) w[e] = w[e] * inv;
   }
-  const float se = k.sign_even, so = -k.sign_even;  // E is even: parity of element = parity of e
+  const float se = k.sign_even, so = -k.sign_even;  // 32 q is even: parity of element = parity of e
 #pragma unroll
-  for (int e = 0; e < E; e++) w[e] = w[e] * ((e & 1) ? so : se);
-  butterfly<E>(w);
-  if constexpr (LPV == 2) {  // stage h = E across the pair: lower x + y, upper x - y
-    const float sg = half ? -1.0f : 1.0f;
+  for (int e = 0; e < 32; e++) w[e] = w[e] * ((e & 1) ? so : se);
+  butterfly_lanes<LPV>(w, q);
+  float thr[(1 << BITS) - 1];
 #pragma unroll
-    for (int e = 0; e < E; e++) w[e] = swap_pair(w[e]) + w[e] * sg;
-  }
+  for (int b = 0; b < (1 << BITS) - 1; b++) thr[b] = k.thr[b];
 #pragma unroll
-  for (int i = 0; i < E * BITS / 32; i++) pk[i] = 0u;
+  for (int i = 0; i < BITS; i++) pk[i] = 0u;
 #pragma unroll
-  for (int e = 0; e < E; e++) {
-    const float r = w[e] * k.wht_norm;
-    uint32_t idx = 0;
-#pragma unroll
-    for (int b = 0; b < NB; b++) idx += (r >= k.thr[b]) ? 1u : 0u;
+  for (int e = 0; e < 32; e++) {
+    const uint32_t idx = bucket_sorted<BITS>(w[e] * k.wht_norm, thr);
     const int bit = e * BITS, wi = bit >> 5, sh = bit & 31;
     pk[wi] |= idx << sh;
     if (sh + BITS > 32) pk[wi + 1] |= idx >> (32 - sh);
@@ -137,32 +185,22 @@ __device__ __forceinline__ float quantize_lane(float (&w)[E], int half, const Co
   return norm;
 }
 
-// Dequantizes one lane's E elements: centroid lookup (s_cent in LDS), then,
+// Dequantizes lane q's 32 elements: centroid lookup (s_cent in LDS), then,
 // with ROTATE, the inverse rotation (WHT with its normalization, then sign,
 // rotation.rs:137-150); finally times the f32 scale.
-template <int E, int LPV, int BITS, bool ROTATE>
-__device__ __forceinline__ void dequant_lane(const uint32_t (&pk)[E * BITS / 32], float sc, int half,
-                                             const float *s_cent, const CodecConsts &k, float (&w)[E]) {
+template <int LPV, int BITS, bool ROTATE>
+__device__ __forceinline__ void dequant_lanes(const uint32_t (&pk)[BITS], float sc, int q, const float *s_cent,
+                                              const CodecConsts &k, float (&w)[32]) {
 #pragma unroll
-  for (int e = 0; e < E; e++) {
-    const int bit = e * BITS, wi = bit >> 5, sh = bit & 31;
-    uint32_t idx = pk[wi] >> sh;
-    if (sh + BITS > 32) idx |= pk[wi + 1] << (32 - sh);
-    w[e] = s_cent[idx & ((1u << BITS) - 1u)];
-  }
+  for (int e = 0; e < 32; e++) w[e] = s_cent[field<BITS>(pk, e)];
   if constexpr (ROTATE) {
-    butterfly<E>(w);
-    if constexpr (LPV == 2) {
-      const float sg = half ? -1.0f : 1.0f;
-#pragma unroll
-      for (int e = 0; e < E; e++) w[e] = swap_pair(w[e]) + w[e] * sg;
-    }
+    butterfly_lanes<LPV>(w, q);
     const float se = k.sign_even, so = -k.sign_even;
 #pragma unroll
-    for (int e = 0; e < E; e++) w[e] = (w[e] * k.wht_norm) * ((e & 1) ? so : se);
+    for (int e = 0; e < 32; e++) w[e] = (w[e] * k.wht_norm) * ((e & 1) ? so : se);
   }
 #pragma unroll
-  for (int e = 0; e < E; e++) w[e] = w[e] * sc;
+  for (int e = 0; e < 32; e++) w[e] = w[e] * sc;
 }
 
 }  // namespace tqd

@@ -3,11 +3,10 @@
 // query projections, batched score estimation, softmax and weighted values.
 //
 // The Rademacher matrix R[j][c] = sign(j, c) / sqrt(d) is implicit in the
-// reference (a SplitMix64 hash per entry, qjl.rs:143-189).  Each workgroup
-// hashes the d x d sign bits it needs into LDS once; a lane then forms a row
-// product as d fused multiply-adds with a wave-uniform +-1 factor, which is
-// exactly the reference's sequential sum of sign * value (the product is
-// exact, so fma(sign, v, s) == fl(s + sign * v)).
+// reference (a SplitMix64 hash per entry, qjl.rs:143-189).  A workgroup hashes
+// the sign bits it needs; a row product is d fused multiply-adds with a +-1
+// factor in column order, which is exactly the reference's sequential sum of
+// sign * value (the product is exact, so fma(sign, v, s) == fl(s + sign * v)).
 //
 // Scores use the rotated domain: <q, x_mse> = scale * <qt, c[idx]> with
 // qt = H(s * q) / sqrt(d), the forward rotation of the query, so keys are
@@ -32,40 +31,16 @@ __device__ __forceinline__ uint64_t mix_seed(uint64_t seed, uint64_t row) {
   return m ^ (m >> 32) ^ 0x6C62272E07BB0142ull;
 }
 
-// qjl.rs:157-171: true where sign(row, col) = -1 (SplitMix64 finalizer odd)
-__device__ __forceinline__ bool sign_negative(uint64_t row_seed, uint64_t row, uint64_t col) {
-  uint64_t z = row_seed + row * kGolden + col;
+// qjl.rs:157-171: true where sign(row, col) = -1 (SplitMix64 finalizer odd),
+// base = row_seed + row * golden.  Only bits 0 and 31 of the last product
+// reach the parity, so its low word is enough.
+__device__ __forceinline__ bool sign_negative(uint64_t base, uint32_t col) {
+  uint64_t z = base + col;
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  z ^= z >> 31;
-  return (z & 1u) != 0;
+  const uint32_t p = (uint32_t)(z ^ (z >> 27)) * 0x133111EBu;
+  return ((p ^ (p >> 31)) & 1u) != 0;
 }
-
-// Fills s_bits[j * D/32 + w] (bit b = sign(j, 32w + b) is -1) for all rows.
-template <int D>
-__device__ void build_sign_bits(uint32_t *s_bits, uint64_t seed) {
-  for (int it = threadIdx.x; it < D * D / 32; it += blockDim.x) {
-    const int j = it / (D / 32), w = it % (D / 32);
-    const uint64_t rs = mix_seed(seed, (uint64_t)j);
-    uint32_t bits = 0;
-    for (int b = 0; b < 32; b++) bits |= (sign_negative(rs, (uint64_t)j, (uint64_t)(32 * w + b)) ? 1u : 0u) << b;
-    s_bits[it] = bits;
-  }
-}
-
-// rademacher_vector_product (qjl.rs:196-208): (sum_c sign(j,c) * v[c]) * inv,
-// summed in column order from -0.0.
-template <int D>
-__device__ __forceinline__ float row_product(const float (&v)[D], const uint32_t *row_bits, float inv) {
-  float s = -0.0f;
-#pragma unroll
-  for (int w = 0; w < D / 32; w++) {
-    const uint32_t bits = __builtin_amdgcn_readfirstlane(row_bits[w]);
-#pragma unroll
-    for (int b = 0; b < 32; b++) s = __builtin_fmaf(((bits >> b) & 1u) ? -1.0f : 1.0f, v[32 * w + b], s);
-  }
-  return s * inv;
-}
+__device__ __forceinline__ uint64_t sign_base(uint64_t seed, uint64_t row) { return mix_seed(seed, row) + row * kGolden; }
 
 struct QjlConsts {
   CodecConsts polar;   // (total_bits - 1)-bit codec of the same dimension
@@ -80,107 +55,90 @@ __device__ __forceinline__ float4 nibble_signs(int nib) {
                      (nib & 8) ? -1.0f : 1.0f);
 }
 
-// quantize_with_qjl (qjl.rs:355-377) for KB = 32 keys per workgroup.  One lane
-// of each group of 8 quantizes its key (polar codes, scale, residual r = x -
-// dequantized x, |r|) and stages r in LDS; then the 8 lanes of the key share
-// its D sign projections, D / 8 rows each.  A row is summed in column order
-// from -0.0 exactly as rademacher_vector_product (qjl.rs:196-208): the signs
-// of four columns come from one table read by the nibble of the row's bits,
-// and fma(+-1, r_c, s) is the reference's fl(s + sign * r_c).  Four rows at a
-// time keep four independent sums in flight.
+// quantize_with_qjl (qjl.rs:355-377) for 32 keys per workgroup of D / 16
+// waves.  D / 32 lanes of a key quantize it (polar codes, scale, residual r =
+// x - dequantized x, |r|) and stage r in LDS; meanwhile every wave hashes the
+// signs of its 16 rows of R straight into the lanes that use them; then it
+// sums those rows for the 32 keys on the matrix cores.  A row is summed in
+// column order from -0.0 as rademacher_vector_product does (qjl.rs:196-208):
+// v_mfma_f32_16x16x4_f32 adds its four products one after the other in k
+// order, each step one fused multiply-add (checked on MI355X against fmaf
+// chains), and fma(+-1, r_c, s) is the reference's fl(s + sign * r_c).
+//
+// Bound by the instructions of one workgroup: 32 hashes a lane, the codec of
+// 32 elements, 2 x 32 matrix steps of 32 cycles.  8,192 keys of d = 128, 3
+// bits: 36.2 us with the codec on one lane per key, all of R hashed into LDS
+// by every workgroup and the sums on the vector unit; 11.1 us now.
 template <int D, int PB>
-__global__ __launch_bounds__(kBlock) void qjl_quant_kernel(const float *__restrict__ x, uint8_t *__restrict__ polar,
-                                                           uint16_t *__restrict__ polar_scales,
-                                                           uint32_t *__restrict__ signs,
-                                                           uint16_t *__restrict__ residual_norms, long long n,
-                                                           QjlConsts k) {
-  constexpr int LPK = 8, KB = kBlock / LPK, RPL = D / LPK, RI = RPL < 4 ? RPL : 4;
-  constexpr int NW = D * PB / 32;
-  constexpr int U = StoreUnit<D * PB / 8>::value;
-  constexpr int RS = D + 4;  // residual row stride (floats): rows of different keys in different banks
-  __shared__ uint32_t s_bits[D * D / 32];
+__global__ __launch_bounds__(4 * D) void qjl_quant_kernel(const float *__restrict__ x, uint8_t *__restrict__ polar,
+                                                          uint16_t *__restrict__ polar_scales,
+                                                          uint16_t *__restrict__ signs,
+                                                          uint16_t *__restrict__ residual_norms, long long n,
+                                                          QjlConsts k) {
+  constexpr int KB = 32, LPV = D / 32, RS = D + 4;  // floats per staged row: the sums' reads hit 64 banks
   __shared__ float s_cent[16];
   __shared__ __attribute__((aligned(16))) float s_res[KB * RS];
-  __shared__ __attribute__((aligned(16))) float4 s_sgn[16];
-  __shared__ uint32_t s_sw[KB * (D / 32)];
-  build_sign_bits<D>(s_bits, k.qjl_seed);
-  const int tid = threadIdx.x, kk = tid / LPK, rq = tid % LPK;
-  if (tid < 16) {
-    s_cent[tid] = k.polar.cent[tid & ((1 << PB) - 1)];
-    s_sgn[tid] = nibble_signs(tid);
-  }
-  for (int e = tid; e < KB * (D / 32); e += kBlock) s_sw[e] = 0u;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const long long key0 = (long long)blockIdx.x * KB;
+  const long long v = key0 + tid / LPV;
+  const int q = tid % LPV;
+  const bool live = tid < KB * LPV && v < n;
+  float w[32];
+  if (live) load_elements(x + v * D + 32 * q, w);
+  if (tid < 16) s_cent[tid] = k.polar.cent[tid & ((1 << PB) - 1)];
+  // bit i: sign of (row 16 wave + l16, column 4 i + lg) is -1
+  uint32_t rb = 0;
+  const uint64_t base = sign_base(k.qjl_seed, (uint64_t)(16 * wave + l16));
+#pragma unroll 8
+  for (int i = 0; i < D / 4; i++) rb |= (sign_negative(base, (uint32_t)(4 * i + lg)) ? 1u : 0u) << i;
   __syncthreads();
-  const long long v = (long long)blockIdx.x * KB + kk;
-  const bool live = v < n;
-  if (rq == 0 && live) {
-    const float4 *xp = reinterpret_cast<const float4 *>(x + v * D);
-    float w[D];
+  if (live) {
+    float r[32];
 #pragma unroll
-    for (int q = 0; q < D / 4; q++) {
-      const float4 f = xp[q];
-      w[4 * q] = f.x; w[4 * q + 1] = f.y; w[4 * q + 2] = f.z; w[4 * q + 3] = f.w;
-    }
-    uint32_t pk[NW];
-    const float norm = quantize_lane<D, 1, PB>(w, 0, k.polar, pk);
+    for (int e = 0; e < 32; e++) r[e] = w[e];
+    uint32_t pk[PB];
+    const float norm = quantize_lanes<LPV, PB>(w, q, k.polar, pk);
     const uint16_t sc = f32_to_f16(norm < kMinNorm ? 0.0f : norm);
+    store_codes<PB>(polar + (v * LPV + q) * (4 * PB), pk);
     // x_mse = dequantize_vec(polar block), residual r = x - x_mse (qjl.rs:362-368)
-    dequant_lane<D, 1, PB, true>(pk, f16_to_f32(sc), 0, s_cent, k.polar, w);
+    dequant_lanes<LPV, PB, true>(pk, f16_to_f32(sc), q, s_cent, k.polar, w);
 #pragma unroll
-    for (int q = 0; q < D / 4; q++) {
-      const float4 f = xp[q];
-      w[4 * q] = f.x - w[4 * q]; w[4 * q + 1] = f.y - w[4 * q + 1];
-      w[4 * q + 2] = f.z - w[4 * q + 2]; w[4 * q + 3] = f.w - w[4 * q + 3];
+    for (int e = 0; e < 32; e++) r[e] = r[e] - w[e];
+    float4 *dst = reinterpret_cast<float4 *>(s_res + (tid / LPV) * RS + 32 * q);
+#pragma unroll
+    for (int i = 0; i < 8; i++) dst[i] = make_float4(r[4 * i], r[4 * i + 1], r[4 * i + 2], r[4 * i + 3]);
+#pragma unroll
+    for (int e = 0; e < 32; e++) r[e] = r[e] * r[e];
+    const float rs = ordered_sum<LPV>(r, q, -0.0f);
+    if (q == 0) {
+      polar_scales[v] = sc;
+      residual_norms[v] = f32_to_f16(sqrtf(rs));
     }
-    float rs = -0.0f;
-#pragma unroll
-    for (int e = 0; e < D; e++) rs = rs + w[e] * w[e];
-#pragma unroll
-    for (int q = 0; q < D / 4; q++)
-      *reinterpret_cast<float4 *>(s_res + kk * RS + 4 * q) = make_float4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
-    store_words<NW, U>(polar + v * (D * PB / 8), pk);
-    polar_scales[v] = sc;
-    residual_norms[v] = f32_to_f16(sqrtf(rs));
   }
   __syncthreads();
   // compute_qjl_signs + pack_sign_bits (qjl.rs:305-319, 245-256): bit j = p_j >= 0
-  if (live) {
-    const float4 *res = reinterpret_cast<const float4 *>(s_res + kk * RS);
-    uint32_t mine = 0u;  // bits of rows rq * RPL .. + RPL, at their place in the row's word
+  tqm::f32x4 acc[2];
 #pragma unroll
-    for (int r0 = 0; r0 < RPL; r0 += RI) {
-      const int j0 = rq * RPL + r0;
-      float sum[RI];
+  for (int g = 0; g < 2; g++) acc[g] = tqm::f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
+  const float *res = s_res + l16 * RS + lg;
 #pragma unroll
-      for (int i = 0; i < RI; i++) sum[i] = -0.0f;
+  for (int i = 0; i < D / 4; i++) {
+    const float a = u2f(((rb << (31 - i)) & 0x80000000u) | 0x3f800000u);
 #pragma unroll
-      for (int w = 0; w < D / 32; w++) {
-        uint32_t bw[RI];
-#pragma unroll
-        for (int i = 0; i < RI; i++) bw[i] = s_bits[(j0 + i) * (D / 32) + w];
-#pragma unroll
-        for (int nb = 0; nb < 8; nb++) {
-          const float4 rv = res[8 * w + nb];
-#pragma unroll
-          for (int i = 0; i < RI; i++) {
-            const float4 sg = s_sgn[(bw[i] >> (4 * nb)) & 15u];
-            sum[i] = __builtin_fmaf(sg.x, rv.x, sum[i]);
-            sum[i] = __builtin_fmaf(sg.y, rv.y, sum[i]);
-            sum[i] = __builtin_fmaf(sg.z, rv.z, sum[i]);
-            sum[i] = __builtin_fmaf(sg.w, rv.w, sum[i]);
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < RI; i++) {
-        const float p = sum[i] * k.inv_sqrt_d;
-        mine |= (p >= 0.0f ? 1u : 0u) << ((j0 + i) & 31);
-      }
-    }
-    if (mine) atomicOr(&s_sw[kk * (D / 32) + (rq * RPL) / 32], mine);
+    for (int g = 0; g < 2; g++)
+      acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, res[16 * g * RS + 4 * i], acc[g], 0, 0, 0);
   }
-  __syncthreads();
-  if (live && rq < D / 32) signs[v * (D / 32) + rq] = s_sw[kk * (D / 32) + rq];
+#pragma unroll
+  for (int g = 0; g < 2; g++) {  // lane: key l16 of the group, rows 4 lg .. + 3 of the wave's 16
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) bits |= (acc[g][i] * k.inv_sqrt_d >= 0.0f ? 1u : 0u) << (4 * lg + i);
+    bits |= __shfl_xor(bits, 16, 64);
+    bits |= __shfl_xor(bits, 32, 64);
+    const long long key = key0 + 16 * g + l16;
+    if (lg == 0 && key < n) signs[key * (D / 16) + wave] = (uint16_t)bits;
+  }
 }
 
 // EstimationContext for a batch of queries (qjl.rs:488-492, 561-572):
@@ -204,7 +162,7 @@ __global__ __launch_bounds__(kBlock) void qjl_query_kernel(const float *__restri
   // gathered into two words by a ballot
   for (int base = (tid >> 6) * 64; base < RB * D; base += kBlock) {
     const int f = base + (tid & 63), j = jb + f / D, col = f % D;
-    const uint64_t m = __ballot(sign_negative(mix_seed(k.qjl_seed, (uint64_t)j), (uint64_t)j, (uint64_t)col));
+    const uint64_t m = __ballot(sign_negative(sign_base(k.qjl_seed, (uint64_t)j), (uint32_t)col));
     if ((tid & 63) == 0) {
       s_bits[base / 32] = (uint32_t)m;
       s_bits[base / 32 + 1] = (uint32_t)(m >> 32);
@@ -287,7 +245,6 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
   constexpr int BT = (D / 2) * PE;         // pair tables per query
   constexpr int CT = (D / 4) * 16;         // sign-nibble tables per query
   constexpr int NW = D * PB / 32;
-  constexpr int U = StoreUnit<D * PB / 8>::value;
   __shared__ float s_tab[QB * (BT + CT)];
   __shared__ float s_cent[16];
   if (threadIdx.x < 16) s_cent[threadIdx.x] = k.polar.cent[threadIdx.x & ((1 << PB) - 1)];
@@ -315,7 +272,8 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
   const long long key = (long long)blockIdx.x * kBlock + threadIdx.x;
   if (key >= nk) return;
   uint32_t pk[NW], sg[D / 32];
-  load_words<NW, U>(polar + key * (D * PB / 8), pk);
+#pragma unroll
+  for (int i = 0; i < NW; i++) pk[i] = reinterpret_cast<const uint32_t *>(polar + key * (D * PB / 8))[i];
 #pragma unroll
   for (int i = 0; i < D / 32; i++) sg[i] = signs[key * (D / 32) + i];
   const float scale = f16_to_f32(polar_scales[key]);
@@ -477,9 +435,9 @@ __global__ __launch_bounds__(kBlock) void qjl_sign_matrix_kernel(uint32_t *__res
   const int it = blockIdx.x * kBlock + threadIdx.x;
   if (it >= D * D / 32) return;
   const int j = it / (D / 32), w = it % (D / 32);
-  const uint64_t rs = mix_seed(seed, (uint64_t)j);
+  const uint64_t base = sign_base(seed, (uint64_t)j);
   uint32_t bits = 0;
-  for (int b = 0; b < 32; b++) bits |= (sign_negative(rs, (uint64_t)j, (uint64_t)(32 * w + b)) ? 1u : 0u) << b;
+  for (int b = 0; b < 32; b++) bits |= (sign_negative(base, (uint32_t)(32 * w + b)) ? 1u : 0u) << b;
   out[it] = bits;
 }
 
@@ -534,7 +492,8 @@ extern "C" int tq_qjl_quantize_batch(const float *data, uint8_t *polar_packed, u
   const long long n = (long long)num_vectors;
   return by_dim_bits(dim, total_bits - 1, [&](auto d, auto pb) {
     hipLaunchKernelGGL((qjl_quant_kernel<decltype(d)::value, decltype(pb)::value>), dim3((unsigned)((n + 31) / 32)),
-                       dim3(kBlock), 0, stream, data, polar_packed, polar_scales, reinterpret_cast<uint32_t *>(signs),
+                       dim3(4 * decltype(d)::value), 0, stream, data, polar_packed, polar_scales,
+                       reinterpret_cast<uint16_t *>(signs),
                        residual_norms, n, k);
     return tqh::check_launch("qjl_quant_kernel");
   });
