@@ -242,6 +242,23 @@ __device__ __forceinline__ int pow2_exponent(float m) {
 }
 __device__ __forceinline__ float exp2i(int e) { return u2f((uint32_t)(127 + e) << 23); }
 
+// ---- rows of an f32 matrix as two f16 parts on a power-of-two scale per row ----
+// The scale 2^-E that brings a row's largest magnitude m into [2^13, 2^14),
+// as the exponent E (m = 0 and tiny rows: clamped; an infinite m takes 114,
+// which keeps every finite element of the row finite in f16).
+__device__ __forceinline__ int row_exponent(float m) {
+  const int e = (int)((f2u(m) >> 23) & 0xffu) - 126;
+  return min(max(e, -100), 128) - 14;
+}
+// x 2^-E as two f16 parts.  An infinity is its own upper part.
+__device__ __forceinline__ void split2(float x, float sc, uint16_t &hi, uint16_t &lo) {
+  const float v = x * sc;
+  hi = f32_to_f16(v);
+  const float h = f16_to_f32(hi);
+  lo = f32_to_f16(h == v ? 0.f : v - h);
+}
+__device__ __forceinline__ uint32_t pack_pair(uint16_t a, uint16_t b) { return (uint32_t)a | ((uint32_t)b << 16); }
+
 // Code pair p (codes 2p, 2p+1) of a qblock's BITS words, LSB-first: the
 // 2 BITS-bit pair-table index (p must fold to a constant after unrolling).
 template <int BITS>

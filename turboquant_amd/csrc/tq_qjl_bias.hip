@@ -54,22 +54,6 @@ struct BiasArgs {
   int token_blocks;
 };
 
-// The scale 2^-E that brings a row's largest magnitude m into [2^13, 2^14),
-// as the exponent E (m = 0 and tiny rows: clamped; an infinite m takes 114,
-// which keeps every finite element of the row finite in f16).
-__device__ __forceinline__ int row_exponent(float m) {
-  const int e = (int)((f2u(m) >> 23) & 0xffu) - 126;
-  return min(max(e, -100), 128) - 14;
-}
-// x 2^-E as two f16 parts.  An infinity is its own upper part.
-__device__ __forceinline__ void split2(float x, float sc, uint16_t &hi, uint16_t &lo) {
-  const float v = x * sc;
-  hi = f32_to_f16(v);
-  const float h = f16_to_f32(hi);
-  lo = f32_to_f16(h == v ? 0.f : v - h);
-}
-__device__ __forceinline__ uint32_t pair(uint16_t a, uint16_t b) { return (uint32_t)a | ((uint32_t)b << 16); }
-
 // Four values as consecutive elements of type OUT.  Rows of kv_len elements
 // start anywhere, so the store is of unaligned bytes.
 template <int OUT>
@@ -78,8 +62,8 @@ __device__ __forceinline__ void store4(char *p, const float (&v)[4]) {
     __builtin_memcpy(p, v, 16);
   } else {
     const uint2 w = OUT == kBF16 ? make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]))
-                                 : make_uint2(pair(f32_to_f16(v[0]), f32_to_f16(v[1])),
-                                              pair(f32_to_f16(v[2]), f32_to_f16(v[3])));
+                                 : make_uint2(pack_pair(f32_to_f16(v[0]), f32_to_f16(v[1])),
+                                              pack_pair(f32_to_f16(v[2]), f32_to_f16(v[3])));
     __builtin_memcpy(p, &w, 8);
   }
 }
@@ -141,8 +125,8 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
       uint16_t hi[4], lo[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) split2(x[i], sc, hi[i], lo[i]);
-      *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pair(hi[0], hi[1]), pair(hi[2], hi[3]));
-      *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pair(lo[0], lo[1]), pair(lo[2], lo[3]));
+      *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
+      *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
       if (lane % LPR == 0) s_scale[row] = exp2i(e);
     }
   } else {
@@ -232,8 +216,8 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
 #pragma unroll
         for (int i = 0; i < 4; i++) split2(rq[jt][i], sc, hi[i], lo[i]);
         const int at = row * RS + 16 * (JH * jh + jt) + 4 * lg;
-        *reinterpret_cast<uint2 *>(s_hi + at) = make_uint2(pair(hi[0], hi[1]), pair(hi[2], hi[3]));
-        *reinterpret_cast<uint2 *>(s_lo + at) = make_uint2(pair(lo[0], lo[1]), pair(lo[2], lo[3]));
+        *reinterpret_cast<uint2 *>(s_hi + at) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
+        *reinterpret_cast<uint2 *>(s_lo + at) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
       }
       if (jh == 0 && lg == 0) s_scale[row] = exp2i(e);
     }
