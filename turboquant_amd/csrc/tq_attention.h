@@ -185,9 +185,7 @@ struct DecCfg {
   static_assert(TPW % 64 == 0, "whole V-scale loads per lane");
   static_assert(QPM * HPM == 8 && HPM >= HG, "one instruction serves every head");
   static_assert(WAVES == 4 || WAVES == 8 || WAVES == 16, "waves per workgroup");
-  // does the workgroup's LDS (with the merge's scratch) fit 64 KiB (the
-  // 8-wave form is taken only then), and gfx950's 160 KiB at all?
-  static constexpr bool LDS_FITS = TOTAL * 4 + MERGE_LDS <= 64 * 1024;
+  // does the workgroup's LDS (with the merge's scratch) fit gfx950's 160 KiB?
   static constexpr bool LDS_OK = TOTAL * 4 + MERGE_LDS <= 160 * 1024;
   // The grid passes (4-bit codes on the MaxNorm codebook) read no codebook
   // table and take one query operand per qblock instead of per slice pair:
@@ -198,6 +196,11 @@ struct DecCfg {
   static constexpr int G_SHIFT = OFF_W - G_OFF_W;
   static constexpr int VSTAGE = WAVES * 64 * VRS;
   static constexpr bool G_LDS_OK = (TOTAL - G_SHIFT) * 4 + MERGE_LDS + VSTAGE <= 160 * 1024;
+  // every kernel of the configuration fits: the 8-wave forms, one workgroup
+  // per compute unit, are taken up to the whole 160 KiB (4 and 8 query heads
+  // per KV head need 69 to 134 KiB; held to 64 KiB they took 4 waves: QJL 3
+  // bits, 4 heads, 3 sequences of up to 6,001 tokens 19.6 us against 17.7)
+  static constexpr bool LDS_FITS = LDS_OK && (BITS != 4 || MODE != kModePqo || G_LDS_OK);
 };
 
 // A buffer resource over the bytes [off, total) of the records at base:

@@ -1327,6 +1327,13 @@ void launch_stream_cfg(AttnArgs &a, dim3 grid, hipStream_t st) {
   if constexpr (INLINE && C::WAVES != 4) {
     const long long wgs = (long long)((a.max_len + C::CHUNK - 1) / C::CHUNK) * grid.y * grid.z;
     if (wgs > device_cus()) return launch_stream_c<C4, INLINE>(a, grid, st);
+    // sequences that 4 waves of 64 tokens hold: 4 more would only join the
+    // combine (head_dim 256, PQ 4 bits, 8 heads, 128 tokens 19.0 us against
+    // 22.0; with the QJL correction they halve the projection instead, 2
+    // heads, 81 tokens 17.5 against 15.9)
+    if constexpr (C::TPW == 64 && !C::QJL) {
+      if (a.max_len <= C4::CHUNK) return launch_stream_c<C4, INLINE>(a, grid, st);
+    }
     // a grid that leaves compute units idle: 64 tokens per wave when that
     // grid still fits one round (C3's shape up to 16,384 tokens: 2,048 and
     // 4,096 tokens 11.8 / 12.0 -> 9.5 us; 32,768 stays at 128)
