@@ -239,11 +239,9 @@ class KvCache {
   // dequantize_full (common.rs:16-62): [num_kv_heads][seq][head_dim]
   int dequantize_full(int l, void *k_out, void *v_out, int dtype, hipStream_t stream) {
     const LayerBuffers &L = storage_.layer(l);
-    int rc = tq_polar_dequantize_from_cache(L.k_idx, L.k_sc, (long long)L.cap, heads_, (int)L.seq, k_out, dtype,
-                                            head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode, stream);
-    if (rc) return rc;
-    return tq_polar_dequantize_from_cache(L.v_idx, L.v_sc, (long long)L.cap, heads_, (int)L.seq, v_out, dtype,
-                                          head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode, stream);
+    return tqh::polar_dequantize_from_cache(L.k_idx, L.k_sc, L.v_idx, L.v_sc, (long long)L.cap, heads_, (int)L.seq,
+                                            k_out, v_out, dtype, head_dim_, mode_.bits, mode_.outlier_blocks,
+                                            mode_.norm_mode, stream);
   }
 
   int rq_scratch(size_t num_rows, hipStream_t stream) {

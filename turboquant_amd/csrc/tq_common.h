@@ -77,6 +77,13 @@ int polar_quantize_to_cache(const void *x, const void *x2, int x_dtype, int num_
                             long long offset, int head_dim, int bits, size_t outlier_blocks, int norm_mode,
                             hipStream_t stream);
 
+// tq_polar_dequantize_from_cache and, unless out2 is null, the same records of
+// packed2 and scales2 into out2, in one launch.
+int polar_dequantize_from_cache(const uint8_t *packed, const uint16_t *scales, const uint8_t *packed2,
+                                const uint16_t *scales2, long long head_stride, int num_heads, int tokens, void *out,
+                                void *out2, int out_dtype, int head_dim, int bits, size_t outlier_blocks,
+                                int norm_mode, hipStream_t stream);
+
 // A TQ cache's append in one launch: k and v [num_heads][tokens][head_dim]
 // quantized into their records, the sketch of the keys' residuals
 // (tq_qjl_cache_sketch) and, for num_q_rows > 0, rq = R q (tq_qjl_project).

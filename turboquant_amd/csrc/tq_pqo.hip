@@ -78,6 +78,13 @@ __global__ __launch_bounds__(256) void pqo_quant_rotated_dev_kernel(
   scales[blk] = f32_to_f16(s * scale_sign);
 }
 
+// A second set of records of a dequantize launch (out null: none).
+struct SecondOut {
+  const uint8_t *packed = nullptr;
+  const uint16_t *scales = nullptr;
+  void *out = nullptr;
+};
+
 struct DequantConsts {
   float cb[16];   // codebook values (f32); the outlier codebook when mixed
   float cbn[16];  // mixed: the standard codebook
@@ -91,7 +98,8 @@ struct DequantConsts {
 // out_j = fl(fl(W_j * fl(1/sqrt(32))) * |scale|), W = butterfly(cb[idx] * sign):
 // butterfly_wht_inverse_cpu (wht_tensor.rs:38-64) then the broadcast_mul by
 // |scale| (quantize_tensor.rs:203, 217-218).
-// MAP: inputs come from cache records (CacheMap); outputs in block order.
+// MAP: inputs come from cache records (CacheMap); outputs in block order; a
+// second set of records (a layer's values beside its keys) is taken by y = 1.
 // MIXED: the codebook per block from the scale's sign (else one codebook).
 // With the library's constants the table holds fl(cb * |sg|) and element j
 // takes it negated where sg[j] < 0: fl(c * -m) = -fl(c * m), the same value
@@ -103,7 +111,13 @@ __global__ __launch_bounds__(256) void pqo_dequant_kernel(const uint8_t *__restr
                                                           void *__restrict__ out, long long nblocks,
                                                           DequantConsts dc,
                                                           const float *__restrict__ dev_cb,
-                                                          const float *__restrict__ dev_sg, CacheMap map = {}) {
+                                                          const float *__restrict__ dev_sg, CacheMap map = {},
+                                                          SecondOut second = {}) {
+  if (MAP && blockIdx.y) {
+    packed = second.packed;
+    scales = second.scales;
+    out = second.out;
+  }
   __shared__ float lut[32];
   constexpr int NC = 1 << BITS;
   if (threadIdx.x < NC) lut[threadIdx.x] = DEV_CONSTS ? dev_cb[threadIdx.x] : dc.cb[threadIdx.x] * dc.sgm;
@@ -306,16 +320,17 @@ int check_shape(int head_dim) {
 
 template <bool MAP>
 int launch_dequant(const uint8_t *packed, const uint16_t *scales, void *out, int out_dtype, long long nblocks,
-                   int bits, const DequantConsts &dc, const CacheMap &m, hipStream_t stream) {
-  const dim3 grid((unsigned)((nblocks + 255) / 256)), block(256);
+                   int bits, const DequantConsts &dc, const CacheMap &m, const SecondOut &second,
+                   hipStream_t stream) {
+  const dim3 grid((unsigned)((nblocks + 255) / 256), second.out ? 2 : 1), block(256);
 #define DL(B, D)                                                                                                  \
   do {                                                                                                            \
     if (dc.mixed)                                                                                                 \
       hipLaunchKernelGGL((pqo_dequant_kernel<B, D, false, MAP, true>), grid, block, 0, stream, packed, scales, out, \
-                         nblocks, dc, nullptr, nullptr, m);                                                       \
+                         nblocks, dc, nullptr, nullptr, m, second);                                               \
     else                                                                                                          \
       hipLaunchKernelGGL((pqo_dequant_kernel<B, D, false, MAP, false>), grid, block, 0, stream, packed, scales,     \
-                         out, nblocks, dc, nullptr, nullptr, m);                                                  \
+                         out, nblocks, dc, nullptr, nullptr, m, second);                                          \
   } while (0)
   if (bits == 3) {
     if (out_dtype == kF32) DL(3, kF32);
@@ -359,7 +374,7 @@ extern "C" int tq_polar_dequantize(const uint8_t *packed, const uint16_t *scales
   if (!packed || !scales || !out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
   const long long nblocks = (long long)num_vectors * (head_dim / 32);
   return launch_dequant<false>(packed, scales, out, out_dtype, nblocks, bits, dequant_consts(codec),
-                               CacheMap{}, stream);
+                               CacheMap{}, SecondOut{}, stream);
 }
 
 extern "C" int tq_pqo_quantize(const void *x, int x_dtype, uint8_t *packed_out, uint16_t *scales_out,
@@ -494,24 +509,35 @@ extern "C" int tq_polar_quantize_to_cache(const void *x, int x_dtype, int num_he
                                       norm_mode, stream);
 }
 
+namespace tqh {
+int polar_dequantize_from_cache(const uint8_t *packed, const uint16_t *scales, const uint8_t *packed2,
+                                const uint16_t *scales2, long long head_stride, int num_heads, int tokens, void *out,
+                                void *out2, int out_dtype, int head_dim, int bits, size_t outlier_blocks,
+                                int norm_mode, hipStream_t stream) {
+  int rc = check_shape(head_dim);
+  if (rc) return rc;
+  PolarCodec codec;
+  rc = polar_codec(bits, norm_mode, outlier_blocks, head_dim / 32, codec);
+  if (rc) return rc;
+  if (!valid_dtype(out_dtype)) return fail(TQ_ERR_INVALID_ARGUMENT, "unknown dtype %d", out_dtype);
+  CacheMap m;
+  rc = cache_map(num_heads, tokens, head_dim, head_stride, 0, m);
+  if (rc) return rc;
+  const long long nblocks = (long long)num_heads * tokens * (head_dim / 32);
+  if (nblocks == 0) return TQ_OK;
+  if (!packed || !scales || !out) return fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
+  return launch_dequant<true>(packed, scales, out, out_dtype, nblocks, bits, dequant_consts(codec), m,
+                              SecondOut{packed2, scales2, out2}, stream);
+}
+}  // namespace tqh
+
 extern "C" int tq_polar_dequantize_from_cache(const uint8_t *packed_cache, const uint16_t *scales_cache,
                                               long long cache_head_stride, int num_heads, int tokens, void *out,
                                               int out_dtype, int head_dim, int bits, size_t outlier_blocks,
                                               int norm_mode, hipStream_t stream) {
-  int rc = check_shape(head_dim);
-  if (rc) return rc;
-  tqh::PolarCodec codec;
-  rc = tqh::polar_codec(bits, norm_mode, outlier_blocks, head_dim / 32, codec);
-  if (rc) return rc;
-  if (!tqh::valid_dtype(out_dtype)) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "unknown dtype %d", out_dtype);
-  CacheMap m;
-  rc = cache_map(num_heads, tokens, head_dim, cache_head_stride, 0, m);
-  if (rc) return rc;
-  const long long nblocks = (long long)num_heads * tokens * (head_dim / 32);
-  if (nblocks == 0) return TQ_OK;
-  if (!packed_cache || !scales_cache || !out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
-  return launch_dequant<true>(packed_cache, scales_cache, out, out_dtype, nblocks, bits, dequant_consts(codec),
-                              m, stream);
+  return tqh::polar_dequantize_from_cache(packed_cache, scales_cache, nullptr, nullptr, cache_head_stride, num_heads,
+                                          tokens, out, nullptr, out_dtype, head_dim, bits, outlier_blocks, norm_mode,
+                                          stream);
 }
 
 extern "C" int tq_pqo_quantize_to_cache(const void *x, int x_dtype, int num_heads, int tokens, uint8_t *packed_cache,
