@@ -94,7 +94,8 @@ def _stream() -> int:
 
 
 def _check_kv(k: torch.Tensor, v: torch.Tensor, heads: int, head_dim: int):
-    if k.shape != v.shape or k.dim() != 4 or k.shape[0] != 1 or k.shape[1] != heads or k.shape[3] != head_dim:
+    s = k.shape
+    if s != v.shape or len(s) != 4 or s[0] != 1 or s[1] != heads or s[3] != head_dim:
         raise ValueError(f"k/v must be [1, {heads}, T, {head_dim}], got {tuple(k.shape)} / {tuple(v.shape)}")
     if k.dtype not in _DT or v.dtype != k.dtype:
         raise ValueError("k/v must share one of f32/bf16/f16")
@@ -102,11 +103,15 @@ def _check_kv(k: torch.Tensor, v: torch.Tensor, heads: int, head_dim: int):
 
 
 def _check_q(q: torch.Tensor, num_kv_heads: int, head_dim: int) -> torch.Tensor:
-    if q.dim() != 4 or q.shape[0] != 1 or q.shape[3] != head_dim or q.shape[1] % num_kv_heads != 0:
+    s = q.shape
+    if len(s) != 4 or s[0] != 1 or s[3] != head_dim or s[1] % num_kv_heads != 0:
         raise ValueError(f"q must be [1, Hq, q_len, {head_dim}] with Hq a multiple of {num_kv_heads}")
     if q.dtype not in _DT:
         raise ValueError("q must be f32/bf16/f16")
     return q.contiguous()
+
+
+_decode = lib.tq_cache_decode
 
 
 class _DeviceCache:
@@ -130,7 +135,7 @@ class _DeviceCache:
             self._h = None
 
     def _layer_out(self, k: torch.Tensor, s: int):
-        k_out = torch.empty((1, self.num_kv_heads, s, self.head_dim), dtype=k.dtype, device=k.device)
+        k_out = k.new_empty((1, self.num_kv_heads, s, self.head_dim))
         return k_out, torch.empty_like(k_out)
 
     def seq_len(self, layer: int) -> int:
@@ -171,7 +176,7 @@ class _DeviceCache:
         records; a TqCache includes the QJL correction.  Returns [1, Hq, q_len, D]."""
         qc = _check_q(q, self.num_kv_heads, self.head_dim)
         hq, ql = qc.shape[1], qc.shape[2]
-        out = torch.empty((1, hq, ql, self.head_dim), dtype=out_dtype or qc.dtype, device=qc.device)
+        out = torch.empty_like(qc) if out_dtype is None or out_dtype == qc.dtype else torch.empty_like(qc, dtype=out_dtype)
         check(lib.tq_cache_attend_prefill(self._h, layer, qc.data_ptr(), _DT[qc.dtype], hq, ql, 1 if causal else 0,
                                           float(softmax_scale), out.data_ptr(), _DT[out.dtype], _stream()))
         return out
@@ -179,19 +184,21 @@ class _DeviceCache:
     def _prefill(self, layer, k, v, q):
         k, v = _check_kv(k, v, self.num_kv_heads, self.head_dim)
         t = k.shape[2]
-        s = self.seq_len(layer) + t
-        k_out, v_out = self._layer_out(k, s)
+        before = self.seq_len(layer)
+        s = before + t
+        # the layer's first call returns the caller's k and v: nothing to write them to
+        k_out, v_out = self._layer_out(k, s) if before else (None, None)
         bias = None
         qc, hq, ql = None, 0, 0
         if self._qjl:
             qc = _check_q(q, self.num_kv_heads, self.head_dim)
             hq, ql = qc.shape[1], qc.shape[2]
-            bias = torch.empty((1, hq, ql, s), dtype=qc.dtype, device=k.device)
+            bias = qc.new_empty((1, hq, ql, s))
         orig = C.c_int(0)
         check(lib.tq_cache_prefill(self._h, layer, k.data_ptr(), v.data_ptr(), _DT[k.dtype], t,
                                    qc.data_ptr() if qc is not None else None, _DT[qc.dtype] if qc is not None else 0,
-                                   hq, ql, k_out.data_ptr(), v_out.data_ptr(), C.byref(orig),
-                                   bias.data_ptr() if bias is not None else None, _stream()))
+                                   hq, ql, k_out.data_ptr() if before else None, v_out.data_ptr() if before else None,
+                                   C.byref(orig), bias.data_ptr() if bias is not None else None, _stream()))
         if orig.value:
             return DequantResult(k, v, bias)
         return DequantResult(k_out, v_out, bias)
@@ -201,11 +208,11 @@ class _DeviceCache:
         qc = _check_q(q, self.num_kv_heads, self.head_dim)
         if qc.shape[2] != 1:
             raise ValueError("decode takes one query position: q [1, Hq, 1, head_dim]")
-        hq = qc.shape[1]
-        out = torch.empty((1, hq, 1, self.head_dim), dtype=k.dtype, device=k.device)
-        check(lib.tq_cache_decode(self._h, layer, k.data_ptr(), v.data_ptr(), _DT[k.dtype], k.shape[2],
-                                  qc.data_ptr(), _DT[qc.dtype], hq, float(config.softmax_scale), out.data_ptr(),
-                                  _DT[out.dtype], _stream()))
+        hq, kd = qc.shape[1], k.dtype
+        out = torch.empty_like(qc) if qc.dtype == kd and qc.device == k.device else k.new_empty((1, hq, 1, self.head_dim))
+        dt = _DT[kd]
+        check(_decode(self._h, layer, k.data_ptr(), v.data_ptr(), dt, k.shape[2], qc.data_ptr(), _DT[qc.dtype], hq,
+                      float(config.softmax_scale), out.data_ptr(), dt, _stream()))
         return out
 
     def _decode_dequantized(self, layer, k, v, q) -> DequantResult:
