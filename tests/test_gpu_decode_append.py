@@ -1,0 +1,65 @@
+"""A one-token decode of a PqoCache, whose launch stores the token before it
+attends: records equal to polar_quantize's and outputs equal, bit for bit, to
+a decode over records that an append of its own has stored, at the edges of
+the chunks (one workgroup per KV head, several, a token that opens a chunk),
+for every dtype, both bit widths and codebooks, 1 to 16 query heads per KV
+head and growth in between."""
+import math
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def tq():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import turboquant_amd
+    return turboquant_amd
+
+
+@pytest.mark.parametrize("d,bits,pq,hkv,nr,dtype,before", [
+    (128, 3, False, 8, 2, "bf16", (0, 76, 511, 512, 1023, 1024, 5000)), (128, 4, False, 2, 4, "f16", (0, 512, 1024, 2047)),
+    (128, 3, True, 2, 8, "f32", (1, 513)), (64, 4, True, 3, 1, "bf16", (63, 512)), (256, 4, False, 2, 8, "f32", (255, 256)),
+    (256, 3, False, 1, 3, "bf16", (130, 1024)), (32, 3, False, 2, 2, "f16", (9, 700)), (128, 3, False, 1, 16, "bf16", (40,)),
+])
+def test_token_stored_in_the_decode_launch(tq, d, bits, pq, hkv, nr, dtype, before):
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    ob = 0 if pq else tq.cache.OUTLIER_ALL
+    cfg = tq.CacheConfig(bits=bits, head_dim=d, num_kv_heads=hkv, num_layers=1, outlier_blocks=ob)
+    att = tq.AttendConfig(1 / math.sqrt(d), nr)
+    g = torch.Generator(device="cuda").manual_seed(d + bits + nr)
+    for t in before:
+        k, v = (torch.randn((1, hkv, t + 2, d), generator=g, device="cuda").to(dt) for _ in range(2))
+        q = torch.randn((1, hkv * nr, 2, d), generator=g, device="cuda").to(dt)
+        one, two = tq.PqoCache(cfg), tq.PqoCache(cfg)
+        if t:
+            for c in (one, two):
+                c.prefill(0, k[:, :, :t].contiguous(), v[:, :, :t].contiguous())
+        for i in range(2):
+            s = slice(t + i, t + i + 1)
+            ki, vi, qi = k[:, :, s].contiguous(), v[:, :, s].contiguous(), q[:, :, i:i + 1].contiguous()
+            got = one.decode(0, ki, vi, qi, att)
+            two.decode_dequantized(0, ki, vi)  # stores with a launch of its own
+            none = torch.empty((1, hkv, 0, d), dtype=dt, device="cuda")
+            ref = two.decode(0, none, none, qi, att)
+            assert torch.equal(got, ref), (t, i)
+            assert one.seq_len(0) == two.seq_len(0) == t + i + 1
+        for a, b in zip(one.read_layer(0), two.read_layer(0)):
+            assert torch.equal(a, b)
+        p, sc = tq.polar_quantize(k.reshape(-1, d), bits, ob)
+        ki, ks, _, _ = one.read_layer(0)
+        assert torch.equal(ki.view(p.shape), p) and torch.equal(ks.view(sc.shape), sc)
+
+
+def test_a_refused_shape_still_stores_its_token(tq):
+    cfg = tq.CacheConfig(bits=3, head_dim=96, num_kv_heads=2, num_layers=1)
+    c = tq.PqoCache(cfg)
+    k = torch.randn((1, 2, 1, 96), device="cuda")
+    with pytest.raises(tq.TurboQuantError, match="head_dim 32, 64, 128 or 256"):
+        c.decode(0, k, k, k, tq.AttendConfig(0.1, 1))
+    assert c.seq_len(0) == 1
+    p, _ = tq.polar_quantize(k.reshape(-1, 96), 3)
+    assert torch.equal(c.read_layer(0)[0].view(p.shape), p)

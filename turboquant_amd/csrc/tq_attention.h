@@ -10,6 +10,7 @@
 #include "tq_common.h"
 #include "tq_device.h"
 #include "tq_mfma.h"
+#include "tq_pqo_dev.h"
 
 #include <type_traits>
 
@@ -98,6 +99,16 @@ struct AttnArgs {
   int cb_args;
   float cb[16];
 };
+
+// A token that the decode launch stores first (tqh::AppendToken).
+struct AppendArgs {
+  const void *k, *v;
+  int dtype;
+  uint8_t *k_idx, *v_idx;
+  uint16_t *k_sc, *v_sc;
+  tqp::QuantConsts qc;
+};
+struct NoAppend {};
 
 // Query element as stored (f32 bits or a 16-bit pattern), converted
 // separately so that the wait for the load lands at the first use.
@@ -395,9 +406,10 @@ int device_cus();
 // heads, batch) for BITS-bit records of cache mode MODE; a.chunk, a.cpr and
 // grid.x are set from the launched configuration.  INLINE: the last
 // workgroup of a (sequence, KV head) merges the split-K partials; else the
-// caller launches stream_merge_kernel after it.  Defined in the
+// caller launches stream_merge_kernel after it.  ap: a token to store before
+// attending (INLINE, PQO and PQ only; its status in ap->rc).  Defined in the
 // tq_attention_k<BITS>_<mode>.hip units.
 template <int BITS, int MODE, bool INLINE>
-void launch_stream_bm(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st);
+void launch_stream_bm(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st, tqh::AppendToken *ap);
 
 }  // namespace tqa

@@ -144,20 +144,22 @@ AttnArgs base_args() {
 // grid: (-, num_kv_heads, batch); the chunk count (grid.x), a.nr / a.ngroups
 // and a.chunk are set here from the launched configuration
 template <bool INLINE>
-int launch_stream(AttnArgs &a, int bits, int mode, int head_dim, dim3 grid, hipStream_t st) {
+int launch_stream(AttnArgs &a, int bits, int mode, int head_dim, dim3 grid, hipStream_t st,
+                  tqh::AppendToken *ap = nullptr) {
   const int hg = stream_hg(a.nr);
   a.ngroups = (a.nr + hg - 1) / hg;
   grid.y *= (unsigned)a.ngroups;
   const int nqb = head_dim / 32;
   if (bits == 3) {
-    if (mode == kModePqo) launch_stream_bm<3, kModePqo, INLINE>(a, nqb, hg, grid, st);
-    else if (mode == kModePq) launch_stream_bm<3, kModePq, INLINE>(a, nqb, hg, grid, st);
-    else launch_stream_bm<3, kModeTq, INLINE>(a, nqb, hg, grid, st);
+    if (mode == kModePqo) launch_stream_bm<3, kModePqo, INLINE>(a, nqb, hg, grid, st, ap);
+    else if (mode == kModePq) launch_stream_bm<3, kModePq, INLINE>(a, nqb, hg, grid, st, ap);
+    else launch_stream_bm<3, kModeTq, INLINE>(a, nqb, hg, grid, st, ap);
   } else {
-    if (mode == kModePqo) launch_stream_bm<4, kModePqo, INLINE>(a, nqb, hg, grid, st);
-    else if (mode == kModePq) launch_stream_bm<4, kModePq, INLINE>(a, nqb, hg, grid, st);
-    else launch_stream_bm<4, kModeTq, INLINE>(a, nqb, hg, grid, st);
+    if (mode == kModePqo) launch_stream_bm<4, kModePqo, INLINE>(a, nqb, hg, grid, st, ap);
+    else if (mode == kModePq) launch_stream_bm<4, kModePq, INLINE>(a, nqb, hg, grid, st, ap);
+    else launch_stream_bm<4, kModeTq, INLINE>(a, nqb, hg, grid, st, ap);
   }
+  if (ap && ap->rc) return ap->rc;
   return tqh::check_launch("stream_decode_kernel");
 }
 int launch_stream_merge(const AttnArgs &a, int head_dim, dim3 grid, hipStream_t st) {
@@ -243,7 +245,7 @@ int decode_attention_ws(const void *q, int q_dtype, const uint8_t *k_indices, co
                         int num_kv_heads, int head_dim, int bits, size_t outlier_blocks, int norm_mode,
                         int max_kv_len, long long kv_head_stride, long long seq_stride, float softmax_scale, void *out,
                         int out_dtype, const DecodeWs *wsd, size_t workspace_bytes, hipStream_t stream,
-                        const uint32_t *rmat = nullptr);
+                        const uint32_t *rmat = nullptr, tqh::AppendToken *append = nullptr);
 
 }  // namespace
 
@@ -255,12 +257,12 @@ int tqh::decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, 
                           int batch, int num_heads, int num_kv_heads, int head_dim, int bits, size_t outlier_blocks,
                           int norm_mode, int max_kv_len, long long kv_head_stride, long long seq_stride,
                           float softmax_scale, void *out, int out_dtype, void *workspace, size_t workspace_bytes,
-                          hipStream_t stream, const uint32_t *rmat) {
+                          hipStream_t stream, const uint32_t *rmat, AppendToken *append) {
   const DecodeWs d = caller_ws(workspace, workspace_bytes);
   return decode_attention_ws(q, q_dtype, k_indices, k_scales, v_indices, v_scales, rq, qjl_signs, qjl_norms, kv_lens,
                              host_len, batch, num_heads, num_kv_heads, head_dim, bits, outlier_blocks, norm_mode,
                              max_kv_len, kv_head_stride, seq_stride, softmax_scale, out, out_dtype,
-                             workspace ? &d : nullptr, workspace_bytes, stream, rmat);
+                             workspace ? &d : nullptr, workspace_bytes, stream, rmat, append);
 }
 
 namespace {
@@ -271,7 +273,7 @@ int decode_attention_ws(const void *q, int q_dtype, const uint8_t *k_indices, co
                         int num_kv_heads, int head_dim, int bits, size_t outlier_blocks, int norm_mode,
                         int max_kv_len, long long kv_head_stride, long long seq_stride, float softmax_scale, void *out,
                         int out_dtype, const DecodeWs *wsd, size_t workspace_bytes, hipStream_t stream,
-                        const uint32_t *rmat) {
+                        const uint32_t *rmat, tqh::AppendToken *append) {
   int rc = check_common(num_heads, num_kv_heads, head_dim, bits, max_kv_len);
   if (rc) return rc;
   tqh::PolarCodec codec;
@@ -353,7 +355,16 @@ int decode_attention_ws(const void *q, int q_dtype, const uint8_t *k_indices, co
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "the QJL-corrected decode takes head_dim 64, 128 or 256");
   a.nr = num_heads / num_kv_heads;
   const dim3 grid((unsigned)w.P, (unsigned)num_kv_heads, (unsigned)batch);
-  return launch_stream<true>(a, bits, mode, head_dim, grid, stream);
+  // The launch that attends also stores the token where one workgroup reads
+  // it: one head group per KV head, MaxNorm codes.  Two launches cost the host
+  // 2.7 us more and the GPU the 4 us of the first; the workgroup that holds
+  // the last tokens starts its keys about 2 us later.
+  if (append && (mode == kModeTq || codec.norm_mode != TQ_NORM_MAXNORM || a.nr > 8)) {
+    rc = tqh::store_token(*append, stream);
+    if (rc) return rc;
+    append = nullptr;
+  }
+  return launch_stream<true>(a, bits, mode, head_dim, grid, stream, append);
 }
 
 }  // namespace

@@ -6,6 +6,6 @@
 #include "tq_decode_kernel.h"
 
 namespace tqa {
-template void launch_stream_bm<3, kModePq, true>(AttnArgs &, int, int, dim3, hipStream_t);
-template void launch_stream_bm<3, kModePq, false>(AttnArgs &, int, int, dim3, hipStream_t);
+template void launch_stream_bm<3, kModePq, true>(AttnArgs &, int, int, dim3, hipStream_t, tqh::AppendToken *);
+template void launch_stream_bm<3, kModePq, false>(AttnArgs &, int, int, dim3, hipStream_t, tqh::AppendToken *);
 }  // namespace tqa

@@ -285,7 +285,7 @@ class KvCache {
   // a TqCache adds the QJL correction inline (rq_ready: the append already
   // projected q)
   int attend(int l, const void *q, int q_dtype, int num_q_heads, float scale, void *out, int out_dtype,
-             hipStream_t stream, bool rq_ready = false) {
+             hipStream_t stream, bool rq_ready = false, tqh::AppendToken *append = nullptr) {
     const LayerBuffers &L = storage_.layer(l);
     int rc = TQ_OK;
     const size_t need = tq_attention_workspace_size(1, num_q_heads, heads_, head_dim_, (int)L.cap);
@@ -309,10 +309,46 @@ class KvCache {
     // the length is known here: the kernel reads none from memory
     return tqh::decode_attention(q, q_dtype, L.k_idx, L.k_sc, L.v_idx, L.v_sc,
                                  mode_.qjl && !in_launch ? static_cast<const float *>(rq_) : nullptr,
-                                 mode_.qjl ? L.signs : nullptr, mode_.qjl ? L.norms : nullptr, nullptr, (int)L.seq, 1,
+                                 mode_.qjl ? L.signs : nullptr, mode_.qjl ? L.norms : nullptr, nullptr,
+                                 (int)L.seq + (append ? 1 : 0), 1,
                                  num_q_heads, heads_, head_dim_, mode_.bits, mode_.outlier_blocks, mode_.norm_mode,
                                  (int)L.cap, (long long)L.cap, 0, scale, out, out_dtype, ws_, ws_bytes_, stream,
-                                 in_launch ? static_cast<const uint32_t *>(rmat_) : nullptr);
+                                 in_launch ? static_cast<const uint32_t *>(rmat_) : nullptr, append);
+  }
+
+  // decode of one token per head: stored by the launch that attends (a PqoCache)
+  int append_attend(int l, const void *k, const void *v, int dtype, const void *q, int q_dtype, int num_q_heads,
+                    float scale, void *out, int out_dtype, hipStream_t stream) {
+    const size_t old = storage_.seq_len(l);
+    int rc = storage_.ensure_capacity(l, old + 1, stream);
+    if (rc) return rc;
+    const LayerBuffers &L = storage_.layer(l);
+    tqh::AppendToken t{};
+    t.k = k;
+    t.v = v;
+    t.dtype = dtype;
+    t.num_heads = heads_;
+    t.k_idx = L.k_idx;
+    t.v_idx = L.v_idx;
+    t.k_sc = L.k_sc;
+    t.v_sc = L.v_sc;
+    t.head_stride = (long long)L.cap;
+    t.offset = (long long)old;
+    t.head_dim = head_dim_;
+    t.bits = mode_.bits;
+    t.outlier_blocks = mode_.outlier_blocks;
+    t.norm_mode = mode_.norm_mode;
+    rc = attend(l, q, q_dtype, num_q_heads, scale, out, out_dtype, stream, false, &t);
+    if (rc == TQ_OK) {
+      storage_.set_seq(l, old + 1);
+      return TQ_OK;
+    }
+    // a shape that the attention refuses still stores its token
+    char why[512];
+    snprintf(why, sizeof why, "%s", tq_last_error());
+    size_t unused = 0;
+    const int stored = append(l, k, v, dtype, 1, &unused, stream);
+    return stored ? stored : tqh::fail(rc, "%s", why);
   }
 
   // multi-query attention of q [num_q_heads][q_len][head_dim] over the whole
@@ -462,6 +498,8 @@ extern "C" int tq_cache_decode(void *cache, int layer, const void *k, const void
   size_t old = 0;
   const bool fuse_rq = m.qjl && tokens > 0;  // the sketch launch projects q too
   c->use_stream(stream);
+  if (!m.qjl && tokens == 1 && k && v)
+    return c->append_attend(layer, k, v, kv_dtype, q, q_dtype, num_q_heads, softmax_scale, out, out_dtype, stream);
   rc = c->append(layer, k, v, kv_dtype, tokens, &old, stream, fuse_rq ? q : nullptr, q_dtype,
                  fuse_rq ? (size_t)num_q_heads : 0);
   if (rc) return rc;

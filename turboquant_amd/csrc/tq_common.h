@@ -58,17 +58,36 @@ struct PolarCodec {
 // status for an invalid mode.
 int polar_codec(int bits, int norm_mode, size_t outlier_blocks, int num_blocks, PolarCodec &codec);
 
+// One token's k and v, [num_heads][1][head_dim] of `dtype` (on 16-byte
+// boundaries), that a decode launch stores at record h * head_stride + offset
+// of every head before it attends; the length it attends over includes it.
+struct AppendToken {
+  const void *k, *v;
+  int dtype, num_heads;
+  uint8_t *k_idx, *v_idx;
+  uint16_t *k_sc, *v_sc;
+  long long head_stride, offset;
+  int head_dim, bits;
+  size_t outlier_blocks;
+  int norm_mode;
+  int rc;  // status of a launch of its own, where the decode took one
+};
+// The same as a launch of its own.
+int store_token(const AppendToken &t, hipStream_t stream);
+
 // Fused decode attention (tq_cache_decode_attention) with the length given
 // by the host: kv_lens null and host_len >= 0 means every sequence holds
 // host_len tokens, no length is read on the device; max_kv_len fixes the
 // workspace layout (a cache passes its capacity, so the layout stays put as
-// the sequence grows).
+// the sequence grows).  append: a token to store first (PQO and PQ caches),
+// inside the launch where that pays.
 int decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, const uint16_t *k_scales,
                      const uint8_t *v_indices, const uint16_t *v_scales, const float *rq, const uint8_t *qjl_signs,
                      const uint16_t *qjl_norms, const int *kv_lens, int host_len, int batch, int num_heads,
                      int num_kv_heads, int head_dim, int bits, size_t outlier_blocks, int norm_mode, int max_kv_len,
                      long long kv_head_stride, long long seq_stride, float softmax_scale, void *out, int out_dtype,
-                     void *workspace, size_t workspace_bytes, hipStream_t stream, const uint32_t *rmat = nullptr);
+                     void *workspace, size_t workspace_bytes, hipStream_t stream, const uint32_t *rmat = nullptr,
+                     AppendToken *append = nullptr);
 
 // tq_polar_quantize_to_cache of x and, unless null, of x2 (the same shape and
 // placement in its own buffers) in one launch per codebook.

@@ -157,14 +157,17 @@ __device__ __forceinline__ float sum_xor16(float v) {
 // MULTI: the launch gives workgroups ranges of several chunks (cpr > 1)
 // PROJ (TQ only): no rq from the caller, R q is formed in the launch; an
 // instance of its own, so that the launches given rq carry none of its code
-template <class C, bool INLINE_MERGE, bool GRID, bool MULTI, bool PROJ = false>
+// APPEND: the launch stores one new token of every KV head first, in the
+// workgroup that holds the sequence's last token (the only one that reads it)
+template <class C, bool INLINE_MERGE, bool GRID, bool MULTI, bool PROJ = false, bool APPEND = false>
 #ifndef TQ_DECODE_WPE
 #define TQ_DECODE_WPE 2
 #endif
 __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kernel(const uint8_t *k_idx, const uint8_t *v_idx,
                                                                const uint16_t *k_sc, const uint16_t *v_sc,
                                                                long long seq_stride, long long kv_head_stride,
-                                                               int len_hint, AttnArgs a) {
+                                                               int len_hint, AttnArgs a,
+                                                               std::conditional_t<APPEND, AppendArgs, NoAppend> ap) {
   constexpr int BITS = C::BITS, HD = C::HD, NQB = C::NQB, HG = C::HG, TPW = C::TPW, QW = C::QW, NW = C::NW;
   static_assert(GRID ? C::G_LDS_OK : C::LDS_OK, "the workgroup's LDS (with the merge's scratch) fits 160 KiB");
   // word offset of the layout from OFF_W on (the grid passes need no
@@ -464,7 +467,32 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
       if (grp < n) issue(grp, tw0);
     issue(NKT, tw0);
   };
-  issue_first(tw_first, LA0);
+  // ---- the new token, quantized by one lane per qblock (keys, then values)
+  // of wave 0; its workgroup requests no records before the setup's barrier,
+  // which the stores have passed by then ----
+  bool late = false;
+  if constexpr (APPEND) {
+    static_assert(INLINE_MERGE && !MULTI && !PROJ && !C::QJL, "an append is part of single-chunk PQO and PQ launches");
+    late = (len - 1) / C::CHUNK == ck0;
+    if (late && wave == 0) {
+      if (lane < 2 * NQB) {
+        const bool is_v = lane >= NQB;
+        const int qb = lane % NQB;
+        const void *x = is_v ? ap.v : ap.k;
+        const long long blk = (long long)g * NQB + qb, rec = (rec0 + len - 1) * NQB + qb;
+        float r[32];
+        if (ap.dtype == kF32) tqp::load_block<kF32>(x, blk, r);
+        else if (ap.dtype == kBF16) tqp::load_block<kBF16>(x, blk, r);
+        else tqp::load_block<kF16>(x, blk, r);
+        uint32_t w[BITS];
+        const float s = tqp::encode_block<BITS, C::CB, true, tqp::kMaxNorm>(r, ap.qc, w);
+        tqp::store_packed<BITS>(is_v ? ap.v_idx : ap.k_idx, rec, w);
+        (is_v ? ap.v_sc : ap.k_sc)[rec] = f32_to_f16(s * ap.qc.scale_sign);
+      }
+      __builtin_amdgcn_s_waitcnt(0);  // written through to the L2 that the workgroup's loads read
+    }
+  }
+  if (!late) issue_first(tw_first, LA0);
   auto issue_k = [&](int i, uint32_t tw0) {  // K tile i is being consumed
     if (i == 0) {
 #pragma unroll
@@ -625,6 +653,9 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
     }
   }
   __syncthreads();
+  if constexpr (APPEND) {
+    if (late) issue_first(tw_first, LA0);
+  }
   auto head_exp = [&](const float *mx, int hl) {
     float m = 0.f;
 #pragma unroll
@@ -1231,7 +1262,32 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
 // 4-bit codes on the compiled-in MaxNorm codebook (evenly spaced) take the
 // grid key pass; a caller's codebook or the L2Norm tables, the pair table
 template <class C, bool INLINE, bool MULTI>
-void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint) {
+void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint, tqh::AppendToken *ap) {
+  if constexpr (INLINE && !MULTI && !C::QJL) {
+    if (ap) {
+      AppendArgs x{};
+      x.k = ap->k;
+      x.v = ap->v;
+      x.dtype = ap->dtype;
+      x.k_idx = ap->k_idx;
+      x.v_idx = ap->v_idx;
+      x.k_sc = ap->k_sc;
+      x.v_sc = ap->v_sc;
+      tqh::PolarCodec codec;
+      ap->rc = tqh::polar_codec(ap->bits, ap->norm_mode, ap->outlier_blocks, ap->head_dim / 32, codec);
+      if (ap->rc) return;
+      x.qc = tqp::make_quant_consts(codec.cb, codec.outer, codec.scale_sign);
+      // MaxNorm: 4-bit PQO takes the grid passes
+      constexpr bool GRID = C::BITS == 4 && C::MODE == kModePqo;
+      hipLaunchKernelGGL((stream_decode_kernel<C, true, GRID, false, false, true>), grid, dim3(C::THREADS), 0, st,
+                         a.k_idx, a.v_idx, a.k_sc, a.v_sc, a.seq_stride, a.kv_head_stride, len_hint, a, x);
+      return;
+    }
+  }
+  if (ap) {  // range launches: long contexts, where a launch more does not show
+    ap->rc = tqh::store_token(*ap, st);
+    if (ap->rc) return;
+  }
   auto go = [&](auto kernel) {
     if (a.bal_nwg < 0) {
       // balanced split: as many workgroups as the compute units hold at once
@@ -1250,7 +1306,7 @@ void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint) {
       grid = dim3((unsigned)a.bal_nwg, 1u, 1u);
     }
     hipLaunchKernelGGL(kernel, grid, dim3(C::THREADS), 0, st, a.k_idx, a.v_idx, a.k_sc, a.v_sc, a.seq_stride,
-                       a.kv_head_stride, len_hint, a);
+                       a.kv_head_stride, len_hint, a, NoAppend{});
   };
   if constexpr (C::BITS == 4 && C::MODE == kModePqo) {
     if (!a.cb_dev && !a.cb_args) return go(stream_decode_kernel<C, INLINE, true, MULTI>);
@@ -1261,7 +1317,7 @@ void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint) {
   go(stream_decode_kernel<C, INLINE, false, MULTI>);
 }
 template <class C, bool INLINE>
-void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st) {
+void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
   a.chunk = C::CHUNK;
   const int chunks = (a.max_len + C::CHUNK - 1) / C::CHUNK;
   // Chunks per workgroup: one while the grid of single chunks fits one round
@@ -1296,7 +1352,7 @@ void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st) {
         a.bal_batch = (int)grid.z;
         a.bal_ny = (int)grid.y;
         const int len_hint = a.kv_lens ? -1 : max(a.single_len, 0);
-        return launch_stream_k<C, INLINE, true>(a, grid, st, len_hint);
+        return launch_stream_k<C, INLINE, true>(a, grid, st, len_hint, ap);
       }
     }
   } else if constexpr (C::CHUNK < kRefPartition) {
@@ -1310,9 +1366,9 @@ void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st) {
   if (grid.x == 0) grid.x = 1;  // an empty batch still zeroes its outputs
   const int len_hint = a.kv_lens ? -1 : max(a.single_len, 0);
   if constexpr (INLINE || C::CHUNK < kRefPartition) {
-    if (a.cpr > 1) return launch_stream_k<C, INLINE, true>(a, grid, st, len_hint);
+    if (a.cpr > 1) return launch_stream_k<C, INLINE, true>(a, grid, st, len_hint, ap);
   }
-  launch_stream_k<C, INLINE, false>(a, grid, st, len_hint);
+  launch_stream_k<C, INLINE, false>(a, grid, st, len_hint, ap);
 }
 // The cache decode picks the workgroup size per launch: 8 waves while the
 // grid of 8-wave workgroups leaves compute units idle (one long sequence:
@@ -1320,50 +1376,50 @@ void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st) {
 // workgroups per compute unit keep more waves per SIMD in flight).  The
 // reference ABI (a separate merge launch) always takes the 8-wave form.
 template <int BITS, int MODE, int NQB, int HG, bool INLINE>
-void launch_stream_cfg(AttnArgs &a, dim3 grid, hipStream_t st) {
+void launch_stream_cfg(AttnArgs &a, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
   using C = StreamCfg<BITS, MODE, NQB, HG>;
   using C4 = StreamCfg4<BITS, MODE, NQB, HG>;
   using C64 = StreamCfg64<BITS, MODE, NQB, HG>;
   if constexpr (INLINE && C::WAVES != 4) {
     const long long wgs = (long long)((a.max_len + C::CHUNK - 1) / C::CHUNK) * grid.y * grid.z;
-    if (wgs > device_cus()) return launch_stream_c<C4, INLINE>(a, grid, st);
+    if (wgs > device_cus()) return launch_stream_c<C4, INLINE>(a, grid, st, ap);
     // sequences that 4 waves of 64 tokens hold: 4 more would only join the
     // combine (head_dim 256, PQ 4 bits, 8 heads, 128 tokens 19.0 us against
     // 22.0; with the QJL correction they halve the projection instead, 2
     // heads, 81 tokens 17.5 against 15.9)
     if constexpr (C::TPW == 64 && !C::QJL) {
-      if (a.max_len <= C4::CHUNK) return launch_stream_c<C4, INLINE>(a, grid, st);
+      if (a.max_len <= C4::CHUNK) return launch_stream_c<C4, INLINE>(a, grid, st, ap);
     }
     // a grid that leaves compute units idle: 64 tokens per wave when that
     // grid still fits one round (C3's shape up to 16,384 tokens: 2,048 and
     // 4,096 tokens 11.8 / 12.0 -> 9.5 us; 32,768 stays at 128)
     if constexpr (C::TPW == 128 && C64::LDS_FITS) {
       const long long wgs64 = (long long)((a.max_len + C64::CHUNK - 1) / C64::CHUNK) * grid.y * grid.z;
-      if (wgs64 <= device_cus()) return launch_stream_c<C64, INLINE>(a, grid, st);
+      if (wgs64 <= device_cus()) return launch_stream_c<C64, INLINE>(a, grid, st, ap);
     }
   }
-  launch_stream_c<C, INLINE>(a, grid, st);
+  launch_stream_c<C, INLINE>(a, grid, st, ap);
 }
 template <int BITS, int MODE, int NQB, bool INLINE>
-void launch_stream_hg(AttnArgs &a, int hg, dim3 grid, hipStream_t st) {
-  if (hg == 2) launch_stream_cfg<BITS, MODE, NQB, 2, INLINE>(a, grid, st);
-  else if (hg == 4) launch_stream_cfg<BITS, MODE, NQB, 4, INLINE>(a, grid, st);
-  else launch_stream_cfg<BITS, MODE, NQB, 8, INLINE>(a, grid, st);
+void launch_stream_hg(AttnArgs &a, int hg, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
+  if (hg == 2) launch_stream_cfg<BITS, MODE, NQB, 2, INLINE>(a, grid, st, ap);
+  else if (hg == 4) launch_stream_cfg<BITS, MODE, NQB, 4, INLINE>(a, grid, st, ap);
+  else launch_stream_cfg<BITS, MODE, NQB, 8, INLINE>(a, grid, st, ap);
 }
 template <int BITS, int MODE, bool INLINE>
-void launch_stream_nqb(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st) {
+void launch_stream_nqb(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
   if constexpr (MODE != kModeTq) {
-    if (nqb == 1) return launch_stream_hg<BITS, MODE, 1, INLINE>(a, hg, grid, st);
+    if (nqb == 1) return launch_stream_hg<BITS, MODE, 1, INLINE>(a, hg, grid, st, ap);
   }
-  if (nqb == 2) launch_stream_hg<BITS, MODE, 2, INLINE>(a, hg, grid, st);
-  else if (nqb == 4) launch_stream_hg<BITS, MODE, 4, INLINE>(a, hg, grid, st);
-  else launch_stream_hg<BITS, MODE, 8, INLINE>(a, hg, grid, st);
+  if (nqb == 2) launch_stream_hg<BITS, MODE, 2, INLINE>(a, hg, grid, st, ap);
+  else if (nqb == 4) launch_stream_hg<BITS, MODE, 4, INLINE>(a, hg, grid, st, ap);
+  else launch_stream_hg<BITS, MODE, 8, INLINE>(a, hg, grid, st, ap);
 }
 }  // namespace
 
 template <int BITS, int MODE, bool INLINE>
-void launch_stream_bm(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st) {
-  launch_stream_nqb<BITS, MODE, INLINE>(a, nqb, hg, grid, st);
+void launch_stream_bm(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
+  launch_stream_nqb<BITS, MODE, INLINE>(a, nqb, hg, grid, st, ap);
 }
 
 }  // namespace tqa

@@ -498,6 +498,11 @@ int polar_quantize_to_cache(const void *x, const void *x2, int x_dtype, int num_
   if (!x || !packed || !scales) return fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
   return launch_polar_quant<true>(x, x_dtype, packed, scales, nblocks, codec, m, Second{x2, packed2, scales2}, stream);
 }
+
+int store_token(const AppendToken &t, hipStream_t stream) {
+  return polar_quantize_to_cache(t.k, t.v, t.dtype, t.num_heads, 1, t.k_idx, t.k_sc, t.v_idx, t.v_sc, t.head_stride,
+                                 t.offset, t.head_dim, t.bits, t.outlier_blocks, t.norm_mode, stream);
+}
 }  // namespace tqh
 
 extern "C" int tq_polar_quantize_to_cache(const void *x, int x_dtype, int num_heads, int tokens,
