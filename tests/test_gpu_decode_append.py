@@ -1,4 +1,4 @@
-"""A one-token decode of a PqoCache, whose launch stores the token before it
+"""A one-token decode, whose launch stores the token before it
 attends: records equal to polar_quantize's and outputs equal, bit for bit, to
 a decode over records that an append of its own has stored, at the edges of
 the chunks (one workgroup per KV head, several, a token that opens a chunk),
@@ -52,6 +52,35 @@ def test_token_stored_in_the_decode_launch(tq, d, bits, pq, hkv, nr, dtype, befo
         p, sc = tq.polar_quantize(k.reshape(-1, d), bits, ob)
         ki, ks, _, _ = one.read_layer(0)
         assert torch.equal(ki.view(p.shape), p) and torch.equal(ks.view(sc.shape), sc)
+
+
+@pytest.mark.parametrize("d,bits,hkv,nr,dtype,before", [
+    (128, 3, 8, 2, "bf16", (0, 76, 511, 1024)), (128, 4, 2, 4, "f16", (512, 2047)), (64, 4, 2, 4, "f32", (63, 512, 1030)),
+    (64, 3, 3, 1, "bf16", (9,)), (256, 3, 1, 2, "f32", (255, 256)), (256, 4, 2, 8, "f16", (130,)), (128, 3, 1, 16, "bf16", (40,)),
+])
+def test_tq_token_stored_and_sketched_in_the_decode_launch(tq, d, bits, hkv, nr, dtype, before):
+    """Records, signs and norms as a prefill of the same tokens stores them; the output equals that of a decode over
+    them, which projects the query in the launch too."""
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    cfg = tq.CacheConfig(bits=bits, head_dim=d, num_kv_heads=hkv, num_layers=1, outlier_blocks=0)
+    att = tq.AttendConfig(1 / math.sqrt(d), nr)
+    g = torch.Generator(device="cuda").manual_seed(d + bits + nr)
+    for t in before:
+        k, v = (torch.randn((1, hkv, t + 1, d), generator=g, device="cuda").to(dt) for _ in range(2))
+        q = torch.randn((1, hkv * nr, 1, d), generator=g, device="cuda").to(dt)
+        one, two = tq.TqCache(cfg), tq.TqCache(cfg)
+        if t:
+            one.prefill(0, k[:, :, :t].contiguous(), v[:, :, :t].contiguous(), q)
+        got = one.decode(0, k[:, :, t:].contiguous(), v[:, :, t:].contiguous(), q, att)
+        two.prefill(0, k, v, q)
+        none = torch.empty((1, hkv, 0, d), dtype=dt, device="cuda")
+        ref = two.decode(0, none, none, q, att)
+        for a, b in zip((*one.read_layer(0), *one.read_qjl(0)), (*two.read_layer(0), *two.read_qjl(0))):
+            assert torch.equal(a, b), t
+        if nr <= 8:
+            assert torch.equal(got, ref), t
+        else:  # several head groups: the append's own launch
+            assert torch.allclose(got.float(), ref.float(), atol=1e-2)
 
 
 def test_a_refused_shape_still_stores_its_token(tq):

@@ -10,7 +10,6 @@
 #include "tq_common.h"
 #include "tq_device.h"
 #include "tq_mfma.h"
-#include "tq_pqo_dev.h"
 
 #include <type_traits>
 
@@ -100,13 +99,18 @@ struct AttnArgs {
   float cb[16];
 };
 
-// A token that the decode launch stores first (tqh::AppendToken).
+// A token that the decode launch stores first (tqh::AppendToken): its key
+// and value, where they go, and the MaxNorm codec's boundaries b, 1 / outer
+// and scale sign.  TQ: the key's sketch too.
 struct AppendArgs {
   const void *k, *v;
   int dtype;
   uint8_t *k_idx, *v_idx;
   uint16_t *k_sc, *v_sc;
-  tqp::QuantConsts qc;
+  uint16_t *signs;  // as pairs of bytes
+  uint16_t *norms;
+  float b[15];
+  float mul, scale_sign;
 };
 struct NoAppend {};
 

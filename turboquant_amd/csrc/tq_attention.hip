@@ -356,10 +356,11 @@ int decode_attention_ws(const void *q, int q_dtype, const uint8_t *k_indices, co
   a.nr = num_heads / num_kv_heads;
   const dim3 grid((unsigned)w.P, (unsigned)num_kv_heads, (unsigned)batch);
   // The launch that attends also stores the token where one workgroup reads
-  // it: one head group per KV head, MaxNorm codes.  Two launches cost the host
-  // 2.7 us more and the GPU the 4 us of the first; the workgroup that holds
-  // the last tokens starts its keys about 2 us later.
-  if (append && (mode == kModeTq || codec.norm_mode != TQ_NORM_MAXNORM || a.nr > 8)) {
+  // it (one head group per KV head) and the codes are MaxNorm's.  Two launches
+  // cost the host 2.7 us more and the GPU the 4.2 us of the first (7.8 with a
+  // sketch); the workgroup that holds the last tokens starts its keys 1.5 us later
+  // (2.9 with a sketch).
+  if (append && (codec.norm_mode != TQ_NORM_MAXNORM || a.nr > 8)) {
     rc = tqh::store_token(*append, stream);
     if (rc) return rc;
     append = nullptr;

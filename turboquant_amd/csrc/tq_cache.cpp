@@ -299,8 +299,8 @@ class KvCache {
       rc = tq_attention_workspace_init(ws_, ws_bytes_, 1, num_q_heads, heads_, head_dim_, (int)L.cap, stream);
       if (rc) return rc;
     }
-    // a TqCache whose append did not project q (no token appended): the
-    // decode launch projects it from the sign matrix
+    // a TqCache whose append did not project q (none, or one token that the
+    // decode launch stores): the decode launch projects it from the sign matrix
     const bool in_launch = mode_.qjl && !rq_ready;
     if (in_launch) {
       rc = sign_matrix(stream);
@@ -316,7 +316,8 @@ class KvCache {
                                  in_launch ? static_cast<const uint32_t *>(rmat_) : nullptr, append);
   }
 
-  // decode of one token per head: stored by the launch that attends (a PqoCache)
+  // decode of one token per head: stored by the launch that attends, which
+  // also projects a TqCache's query
   int append_attend(int l, const void *k, const void *v, int dtype, const void *q, int q_dtype, int num_q_heads,
                     float scale, void *out, int out_dtype, hipStream_t stream) {
     const size_t old = storage_.seq_len(l);
@@ -332,6 +333,13 @@ class KvCache {
     t.v_idx = L.v_idx;
     t.k_sc = L.k_sc;
     t.v_sc = L.v_sc;
+    if (mode_.qjl) {
+      rc = sign_matrix(stream);
+      if (rc) return rc;
+      t.signs = L.signs;
+      t.norms = L.norms;
+      t.sign_matrix = static_cast<const uint32_t *>(rmat_);
+    }
     t.head_stride = (long long)L.cap;
     t.offset = (long long)old;
     t.head_dim = head_dim_;
@@ -498,7 +506,7 @@ extern "C" int tq_cache_decode(void *cache, int layer, const void *k, const void
   size_t old = 0;
   const bool fuse_rq = m.qjl && tokens > 0;  // the sketch launch projects q too
   c->use_stream(stream);
-  if (!m.qjl && tokens == 1 && k && v)
+  if (tokens == 1 && k && v)
     return c->append_attend(layer, k, v, kv_dtype, q, q_dtype, num_q_heads, softmax_scale, out, out_dtype, stream);
   rc = c->append(layer, k, v, kv_dtype, tokens, &old, stream, fuse_rq ? q : nullptr, q_dtype,
                  fuse_rq ? (size_t)num_q_heads : 0);

@@ -58,14 +58,18 @@ struct PolarCodec {
 // status for an invalid mode.
 int polar_codec(int bits, int norm_mode, size_t outlier_blocks, int num_blocks, PolarCodec &codec);
 
-// One token's k and v, [num_heads][1][head_dim] of `dtype` (on 16-byte
-// boundaries), that a decode launch stores at record h * head_stride + offset
-// of every head before it attends; the length it attends over includes it.
+// One token's k and v, [num_heads][1][head_dim] of `dtype`, that a decode
+// launch stores at record h * head_stride + offset of every head before it
+// attends; the length it attends over includes it.  signs, norms and
+// sign_matrix: a TQ cache's, whose key is sketched too.
 struct AppendToken {
   const void *k, *v;
   int dtype, num_heads;
   uint8_t *k_idx, *v_idx;
   uint16_t *k_sc, *v_sc;
+  uint8_t *signs;
+  uint16_t *norms;
+  const uint32_t *sign_matrix;
   long long head_stride, offset;
   int head_dim, bits;
   size_t outlier_blocks;
@@ -79,8 +83,8 @@ int store_token(const AppendToken &t, hipStream_t stream);
 // by the host: kv_lens null and host_len >= 0 means every sequence holds
 // host_len tokens, no length is read on the device; max_kv_len fixes the
 // workspace layout (a cache passes its capacity, so the layout stays put as
-// the sequence grows).  append: a token to store first (PQO and PQ caches),
-// inside the launch where that pays.
+// the sequence grows).  append: a token to store first, inside the launch
+// where that pays.
 int decode_attention(const void *q, int q_dtype, const uint8_t *k_indices, const uint16_t *k_scales,
                      const uint8_t *v_indices, const uint16_t *v_scales, const float *rq, const uint8_t *qjl_signs,
                      const uint16_t *qjl_norms, const int *kv_lens, int host_len, int batch, int num_heads,

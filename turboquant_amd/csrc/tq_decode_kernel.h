@@ -154,6 +154,108 @@ __device__ __forceinline__ float sum_xor16(float v) {
   return a + b;
 }
 
+// Quantizes the new token's key and value of KV head g into record rec (and
+// sketches the key's residual for TQ), one lane per element: the codes are
+// those of the append's own launch bit for bit (butterfly stages in the same
+// order, the reference's quotient compared with its boundaries), in a chain a
+// third as long as one lane's 32 elements.  Called by the whole workgroup;
+// every store has been acknowledged when it returns.
+template <class C, int RT, int RW>
+__device__ __forceinline__ void store_new_token(const AppendArgs &ap, const uint32_t (&rsw)[RT][RW], float inv, int g,
+                                                long long rec, int tid, int lane, int wave) {
+  constexpr int BITS = C::BITS, HD = C::HD, NQB = C::NQB, NB = (1 << C::CB) - 1, REC = NQB * BITS;  // words per record
+  constexpr int IT = (2 * HD + C::THREADS - 1) / C::THREADS;
+  __shared__ uint32_t s_word[2 * REC];
+  __shared__ __attribute__((aligned(16))) float s_res[C::QJL ? HD : 4];
+  for (int i = tid; i < 2 * REC; i += C::THREADS) s_word[i] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < IT; it++) {
+    const int e = tid + it * C::THREADS;  // keys, then values: uniform per 32 lanes
+    if (e < 2 * HD) {
+      const bool is_v = e >= HD;
+      const int d = is_v ? e - HD : e, i = e & 31, qb = d >> 5;
+      const void *src = is_v ? ap.v : ap.k;
+      const long long xi = (long long)g * HD + d;
+      float x;
+      if (ap.dtype == kF32) x = static_cast<const float *>(src)[xi];
+      else if (ap.dtype == kBF16) x = bf16_to_f32(static_cast<const uint16_t *>(src)[xi]);
+      else x = f16_to_f32(static_cast<const uint16_t *>(src)[xi]);
+      const float r = wht32_lanes(x, i) * (((kPqoSignMask >> i) & 1u) ? -kInvSqrt32 : kInvSqrt32);
+      float m = fabsf(r);
+      m = fmaxf(m, lane_xor<1>(m));
+      m = fmaxf(m, lane_xor<2>(m));
+      m = fmaxf(m, lane_xor<4>(m));
+      m = fmaxf(m, lane_xor<8>(m));
+      m = fmaxf(m, lane_xor<16>(m));
+      float s = fmaxf(0.0f, m) * ap.mul;
+      if (s < 1e-10f) s = 1e-10f;
+      const float v = r / s;
+      uint32_t code = 0;
+#pragma unroll
+      for (int t = 0; t < NB; t++) code += v > ap.b[t] ? 1u : 0u;
+      const int pos = i * BITS, wi = pos >> 5, sh = pos & 31;
+      uint32_t *word = s_word + (is_v ? REC : 0) + qb * BITS + wi;
+      atomicOr(word, code << sh);
+      if (sh + BITS > 32) atomicOr(word + 1, code >> (32 - sh));
+      const uint16_t h = f32_to_f16(s * ap.scale_sign);
+      if (i == 0) (is_v ? ap.v_sc : ap.k_sc)[rec * NQB + qb] = h;
+      if constexpr (C::QJL) {
+        if (!is_v) {  // the residual: k less its record, decoded as the append decodes it
+          const float c = pqo_centroid<C::CB>((int)code) * kDecodeFactor;
+          const float y = wht32_lanes(((kPqoSignMask >> i) & 1u) ? -c : c, i);
+          s_res[d] = x - (y * kInvSqrt32) * fabsf(f16_to_f32(h));
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < 2 * REC; i += C::THREADS) {
+    uint32_t *dst = reinterpret_cast<uint32_t *>(i < REC ? ap.k_idx : ap.v_idx) + rec * REC + (i < REC ? i : i - REC);
+    *dst = s_word[i];
+  }
+  if constexpr (C::QJL) {
+    const int l16 = lane & 15, lg = lane >> 4;
+    // rows 16 (wave + WAVES t) .. of R r in column order from -0.0
+    // (qjl.rs:196-208): v_mfma_f32_16x16x4_f32 adds its four products one
+    // after the other as fused multiply-adds; every column is the key
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+      const int rt = wave + C::WAVES * t;
+      if (rt < HD / 16) {  // uniform per wave
+        f32x4 acc = {-0.0f, -0.0f, -0.0f, -0.0f};
+#pragma unroll
+        for (int w = 0; w < NQB; w++) {
+          const uint32_t rb = rsw[t][w] >> lg;
+#pragma unroll
+          for (int k = 0; k < 8; k++)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(u2f(((rb << (31 - 4 * k)) & 0x80000000u) | 0x3f800000u),
+                                                       s_res[32 * w + 4 * k + lg], acc, 0, 0, 0);
+        }
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) bits |= (acc[i] * inv >= 0.0f ? 1u : 0u) << (4 * lg + i);
+        bits |= __shfl_xor(bits, 16, 64);
+        bits |= __shfl_xor(bits, 32, 64);
+        if (lane == 0) ap.signs[rec * (HD / 16) + rt] = (uint16_t)bits;
+      }
+    }
+    if (wave == C::WAVES - 1) {  // the norm, in element order
+      float ss = 0.f;
+#pragma unroll 4
+      for (int i = 0; i < HD / 4; i++) {
+        const float4 r = reinterpret_cast<const float4 *>(s_res)[i];
+        ss = ss + r.x * r.x;
+        ss = ss + r.y * r.y;
+        ss = ss + r.z * r.z;
+        ss = ss + r.w * r.w;
+      }
+      if (lane == 0) ap.norms[rec] = f32_to_f16(sqrtf(ss));
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // written through to the L2 that the workgroup's loads read
+}
+
 // MULTI: the launch gives workgroups ranges of several chunks (cpr > 1)
 // PROJ (TQ only): no rq from the caller, R q is formed in the launch; an
 // instance of its own, so that the launches given rq carry none of its code
@@ -467,30 +569,13 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
       if (grp < n) issue(grp, tw0);
     issue(NKT, tw0);
   };
-  // ---- the new token, quantized by one lane per qblock (keys, then values)
-  // of wave 0; its workgroup requests no records before the setup's barrier,
-  // which the stores have passed by then ----
+  // ---- the new token.  Its workgroup requests no records before the
+  // setup's barrier, which the stores have passed by then ----
   bool late = false;
   if constexpr (APPEND) {
-    static_assert(INLINE_MERGE && !MULTI && !PROJ && !C::QJL, "an append is part of single-chunk PQO and PQ launches");
+    static_assert(INLINE_MERGE && !MULTI && (PROJ || !C::QJL), "an append is part of single-chunk launches without rq");
     late = (len - 1) / C::CHUNK == ck0;
-    if (late && wave == 0) {
-      if (lane < 2 * NQB) {
-        const bool is_v = lane >= NQB;
-        const int qb = lane % NQB;
-        const void *x = is_v ? ap.v : ap.k;
-        const long long blk = (long long)g * NQB + qb, rec = (rec0 + len - 1) * NQB + qb;
-        float r[32];
-        if (ap.dtype == kF32) tqp::load_block<kF32>(x, blk, r);
-        else if (ap.dtype == kBF16) tqp::load_block<kBF16>(x, blk, r);
-        else tqp::load_block<kF16>(x, blk, r);
-        uint32_t w[BITS];
-        const float s = tqp::encode_block<BITS, C::CB, true, tqp::kMaxNorm>(r, ap.qc, w);
-        tqp::store_packed<BITS>(is_v ? ap.v_idx : ap.k_idx, rec, w);
-        (is_v ? ap.v_sc : ap.k_sc)[rec] = f32_to_f16(s * ap.qc.scale_sign);
-      }
-      __builtin_amdgcn_s_waitcnt(0);  // written through to the L2 that the workgroup's loads read
-    }
+    if (late) store_new_token<C>(ap, rsw, a.qjl_inv, g, rec0 + len - 1, tid, lane, wave);
   }
   if (!late) issue_first(tw_first, LA0);
   auto issue_k = [&](int i, uint32_t tw0) {  // K tile i is being consumed
@@ -1263,7 +1348,7 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
 // grid key pass; a caller's codebook or the L2Norm tables, the pair table
 template <class C, bool INLINE, bool MULTI>
 void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint, tqh::AppendToken *ap) {
-  if constexpr (INLINE && !MULTI && !C::QJL) {
+  if constexpr (INLINE && !MULTI) {
     if (ap) {
       AppendArgs x{};
       x.k = ap->k;
@@ -1273,13 +1358,17 @@ void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint, tqh::
       x.v_idx = ap->v_idx;
       x.k_sc = ap->k_sc;
       x.v_sc = ap->v_sc;
+      x.signs = reinterpret_cast<uint16_t *>(ap->signs);
+      x.norms = ap->norms;
       tqh::PolarCodec codec;
       ap->rc = tqh::polar_codec(ap->bits, ap->norm_mode, ap->outlier_blocks, ap->head_dim / 32, codec);
       if (ap->rc) return;
-      x.qc = tqp::make_quant_consts(codec.cb, codec.outer, codec.scale_sign);
-      // MaxNorm: 4-bit PQO takes the grid passes
+      for (int i = 0; i + 1 < codec.cb.nc; i++) x.b[i] = codec.cb.b[i];
+      x.mul = (float)(1.0 / (double)codec.outer);
+      x.scale_sign = codec.scale_sign;
+      // MaxNorm: 4-bit PQO takes the grid passes; a TQ query is projected here
       constexpr bool GRID = C::BITS == 4 && C::MODE == kModePqo;
-      hipLaunchKernelGGL((stream_decode_kernel<C, true, GRID, false, false, true>), grid, dim3(C::THREADS), 0, st,
+      hipLaunchKernelGGL((stream_decode_kernel<C, true, GRID, false, C::QJL, true>), grid, dim3(C::THREADS), 0, st,
                          a.k_idx, a.v_idx, a.k_sc, a.v_sc, a.seq_stride, a.kv_head_stride, len_hint, a, x);
       return;
     }

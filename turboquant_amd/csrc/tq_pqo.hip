@@ -500,6 +500,27 @@ int polar_quantize_to_cache(const void *x, const void *x2, int x_dtype, int num_
 }
 
 int store_token(const AppendToken &t, hipStream_t stream) {
+  if (t.signs) {
+    TqAppend a{};
+    a.k = t.k;
+    a.v = t.v;
+    a.dtype = t.dtype;
+    a.num_heads = t.num_heads;
+    a.tokens = 1;
+    a.k_idx = t.k_idx;
+    a.v_idx = t.v_idx;
+    a.k_sc = t.k_sc;
+    a.v_sc = t.v_sc;
+    a.signs = t.signs;
+    a.norms = t.norms;
+    a.head_stride = t.head_stride;
+    a.offset = t.offset;
+    a.head_dim = t.head_dim;
+    a.bits = t.bits;
+    a.norm_mode = t.norm_mode;
+    a.sign_matrix = t.sign_matrix;
+    return tq_append(a, stream);
+  }
   return polar_quantize_to_cache(t.k, t.v, t.dtype, t.num_heads, 1, t.k_idx, t.k_sc, t.v_idx, t.v_sc, t.head_stride,
                                  t.offset, t.head_dim, t.bits, t.outlier_blocks, t.norm_mode, stream);
 }
