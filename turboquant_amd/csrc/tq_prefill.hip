@@ -207,7 +207,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   __shared__ __attribute__((aligned(16))) uint32_t s_sg[2][kTile * 4];  // TQ: sign words
   __shared__ float s_cb[16];
   __shared__ int s_eq[kRows], s_er[kRows];
-  __shared__ uint2 s_nib[16];
+  __shared__ __attribute__((aligned(16))) u32x4 s_sign[QJL && PH != kStage ? 256 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // -1 in a register the compiler cannot see through, so x + (-1) * hi stays
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   const long long rec0 = (long long)g * a.kv_head_stride;
   const float lscale = a.softmax_scale * kLog2e;
 
-  // the codebook (for decoding) and the sign-nibble table (QJL correction)
+  // the codebook (for decoding)
   if (tid < 16) {
     if (PH != kStaged) {
       constexpr int CM = (1 << CB) - 1;
@@ -254,8 +254,14 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
       }
       s_cb[tid] = c;
     }
-    auto pm1 = [&](int bit) { return ((tid >> bit) & 1) ? 0x3C00u : 0xBC00u; };
-    s_nib[tid] = make_uint2(pm1(0) | (pm1(1) << 16), pm1(2) | (pm1(3) << 16));
+  }
+  // +-1 in f16 for the eight sign bits of a byte, LSB first (bit set: +1):
+  // one 16-byte read per byte
+  if constexpr (QJL && PH != kStage) {
+    if (tid < 256) {
+      auto pm1 = [&](int bit) { return ((tid >> bit) & 1) ? 0x3C00u : 0xBC00u; };
+      s_sign[tid] = u32x4{pm1(0) | (pm1(1) << 16), pm1(2) | (pm1(3) << 16), pm1(4) | (pm1(5) << 16), pm1(6) | (pm1(7) << 16)};
+    }
   }
 
   // thread (token, qblock) fetches one record of K and V per tile
@@ -744,9 +750,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
         const uint32_t *sgrow = s_sg[cur] + (16 * tb + l16) * 4;
 #pragma unroll
         for (int sl = 0; sl < 4; sl++) {
-          const uint32_t byte = (sgrow[sl] >> (8 * lg)) & 0xffu;
-          const uint2 n0 = s_nib[byte & 15u], n1 = s_nib[byte >> 4];
-          const u32x4 sa = {n0.x, n0.y, n1.x, n1.y};
+          const u32x4 sa = s_sign[__builtin_amdgcn_ubfe(sgrow[sl], 8 * lg, 8)];
           dc = mfma(sa, rop[sl][0], dc);
           dc = mfma(sa, rop[sl][1], dc);
         }
