@@ -675,6 +675,9 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   const float er_scale = QJL ? exp2i(s_er[myrow]) : 0.f;
   const int qpos = a.kv_len - a.q_len + my_qi;  // causal limit of this row
   const int qmin = a.kv_len - a.q_len + i0;     // the workgroup's first query position
+  // this lane's tokens 4 lg + 16 tb + i of a tile at t0 are visible to its row
+  // below row_end: t0 + 4 lg + 16 tb + i < the row's end
+  const int row_end = (my_ok ? (a.causal ? min(a.kv_len, qpos + 1) : a.kv_len) : 0) - 4 * lg;
   __syncthreads();  // operands built: the tiles may overwrite the query staging
 
   // ---- tiles ----
@@ -742,34 +745,38 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
 #pragma unroll
       for (int tb = 0; tb < 4; tb++) dk[tb] = mfma(al[tb], qop[s][0], dk[tb]);
     }
+    f32x4 dc[4];
+    if constexpr (QJL) {
+#pragma unroll
+      for (int tb = 0; tb < 4; tb++) dc[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int sl = 0; sl < 4; sl++) {
+        u32x4 sa[4];
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++)
+          sa[tb] = s_sign[__builtin_amdgcn_ubfe(s_sg[cur][(16 * tb + l16) * 4 + sl], 8 * lg, 8)];
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++) dc[tb] = mfma(sa[tb], rop[sl][0], dc[tb]);
+#pragma unroll
+        for (int tb = 0; tb < 4; tb++) dc[tb] = mfma(sa[tb], rop[sl][1], dc[tb]);
+      }
+    }
 #pragma unroll
     for (int tb = 0; tb < 4; tb++) {
-      const f32x4 d = dk[tb];
-      f32x4 dc = f32x4{0.f, 0.f, 0.f, 0.f};
-      if constexpr (QJL) {
-        const uint32_t *sgrow = s_sg[cur] + (16 * tb + l16) * 4;
-#pragma unroll
-        for (int sl = 0; sl < 4; sl++) {
-          const u32x4 sa = s_sign[__builtin_amdgcn_ubfe(sgrow[sl], 8 * lg, 8)];
-          dc = mfma(sa, rop[sl][0], dc);
-          dc = mfma(sa, rop[sl][1], dc);
-        }
-      }
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         // without QJL the slice's 2^E_k and the row's 2^E_q are applied in the softmax
-        float v = QJL ? d[i] * (exp2i(ekt[tb]) * eqz) : d[i];
-        if constexpr (QJL) v = __builtin_fmaf(dc[i], s_cn[cur][16 * tb + 4 * lg + i] * er_scale, v);
+        float v = QJL ? dk[tb][i] * (exp2i(ekt[tb]) * eqz) : dk[tb][i];
+        if constexpr (QJL) v = __builtin_fmaf(dc[tb][i], s_cn[cur][16 * tb + 4 * lg + i] * er_scale, v);
         x[tb][i] = v;
       }
-      // the mask, in place, for tiles that are not open to every row
-      if (!(open && wave_rows_ok)) {
+    }
+    // the mask, in place, for tiles that are not open to every row
+    if (!(open && wave_rows_ok)) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int tp = t0 + 16 * tb + 4 * lg + i;
-          const bool ok = my_ok && (open || (tp < a.kv_len && (!a.causal || tp <= qpos)));
-          x[tb][i] = ok ? x[tb][i] : -INFINITY;
-        }
+      for (int tb = 0; tb < 4; tb++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[tb][i] = 16 * tb + i < row_end - t0 ? x[tb][i] : -INFINITY;
       }
     }
     // ---- online softmax of this row (its 64 logits sit in the 4 lanes l16 + 16 k) ----
