@@ -1,0 +1,58 @@
+"""Staged prefill tiles whose waves work in pairs, each pair on 32 rows and
+each wave of it on half of every tile: halves that no row sees (sequences and
+causal rows that end in a tile's first half), ragged last rows of a pair, and
+rows whose two halves hold very different maxima, against the oracle in
+double.  Tolerance 1e-3 max-abs, as for every prefill (fp32 accumulation, f16
+two-part operands)."""
+import math
+
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from tq_testdata import bf16_bits, bf16_round, kv_outlier
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+D = 128
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("bits,outlier,hq,hkv,ql,t,causal,peak", [
+    (3, orc.OUTLIER_ALL, 2, 1, 1, 20, True, None),     # nothing in the only tile's second half
+    (4, orc.OUTLIER_ALL, 4, 1, 9, 64 + 32, False, None),  # the last tile's second half is empty
+    (3, 0, 2, 2, 97, 97, True, None),                  # causal rows that end in either half; ragged rows
+    (4, 0, 1, 1, 130, 193, True, None),                # one row of a second workgroup
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 130, False, 5),     # the maximum in a first half
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 130, False, 64 + 40),  # and in a second half
+])
+@pytest.mark.parametrize("qdt", ["bf16", "f32"])
+def test_staged_row_pairs(monkeypatch, bits, outlier, hq, hkv, ql, t, causal, peak, qdt):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import turboquant_amd as tq
+    rng = np.random.default_rng(4100 + 7 * t + ql)
+    k, v = kv_outlier(rng, hkv, t), kv_outlier(rng, hkv, t)
+    q = rng.standard_normal((hq, ql, D)).astype(np.float32) / np.float32(math.sqrt(D))
+    scale = 1 / math.sqrt(D)
+    if peak is not None:
+        k[:, peak] = 30.0 * q[0, 0] / np.linalg.norm(q[0, 0])
+        q[:] = q[0, 0] * 20.0
+    q = bf16_round(q)
+    recs, deq = [], []
+    for x in (k, v):
+        p, s = orc.polar_quantize(bits, outlier, x.reshape(-1, D), D)
+        deq.append(orc.polar_dequantize(bits, outlier, p, s, D).reshape(hkv, t, D))
+        recs += [_dev(p.reshape(hkv, t, -1)), _dev(s.reshape(hkv, t, 4).view(np.int16))]
+    qd = _dev(bf16_bits(q)).view(torch.bfloat16) if qdt == "bf16" else _dev(q)
+    monkeypatch.setenv("TQ_PREFILL_STAGING", "1")
+    out = tq.cache_prefill_attention(qd, recs[0], recs[1], recs[2], recs[3], hkv, bits, t, t, scale, outlier,
+                                     causal=causal)
+    torch.cuda.synchronize()
+    ref = orc.attention_prefill(q, deq[0], deq[1], scale, causal)
+    err = np.abs(out.float().cpu().numpy() - ref).max()
+    assert err <= 1e-3, err

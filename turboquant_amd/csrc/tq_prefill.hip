@@ -13,7 +13,8 @@
 // decoded tile.  Per 64-token tile the
 // workgroup decodes K and V (token-major, one K and one V exponent per
 // 16-token slice folded out) into LDS as two-part f16 values (hi = 11
-// significant bits, lo = the remainder), then each wave (16 rows) runs
+// significant bits, lo = the remainder), then each wave (16 rows of
+// every token; staged PQO and PQ tiles: 32 rows of half the tokens) runs
 //   S^T = K Q^T          16x16x32 MFMAs per 32-element slice: K hi x Q hi,
 //                        K hi x Q lo, K lo x Q hi (22-bit products, lo x lo
 //                        dropped, f32 accumulation; staged tiles with a bf16
@@ -24,9 +25,9 @@
 //                        lane and block), the V operand read through the
 //                        transposing LDS read, V hi/lo x P hi/lo (three
 //                        products, lo x lo dropped)
-// with an online base-2 softmax per row.  The four 16-token blocks of the
-// key pass and pairs of 16-element blocks of the value pass run as
-// independent accumulator chains, interleaved (each accumulator still sums
+// with an online base-2 softmax per row.  The four accumulators of the key
+// pass (and of the QJL correction) and pairs of 16-element blocks of the
+// value pass run as independent chains, interleaved (each accumulator still sums
 // its products in the same order); the value pass runs at raised wave
 // priority.  Values stay in the rotated domain; each
 // row is inverse-rotated once at the end.  Two tile buffers: tile t + 1 is
@@ -91,9 +92,9 @@ constexpr int kORow = 128 + 4;  // floats
 // must repay: each tile is decoded by up to q_blocks workgroups otherwise;
 // 16/8 heads, bf16 queries, both paths split over the tiles where the grid
 // is small, in-workgroup vs staged, us: 128 causal queries at the end of
-// 32768 tokens 135.8 vs 184.5, 256 x 32768 236.6 vs 261.8, 256 x 8192 80.9
-// vs 80.0, 512 x 32768 450.7 vs 428.1; without splits 512 x 512 causal 36.1
-// vs 36.1, 768 x 768 causal 49.1 vs 45.8, 2048 x 2048 causal 117.3 vs 93.8)
+// 32768 tokens 125.6 vs 160.3, 256 x 32768 227.8 vs 233.5, 256 x 8192 76.6
+// vs 75.1, 512 x 32768 436.6 vs 393.3; without splits 512 x 512 causal 30.5
+// vs 34.0, 768 x 768 causal 44.3 vs 43.8, 2048 x 2048 causal 112.1 vs 90.8)
 constexpr int kStagingMinQueryBlocks = 6;
 constexpr int kStagingMinTokens = 768;
 // A staged tile image: the tile buffer's K rows and V planes, then its
@@ -182,6 +183,18 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   constexpr int SPLIT = NW / 4;             // waves per 16-token slice of a tile's decode
   constexpr int NP = 16 / SPLIT;            // code pairs per decoding thread
   constexpr int QB = kRows / NR;  // queries per workgroup
+  // 16-row groups per wave.  2: waves 2 k and 2 k + 1 share rows 32 k .. + 31,
+  // each takes half of every tile's tokens with its own running maximum, and
+  // the halves are added at the end: each K and V operand read from LDS then
+  // serves two groups' products (an 8-wave workgroup reads 256 KiB of tile per
+  // tile instead of 512).  Staged PQO and PQ: 4096 causal queries, 16 / 8 heads
+  // 198 -> 187 us, 512 x 32768 422 -> 394 us (one exchange of 64 KiB at the end: 1024
+  // queries 54.1 -> 53.7).  Not for tiles decoded in the workgroup (77 x 77
+  // 14.3 -> 16.5 us, 512 x 512 44.7 -> 46.9: the tile's decode is what the
+  // registers are needed for) and not for TQ (its rq operands too would need
+  // 130 registers more than a wave has at 8 waves).
+  constexpr int RG = !QJL && PH == kStaged ? 2 : 1;
+  constexpr int TBN = 4 / RG;           // the wave's 16-token blocks of a tile
   // LDS: K tile | V tiles (hi, lo) per buffer; slice exponents, TQ sign
   // words and norms, and per-row scalars beside them
   constexpr int K_WORDS = kTile * kKStride * 2;
@@ -256,7 +269,10 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
     }
   }
   // +-1 in f16 for the eight sign bits of a byte, LSB first (bit set: +1):
-  // one 16-byte read per byte
+  // one 16-byte read per byte and operand (two 8-byte reads by nibble: 500
+  // queries x 20,001 tokens, 32 heads 695 -> 658 us; two vector operations per
+  // word from the bits themselves: slower than the nibbles, the loop's vector
+  // instructions are its bound)
   if constexpr (QJL && PH != kStage) {
     if (tid < 256) {
       auto pm1 = [&](int bit) { return ((tid >> bit) & 1) ? 0x3C00u : 0xBC00u; };
@@ -637,57 +653,64 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   }
   __syncthreads();
 
-  // ---- per-wave operands for its 16 rows (lane column = row 16 wave + l16) ----
-  const int myrow = 16 * wave + l16;
+  // ---- per-wave operands for its RG groups of 16 rows (lane column = row
+  // row0 + 16 rg + l16) ----
+  const int row0 = RG * 16 * (wave / RG) + l16;
+  const int tb0 = __builtin_amdgcn_readfirstlane(TBN * (wave % RG));  // the wave's first 16-token block
   // per 32-element slice s, lane (row, lg) holds elements 32 s + 8 lg .. + 7
   // of its row, hi and lo
-  u32x4 qop[4][2];
+  u32x4 qop[RG][4][2];
+  u32x4 rop[QJL ? RG : 1][4][2];
 #pragma unroll
-  for (int s = 0; s < 4; s++) {
-    const int e = myrow * kQRow + 32 * s + 8 * lg;
-    const uint4 h = *reinterpret_cast<const uint4 *>(s_qh + e);
-    const uint4 l = *reinterpret_cast<const uint4 *>(s_ql + e);
-    qop[s][0] = u32x4{h.x, h.y, h.z, h.w};
-    qop[s][1] = u32x4{l.x, l.y, l.z, l.w};
-  }
-  u32x4 rop[4][2];
-  if constexpr (QJL) {
+  for (int rg = 0; rg < RG; rg++)
 #pragma unroll
-    for (int sl = 0; sl < 4; sl++) {
-      const int e = myrow * kQRow + 32 * sl + 8 * lg;
-      const uint4 h = *reinterpret_cast<const uint4 *>(s_rh + e);
-      const uint4 l = *reinterpret_cast<const uint4 *>(s_rl + e);
-      rop[sl][0] = u32x4{h.x, h.y, h.z, h.w};
-      rop[sl][1] = u32x4{l.x, l.y, l.z, l.w};
+    for (int s = 0; s < 4; s++) {
+      const int e = (row0 + 16 * rg) * kQRow + 32 * s + 8 * lg;
+      qop[rg][s][0] = *reinterpret_cast<const u32x4 *>(s_qh + e);
+      qop[rg][s][1] = *reinterpret_cast<const u32x4 *>(s_ql + e);
+      if constexpr (QJL) {
+        rop[rg][s][0] = *reinterpret_cast<const u32x4 *>(s_rh + e);
+        rop[rg][s][1] = *reinterpret_cast<const u32x4 *>(s_rl + e);
+      }
     }
-  }
-  const int my_qi = i0 + myrow / NR;
-  const bool my_ok = my_qi < a.q_len;
-  const bool wave_rows_ok = __all(my_ok);  // every row of the wave is a query
-  const float eq_scale = exp2i(s_eq[myrow]);
   // the row's factor on the key products: 2^E_q (staged: times the softmax
   // scale, which the unrotated query does not carry)
-  const float eqz = ORIG ? eq_scale * lscale : eq_scale;
+  float eqz[RG], er_scale[RG];
+  // this lane's tokens 16 tb + 4 lg + i of a tile at t0 are visible to its
+  // row below the row's end: 16 tb + i < row_end - t0
+  int row_end[RG];
+  bool rows_ok = true;
+#pragma unroll
+  for (int rg = 0; rg < RG; rg++) {
+    const int myrow = row0 + 16 * rg, my_qi = i0 + myrow / NR;
+    const bool my_ok = my_qi < a.q_len;
+    const int qpos = a.kv_len - a.q_len + my_qi;  // causal limit of this row
+    eqz[rg] = exp2i(s_eq[myrow]) * (ORIG ? lscale : 1.f);
+    er_scale[rg] = QJL ? exp2i(s_er[myrow]) : 0.f;
+    row_end[rg] = (my_ok ? (a.causal ? min(a.kv_len, qpos + 1) : a.kv_len) : 0) - 4 * lg - 16 * tb0;
+    rows_ok = rows_ok && my_ok;
+  }
+  const bool wave_rows_ok = __all(rows_ok);  // every row of the wave is a query
   // the product with the query's lo part: every query in the workgroup's
   // decode, f32 queries on staged tiles (a bf16 or f16 query scaled by 2^-E_q
   // is exact in f16 down to 2^-24 of the row's maximum)
   const bool q_lo = !ORIG || a.q_dtype == kF32;
-  const float er_scale = QJL ? exp2i(s_er[myrow]) : 0.f;
-  const int qpos = a.kv_len - a.q_len + my_qi;  // causal limit of this row
   const int qmin = a.kv_len - a.q_len + i0;     // the workgroup's first query position
-  // this lane's tokens 4 lg + 16 tb + i of a tile at t0 are visible to its row
-  // below row_end: t0 + 4 lg + 16 tb + i < the row's end
-  const int row_end = (my_ok ? (a.causal ? min(a.kv_len, qpos + 1) : a.kv_len) : 0) - 4 * lg;
   __syncthreads();  // operands built: the tiles may overwrite the query staging
 
   // ---- tiles ----
 
 
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run[RG], l_run[RG];
   int ev_cur = -1000;
-  f32x4 o[8];
+  f32x4 o[RG][8];
 #pragma unroll
-  for (int eb = 0; eb < 8; eb++) o[eb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int rg = 0; rg < RG; rg++) {
+    m_run[rg] = -INFINITY;
+    l_run[rg] = 0.f;
+#pragma unroll
+    for (int eb = 0; eb < 8; eb++) o[rg][eb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   if (tile_hi > tile_lo) {
     decode_tile(0);
@@ -713,87 +736,92 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
     // a tile wholly before the workgroup's first query position (and inside
     // the sequence) is visible to every row: no per-element mask
     const bool open = t0 + kTile <= a.kv_len && (!a.causal || t0 + kTile - 1 <= qmin);
-    float x[4][4];
     // the tile's slice exponents (wave-uniform)
-    int ekt[4];
+    int ekt[TBN];
     {
       const int4 e4 = *reinterpret_cast<const int4 *>(s_xe[cur]);
-      ekt[0] = __builtin_amdgcn_readfirstlane(e4.x);
-      ekt[1] = __builtin_amdgcn_readfirstlane(e4.y);
-      ekt[2] = __builtin_amdgcn_readfirstlane(e4.z);
-      ekt[3] = __builtin_amdgcn_readfirstlane(e4.w);
+      if constexpr (RG == 1) {
+        ekt[0] = __builtin_amdgcn_readfirstlane(e4.x);
+        ekt[1] = __builtin_amdgcn_readfirstlane(e4.y);
+        ekt[TBN - 2] = __builtin_amdgcn_readfirstlane(e4.z);
+        ekt[TBN - 1] = __builtin_amdgcn_readfirstlane(e4.w);
+      } else {
+        ekt[0] = __builtin_amdgcn_readfirstlane(tb0 ? e4.z : e4.x);
+        ekt[1] = __builtin_amdgcn_readfirstlane(tb0 ? e4.w : e4.y);
+      }
     }
-    f32x4 dk[4];
+    f32x4 x[RG][TBN];
 #pragma unroll
-    for (int tb = 0; tb < 4; tb++) dk[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+      for (int tb = 0; tb < TBN; tb++) x[rg][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; s++) {
-      u32x4 ah[4], al[4];
+      u32x4 ah[TBN], al[TBN];
 #pragma unroll
-      for (int tb = 0; tb < 4; tb++) {
-        const uint4 *krow = reinterpret_cast<const uint4 *>(kt + (16 * tb + l16) * kKStride);
-        const uint4 kh = krow[kchunk(8 * s + 2 * lg, l16)], kl = krow[kchunk(8 * s + 2 * lg + 1, l16)];
-        ah[tb] = u32x4{kh.x, kh.y, kh.z, kh.w};
-        al[tb] = u32x4{kl.x, kl.y, kl.z, kl.w};
+      for (int tb = 0; tb < TBN; tb++) {
+        const u32x4 *krow = reinterpret_cast<const u32x4 *>(kt + (16 * (tb0 + tb) + l16) * kKStride);
+        ah[tb] = krow[kchunk(8 * s + 2 * lg, l16)];
+        al[tb] = krow[kchunk(8 * s + 2 * lg + 1, l16)];
       }
 #pragma unroll
-      for (int tb = 0; tb < 4; tb++) dk[tb] = mfma(ah[tb], qop[s][0], dk[tb]);
+      for (int tb = 0; tb < TBN; tb++)
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++) x[rg][tb] = mfma(ah[tb], qop[rg][s][0], x[rg][tb]);
       if (q_lo) {
 #pragma unroll
-        for (int tb = 0; tb < 4; tb++) dk[tb] = mfma(ah[tb], qop[s][1], dk[tb]);
+        for (int tb = 0; tb < TBN; tb++)
+#pragma unroll
+          for (int rg = 0; rg < RG; rg++) x[rg][tb] = mfma(ah[tb], qop[rg][s][1], x[rg][tb]);
       }
 #pragma unroll
-      for (int tb = 0; tb < 4; tb++) dk[tb] = mfma(al[tb], qop[s][0], dk[tb]);
-    }
-    f32x4 dc[4];
-    if constexpr (QJL) {
+      for (int tb = 0; tb < TBN; tb++)
 #pragma unroll
-      for (int tb = 0; tb < 4; tb++) dc[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int rg = 0; rg < RG; rg++) x[rg][tb] = mfma(al[tb], qop[rg][s][0], x[rg][tb]);
+    }
+    if constexpr (QJL) {
+      f32x4 dc[RG][TBN];
+#pragma unroll
+      for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+        for (int tb = 0; tb < TBN; tb++) dc[rg][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int sl = 0; sl < 4; sl++) {
-        u32x4 sa[4];
+        u32x4 sa[TBN];
 #pragma unroll
-        for (int tb = 0; tb < 4; tb++)
-          sa[tb] = s_sign[__builtin_amdgcn_ubfe(s_sg[cur][(16 * tb + l16) * 4 + sl], 8 * lg, 8)];
+        for (int tb = 0; tb < TBN; tb++)
+          sa[tb] = s_sign[__builtin_amdgcn_ubfe(s_sg[cur][(16 * (tb0 + tb) + l16) * 4 + sl], 8 * lg, 8)];
 #pragma unroll
-        for (int tb = 0; tb < 4; tb++) dc[tb] = mfma(sa[tb], rop[sl][0], dc[tb]);
+        for (int part = 0; part < 2; part++)
 #pragma unroll
-        for (int tb = 0; tb < 4; tb++) dc[tb] = mfma(sa[tb], rop[sl][1], dc[tb]);
+          for (int tb = 0; tb < TBN; tb++)
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++) dc[rg][tb] = mfma(sa[tb], rop[rg][sl][part], dc[rg][tb]);
       }
-    }
+      // (without QJL the slice's 2^E_k and the row's 2^E_q are applied in the softmax)
 #pragma unroll
-    for (int tb = 0; tb < 4; tb++) {
+      for (int tb = 0; tb < TBN; tb++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        // without QJL the slice's 2^E_k and the row's 2^E_q are applied in the softmax
-        float v = QJL ? dk[tb][i] * (exp2i(ekt[tb]) * eqz) : dk[tb][i];
-        if constexpr (QJL) v = __builtin_fmaf(dc[tb][i], s_cn[cur][16 * tb + 4 * lg + i] * er_scale, v);
-        x[tb][i] = v;
-      }
+        for (int rg = 0; rg < RG; rg++) {
+          const float zk = exp2i(ekt[tb]) * eqz[rg];
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            x[rg][tb][i] = __builtin_fmaf(dc[rg][tb][i], s_cn[cur][16 * (tb0 + tb) + 4 * lg + i] * er_scale[rg],
+                                          x[rg][tb][i] * zk);
+        }
     }
-    // the mask, in place, for tiles that are not open to every row
+    // the mask, for tiles that are not open to every row: one pass outside
+    // the products, whose chains a branch per block would part (with the QJL
+    // chains interleaved, 500 x 20,001: 658 -> 619 us)
     if (!(open && wave_rows_ok)) {
 #pragma unroll
-      for (int tb = 0; tb < 4; tb++) {
+      for (int rg = 0; rg < RG; rg++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) x[tb][i] = 16 * tb + i < row_end - t0 ? x[tb][i] : -INFINITY;
-      }
+        for (int tb = 0; tb < TBN; tb++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) x[rg][tb][i] = 16 * tb + i < row_end[rg] - t0 ? x[rg][tb][i] : -INFINITY;
     }
-    // ---- online softmax of this row (its 64 logits sit in the 4 lanes l16 + 16 k) ----
-    // logit = x z_tb, z_tb = 2^E_k,tb 2^E_q (a power of 2, exact; staged
-    // tiles: times the softmax scale) (QJL: 1)
-    float zt[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; tb++) zt[tb] = QJL ? 1.f : exp2i(ekt[tb]) * eqz;
-    float mt = -INFINITY;
-#pragma unroll
-    for (int tb = 0; tb < 4; tb++)
-      mt = fmaxf(mt, fmaxf(fmaxf(x[tb][0], x[tb][1]), fmaxf(x[tb][2], x[tb][3])) * zt[tb]);
-    mt = max_xor32(max_xor16(mt));
-    const float m_new = fmaxf(m_run, mt);
-    const float m_exp = m_new == -INFINITY ? 0.f : m_new;  // a row with nothing visible yet
-    const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
-    // V exponent of the tile (each wave reads all 64)
+    // V exponents of the tile
     static_assert(NW % 4 == 0, "the wave exponents are read 4 at a time");
     int evw[NW];
 #pragma unroll
@@ -808,38 +836,59 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
 #pragma unroll
     for (int w = 0; w < NW; w++) evt = max(evt, evw[w]);
     const int ev_new = max(ev_cur, evt);
-    const float rescale = alpha * exp2i(max(ev_cur - ev_new, -126));
+    const float ev_rescale = exp2i(max(ev_cur - ev_new, -126));
     ev_cur = ev_new;
-    m_run = m_new;
-    float ls = 0.f;
-    u32x2 pb[4][2];
+    int dv[TBN];
 #pragma unroll
-    for (int tb = 0; tb < 4; tb++) {
-      // p = e 2^(E_v,tb - Ev) with e = 2^(logit - m): the slice's V factor is
-      // a shift of exp2's argument (E_v,tb - Ev in [-40, 0]: p stays normal
-      // for every e above 2^-80), and e = p 2^(Ev - E_v,tb) for the row sum
-      const int dv = evw[SPLIT * tb] - ev_new;
-      const float cb = (float)dv - m_exp, gb = exp2i(-dv);
-      float p[4];
+    for (int tb = 0; tb < TBN; tb++) dv[tb] = (RG == 1 || tb0 == 0 ? evw[SPLIT * tb] : evw[SPLIT * (4 - TBN + tb)]) - ev_new;
+    // ---- online softmax of each row (its 16 TBN logits sit in the 4 lanes l16 + 16 k) ----
+    // logit = x z_tb, z_tb = 2^E_k,tb 2^E_q (a power of 2, exact; staged
+    // tiles: times the softmax scale) (QJL: 1)
+    u32x2 pb[RG][TBN][2];
+    float rescale[RG];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[tb][i], zt[tb], cb));  // 2^-inf = 0 for masked tokens
-        ls = __builtin_fmaf(p[i], gb, ls);
+    for (int rg = 0; rg < RG; rg++) {
+      float zt[TBN];
+#pragma unroll
+      for (int tb = 0; tb < TBN; tb++) zt[tb] = QJL ? 1.f : exp2i(ekt[tb]) * eqz[rg];
+      float mt = -INFINITY;
+#pragma unroll
+      for (int tb = 0; tb < TBN; tb++)
+        mt = fmaxf(mt, fmaxf(fmaxf(x[rg][tb][0], x[rg][tb][1]), fmaxf(x[rg][tb][2], x[rg][tb][3])) * zt[tb]);
+      mt = max_xor32(max_xor16(mt));
+      const float m_new = fmaxf(m_run[rg], mt);
+      const float m_exp = m_new == -INFINITY ? 0.f : m_new;  // a row with nothing visible yet
+      const float alpha = (m_run[rg] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run[rg] - m_new);
+      rescale[rg] = alpha * ev_rescale;
+      m_run[rg] = m_new;
+      float ls = 0.f;
+#pragma unroll
+      for (int tb = 0; tb < TBN; tb++) {
+        // p = e 2^(E_v,tb - Ev) with e = 2^(logit - m): the slice's V factor is
+        // a shift of exp2's argument (E_v,tb - Ev in [-40, 0]: p stays normal
+        // for every e above 2^-80), and e = p 2^(Ev - E_v,tb) for the row sum
+        const float cb = (float)dv[tb] - m_exp, gb = exp2i(-dv[tb]);
+        float p[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[rg][tb][i], zt[tb], cb));  // 2^-inf = 0 for masked tokens
+          ls = __builtin_fmaf(p[i], gb, ls);
+        }
+        pb[rg][tb][0] = u32x2{pack_f16(p[0], p[1]), pack_f16(p[2], p[3])};
+        pb[rg][tb][1] = u32x2{pack_rem(p[0], p[1], pb[rg][tb][0][0], mone), pack_rem(p[2], p[3], pb[rg][tb][0][1], mone)};
       }
-      pb[tb][0] = u32x2{pack_f16(p[0], p[1]), pack_f16(p[2], p[3])};
-      pb[tb][1] = u32x2{pack_rem(p[0], p[1], pb[tb][0][0], mone), pack_rem(p[2], p[3], pb[tb][0][1], mone)};
+      l_run[rg] = l_run[rg] * alpha + ls;
+      // the accumulators' rescale, skipped when every row's factor is 1
+      if (!__all(rescale[rg] == 1.f)) {
+#pragma unroll
+        for (int eb = 0; eb < 8; eb++) o[rg][eb] = o[rg][eb] * rescale[rg];
+      }
     }
-    l_run = l_run * alpha + ls;
     // ---- O^T += V^T P^T, two 16-token blocks per 16x16x32 product.  The
     // value operand comes through the transposing LDS read: lane (4 a + b)
     // of group lg receives element 16 eb + 4 a + b of tokens 16 tb + 4 lg ..
     // + 3 from the token-major rows addressed by lanes a + 4 j. ----
-    const int vrow = 4 * lg + (l16 >> 2), vcol = 4 * (l16 & 3);
-    // the accumulators' rescale, skipped when every row's factor is 1
-    if (!__all(rescale == 1.f)) {
-#pragma unroll
-      for (int eb = 0; eb < 8; eb++) o[eb] = o[eb] * rescale;
-    }
+    const int vrow = 16 * tb0 + 4 * lg + (l16 >> 2), vcol = 4 * (l16 & 3);
     // the value pass at raised issue priority: the SIMD's other wave, often
     // in its softmax, fills the matrix products' gaps instead of delaying
     // them (0.2401 -> 0.2365 ms at the bench shape; the key pass gains nothing)
@@ -847,9 +896,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
 #pragma unroll
     for (int e2 = 0; e2 < 8; e2 += 2) {
 #pragma unroll
-      for (int tp = 0; tp < 2; tp++) {
-        const u32x4 bh = {pb[2 * tp][0][0], pb[2 * tp][0][1], pb[2 * tp + 1][0][0], pb[2 * tp + 1][0][1]};
-        const u32x4 bl = {pb[2 * tp][1][0], pb[2 * tp][1][1], pb[2 * tp + 1][1][0], pb[2 * tp + 1][1][1]};
+      for (int tp = 0; tp < TBN / 2; tp++) {
         u32x4 ah[2], al[2];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -861,12 +908,20 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
           ah[j] = u32x4{h0[0], h0[1], h1[0], h1[1]};
           al[j] = u32x4{q0[0], q0[1], q1[0], q1[1]};
         }
-        o[e2] = mfma(ah[0], bh, o[e2]);
-        o[e2 + 1] = mfma(ah[1], bh, o[e2 + 1]);
-        o[e2] = mfma(ah[0], bl, o[e2]);
-        o[e2 + 1] = mfma(ah[1], bl, o[e2 + 1]);
-        o[e2] = mfma(al[0], bh, o[e2]);
-        o[e2 + 1] = mfma(al[1], bh, o[e2 + 1]);
+        u32x4 bp[RG][2];
+#pragma unroll
+        for (int rg = 0; rg < RG; rg++)
+#pragma unroll
+          for (int part = 0; part < 2; part++)
+            bp[rg][part] = u32x4{pb[rg][2 * tp][part][0], pb[rg][2 * tp][part][1], pb[rg][2 * tp + 1][part][0],
+                                 pb[rg][2 * tp + 1][part][1]};
+#pragma unroll
+        for (int part = 0; part < 3; part++)  // hi hi, hi lo, lo hi
+#pragma unroll
+          for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int rg = 0; rg < RG; rg++)
+              o[rg][e2 + j] = mfma(part < 2 ? ah[j] : al[j], bp[rg][part & 1], o[rg][e2 + j]);
       }
     }
     __builtin_amdgcn_s_setprio(0);
@@ -878,20 +933,49 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   }
 
   // ---- finish: row sums, inverse rotation per 32-element block, store ----
-  float L = l_run;
-  L += __shfl_xor(L, 16, 64);
-  L += __shfl_xor(L, 32, 64);
   float *s_o = reinterpret_cast<float *>(s_tile);  // [row][kORow] (rotated, in units of 2^ev_cur)
-  const float ofac = exp2i(max(min(ev_cur, 126), -126));
-#pragma unroll
-  for (int eb = 0; eb < 8; eb++)
-    *reinterpret_cast<float4 *>(s_o + myrow * kORow + 16 * eb + 4 * lg) =
-        make_float4(o[eb][0] * ofac, o[eb][1] * ofac, o[eb][2] * ofac, o[eb][3] * ofac);
   float *s_rowl = s_o + kRows * kORow;  // [rows] (the tiles are done)
   float *s_rowm = s_rowl + kRows;
-  if (lg == 0) {
-    s_rowl[myrow] = L;
-    s_rowm[myrow] = m_run;
+  const float ofac = exp2i(max(min(ev_cur, 126), -126));
+  // RG == 2: each wave of a pair leaves its half's sums of the group that the
+  // other one finishes, then adds the other's to its own on the common
+  // maximum (2^0 where a half saw nothing: its sums are 0).  Step 0 leaves,
+  // step 1 finishes; with one group per wave there is only step 1.
+#pragma unroll
+  for (int step = RG == 2 ? 0 : 1; step < 2; step++) {
+#pragma unroll
+    for (int rg = 0; rg < RG; rg++) {
+      if (RG == 2 && (wave % RG == rg) != (step == 1)) continue;
+      const int myrow = row0 + 16 * rg;
+      const bool add = RG == 2 && step == 1;
+      float L = l_run[rg], M = m_run[rg], own = ofac, oth = 0.f;
+      L += __shfl_xor(L, 16, 64);
+      L += __shfl_xor(L, 32, 64);
+      if (add) {
+        const float m1 = s_rowm[myrow];
+        M = fmaxf(m_run[rg], m1);
+        const float w0 = m_run[rg] == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run[rg] - M);
+        oth = m1 == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m1 - M);
+        L = __builtin_fmaf(s_rowl[myrow], oth, L * w0);
+        own = ofac * w0;
+      }
+#pragma unroll
+      for (int eb = 0; eb < 8; eb++) {
+        f32x4 *po = reinterpret_cast<f32x4 *>(s_o + myrow * kORow + 16 * eb + 4 * lg);
+        f32x4 v = o[rg][eb] * own;
+        if (add) {
+          const f32x4 v1 = *po;
+#pragma unroll
+          for (int i = 0; i < 4; i++) v[i] = __builtin_fmaf(v1[i], oth, v[i]);
+        }
+        *po = v;
+      }
+      if (lg == 0) {
+        s_rowl[myrow] = L;
+        s_rowm[myrow] = M;
+      }
+    }
+    if (step == 0) __syncthreads();
   }
   __syncthreads();
   {
