@@ -17,9 +17,9 @@
 // leave the residual in LDS, then wave w sums rows 32 w .. + 31 of R for all
 // 16 (two chains, so neither waits for its own last step).  Bound by the
 // chains: D / 4 steps of 32 cycles for two tiles each, 0.9 us at D = 128;
-// launches bound a decode step's append, which took four (keys, values,
-// sketch with projection; two of them 3.8 us, one 4.0 us, 16 tokens) and now
-// takes one.
+// launches bound a short append (prefill, extension, a decode whose token the
+// attention launch does not store), which took three (keys, values, sketch
+// with projection: two of 3.8 us and one of 4.0 us, 16 tokens) and takes one.
 #include "tq_pqo_dev.h"
 
 #include <type_traits>
