@@ -22,16 +22,17 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-@pytest.mark.parametrize("bits,outlier,hq,hkv,ql,t,causal,peak", [
-    (3, orc.OUTLIER_ALL, 2, 1, 1, 20, True, None),     # nothing in the only tile's second half
-    (4, orc.OUTLIER_ALL, 4, 1, 9, 64 + 32, False, None),  # the last tile's second half is empty
-    (3, 0, 2, 2, 97, 97, True, None),                  # causal rows that end in either half; ragged rows
-    (4, 0, 1, 1, 130, 193, True, None),                # one row of a second workgroup
-    (3, orc.OUTLIER_ALL, 1, 1, 65, 130, False, 5),     # the maximum in a first half
-    (3, orc.OUTLIER_ALL, 1, 1, 65, 130, False, 64 + 40),  # and in a second half
+@pytest.mark.parametrize("bits,outlier,hq,hkv,ql,t,causal,peak,splits", [
+    (3, orc.OUTLIER_ALL, 2, 1, 1, 768 + 20, True, None, 1),     # nothing in the last tile's second half
+    (4, orc.OUTLIER_ALL, 4, 1, 9, 704 + 32, False, None, 1),    # 12 tiles, the last one's second half is empty
+    (4, 0, 4, 1, 9, 704, False, None, 1),                       # 11 tiles: one group per wave
+    (3, 0, 2, 2, 707, 707, True, None, 1),                      # causal rows that see one half only; ragged rows
+    (4, 0, 1, 1, 130, 1601, True, None, 2),                     # two splits of 13 tiles, one row of a second workgroup
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 5, 1),           # the maximum in a first half
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 64 + 40, 1),     # and in a second half
 ])
 @pytest.mark.parametrize("qdt", ["bf16", "f32"])
-def test_staged_row_pairs(monkeypatch, bits, outlier, hq, hkv, ql, t, causal, peak, qdt):
+def test_staged_row_pairs(monkeypatch, bits, outlier, hq, hkv, ql, t, causal, peak, splits, qdt):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     import turboquant_amd as tq
@@ -50,6 +51,7 @@ def test_staged_row_pairs(monkeypatch, bits, outlier, hq, hkv, ql, t, causal, pe
         recs += [_dev(p.reshape(hkv, t, -1)), _dev(s.reshape(hkv, t, 4).view(np.int16))]
     qd = _dev(bf16_bits(q)).view(torch.bfloat16) if qdt == "bf16" else _dev(q)
     monkeypatch.setenv("TQ_PREFILL_STAGING", "1")
+    monkeypatch.setenv("TQ_PREFILL_SPLITS", str(splits))
     out = tq.cache_prefill_attention(qd, recs[0], recs[1], recs[2], recs[3], hkv, bits, t, t, scale, outlier,
                                      causal=causal)
     torch.cuda.synchronize()

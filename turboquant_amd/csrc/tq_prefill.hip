@@ -96,6 +96,13 @@ constexpr int kORow = 128 + 4;  // floats
 // vs 75.1, 512 x 32768 436.6 vs 393.3; without splits 512 x 512 causal 30.5
 // vs 34.0, 768 x 768 causal 44.3 vs 43.8, 2048 x 2048 causal 112.1 vs 90.8)
 constexpr int kStagingMinQueryBlocks = 6;
+// Staged PQO and PQ tiles are taken by pairs of waves where the longest
+// workgroup walks at least this many: a pair saves half of a tile's LDS reads
+// and pays once for the second group's operands and the exchange of the
+// halves (one group per wave vs pairs, us: 64 tiles, 4096 x 4096 causal, 16 / 8
+// heads 198 vs 187; 32 tiles, 2048 x 2048 94.0 vs 90.7; 8 tiles, 1024 x 1024
+// 52.9 vs 53.7; 6 tiles, 768 x 768 42.8 vs 43.8)
+constexpr int kPairMinTiles = 12;
 constexpr int kStagingMinTokens = 768;
 // A staged tile image: the tile buffer's K rows and V planes, then its
 // exponent words (the slices' K exponents, the waves' V exponents), for a TQ
@@ -166,8 +173,9 @@ constexpr int kPartRow = 132;
 
 // Kernel phases: decode every tile in the workgroup (kDecode); the staging
 // pass, one workgroup per tile and KV head, which writes the tile's image
-// (kStage); read the tiles as those images (kStaged)
-enum PPhase : int { kDecode = 0, kStaged = 1, kStage = 2 };
+// (kStage); read the tiles as those images, each wave 16 rows of every token
+// (kStaged) or each pair of waves 32 rows, half of the tokens each (kPair)
+enum PPhase : int { kDecode = 0, kStaged = 1, kStage = 2, kPair = 3 };
 
 template <int BITS, int MODE, int NR, int PH>
 __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(PrefillArgs a) {
@@ -177,6 +185,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   // rotates it) and the query is taken as it is: a bf16 or f16 query is then
   // exact in f16 and the key pass needs no product with its lo part
   constexpr bool ORIG = PH != kDecode;
+  constexpr bool STG = PH == kStaged || PH == kPair;
   constexpr int HD = 128, QW = BITS, PACKED = 16 * QW;
   constexpr int kRows = prefill_rows(MODE);
   constexpr int NW = kRows / 16;            // waves
@@ -187,13 +196,12 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   // each takes half of every tile's tokens with its own running maximum, and
   // the halves are added at the end: each K and V operand read from LDS then
   // serves two groups' products (an 8-wave workgroup reads 256 KiB of tile per
-  // tile instead of 512).  Staged PQO and PQ: 4096 causal queries, 16 / 8 heads
-  // 198 -> 187 us, 512 x 32768 422 -> 394 us (one exchange of 64 KiB at the end: 1024
-  // queries 54.1 -> 53.7).  Not for tiles decoded in the workgroup (77 x 77
+  // tile instead of 512).  Not for tiles decoded in the workgroup (77 x 77
   // 14.3 -> 16.5 us, 512 x 512 44.7 -> 46.9: the tile's decode is what the
   // registers are needed for) and not for TQ (its rq operands too would need
   // 130 registers more than a wave has at 8 waves).
-  constexpr int RG = !QJL && PH == kStaged ? 2 : 1;
+  constexpr int RG = PH == kPair ? 2 : 1;
+  static_assert(RG == 1 || !QJL, "a wave's registers hold one group's rq operands");
   constexpr int TBN = 4 / RG;           // the wave's 16-token blocks of a tile
   // LDS: K tile | V tiles (hi, lo) per buffer; slice exponents, TQ sign
   // words and norms, and per-row scalars beside them
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
 
   // the codebook (for decoding)
   if (tid < 16) {
-    if (PH != kStaged) {
+    if (!STG) {
       constexpr int CM = (1 << CB) - 1;
       float c = a.cb[0];
       if (a.cb_args) {
@@ -292,7 +300,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   // staged: thread tid moves chunks tid + 4 kRows r of a tile image
   constexpr int IMG_ROUNDS = (IMG + 4 * kRows - 1) / (4 * kRows);
   // (native vectors: an array of uint4 structs stays in scratch memory)
-  u32x4 img[PH == kStaged ? IMG_ROUNDS : 1];
+  u32x4 img[STG ? IMG_ROUNDS : 1];
   // staged: KV head g's tile images as one buffer resource (scalar registers;
   // the host bounds a head's images below 2^31 bytes)
   auto make_img_rsrc = [&]() {
@@ -321,7 +329,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
     }
   };
   auto fetch = [&](int t0) {
-    if constexpr (PH == kStaged) {
+    if constexpr (STG) {
       // buffer loads: the lane's offset in a vector register (the same for
       // every tile), the tile's and the round's in a scalar register
       const uint32_t soff = (uint32_t)(t0 / kTile) * (uint32_t)(IMG * 16);
@@ -376,7 +384,7 @@ __global__ __launch_bounds__(4 * prefill_rows(MODE)) void prefill_attn_kernel(Pr
   // ---- decode this thread's record into tile buffer b (staged: store the
   // fetched image chunks) ----
   auto decode_tile = [&](int b) {
-    if constexpr (PH == kStaged) {
+    if constexpr (STG) {
 #pragma unroll
       for (int r = 0; r < IMG_ROUNDS; r++) {
         const int c = tid + 4 * kRows * r;
@@ -1195,7 +1203,10 @@ int launch_prefill_m(PrefillArgs &a, int nr, hipStream_t st) {
     a.stage_tpw = cus > 0 ? (int)max(1ll, (units + 2ll * cus - 1) / (2ll * cus)) : 1;
     const unsigned stage_wgs = (unsigned)((a.stage_tiles + a.stage_tpw - 1) / a.stage_tpw) * grid.y;
     hipLaunchKernelGGL((prefill_attn_kernel<BITS, MODE, 1, kStage>), dim3(stage_wgs), block, 0, st, a);
-    launch_attn<BITS, MODE, kStaged>(a, nr, grid, block, st);
+    if (MODE != kPTq && a.tps >= kPairMinTiles)
+      launch_attn<BITS, MODE, MODE == kPTq ? kStaged : kPair>(a, nr, grid, block, st);
+    else
+      launch_attn<BITS, MODE, kStaged>(a, nr, grid, block, st);
   } else {
     launch_attn<BITS, MODE, kDecode>(a, nr, grid, block, st);
   }
