@@ -448,8 +448,10 @@ constexpr int kWvQueries = 16;
 // of a lane that walks the chunk, for 16 queries x 16 elements at a time.
 // The scaled weights and the code words of the chunk are staged in LDS in the
 // order the steps take them (value 4 s + g at [g][s]), so one 16-byte read
-// feeds four steps.  64 queries x 8,192 values, d = 128, 2-bit codes: 16.7 us
-// with a lane per element and 4 queries per workgroup, 10.2 us now.
+// feeds four steps.  Bound by the latency of the staging: 128 workgroups of
+// 64 queries x 8,192 values, d = 128, 2-bit codes, take 16.7 us with a lane
+// per element and 4 queries per workgroup, 9.5 us with each staged value
+// loaded under its own bounds check, 6.3 us with all loads in flight at once.
 template <int D, int PB>
 __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__restrict__ polar,
                                                                const uint16_t *__restrict__ polar_scales,
@@ -466,16 +468,34 @@ __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__
   const long long t0 = (long long)blockIdx.x * kWvChunk, q0 = (long long)blockIdx.y * kWvQueries;
   const int cnt = (int)min<long long>(kWvChunk, nv - t0);
   if (tid < 16) s_cent[tid] = k.polar.cent[tid & ((1 << PB) - 1)];
-  for (int i = tid; i < kWvChunk * RW; i += THREADS) {
-    const int t = i / RW, w = i % RW;
-    s_codes[w][(t & 3) * GS + (t >> 2)] =
-        t < cnt ? reinterpret_cast<const uint32_t *>(polar + (t0 + t) * (D * PB / 8))[w] : 0u;
+  // every load goes out before the first is used; places past the end read
+  // the last value or query and are stored as zeros
+  constexpr int NC = kWvChunk * RW / THREADS, NWT = kWvChunk * kWvQueries / THREADS;
+  static_assert(NC * THREADS == kWvChunk * RW && NWT * THREADS == kWvChunk * kWvQueries, "whole rounds");
+  uint32_t cd[NC];
+  float wt[NWT];
+  uint16_t sc[NWT];
+#pragma unroll
+  for (int j = 0; j < NC; j++) {
+    const int i = tid + j * THREADS;
+    cd[j] = reinterpret_cast<const uint32_t *>(polar + (t0 + min(i / RW, cnt - 1)) * (D * PB / 8))[i % RW];
   }
-  for (int i = tid; i < kWvChunk * kWvQueries; i += THREADS) {
-    const int t = i % kWvChunk, qq = i / kWvChunk;
-    float w = 0.f;
-    if (t < cnt && q0 + qq < nq) w = weights[(q0 + qq) * nv + t0 + t] * f16_to_f32(polar_scales[t0 + t]);
-    s_w[qq][(t & 3) * GS + (t >> 2)] = w;
+#pragma unroll
+  for (int j = 0; j < NWT; j++) {
+    const int i = tid + j * THREADS;
+    const long long t = t0 + min(i % kWvChunk, cnt - 1);
+    wt[j] = weights[min<long long>(q0 + i / kWvChunk, nq - 1) * nv + t];
+    sc[j] = polar_scales[t];
+  }
+#pragma unroll
+  for (int j = 0; j < NC; j++) {
+    const int i = tid + j * THREADS, t = i / RW;
+    s_codes[i % RW][(t & 3) * GS + (t >> 2)] = t < cnt ? cd[j] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < NWT; j++) {
+    const int i = tid + j * THREADS, t = i % kWvChunk, qq = i / kWvChunk;
+    s_w[qq][(t & 3) * GS + (t >> 2)] = t < cnt && q0 + qq < nq ? wt[j] * f16_to_f32(sc[j]) : 0.f;
   }
   __syncthreads();
   // the wave's 16 elements start at bit 16 PB w of a value's words
