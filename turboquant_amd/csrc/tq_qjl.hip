@@ -240,8 +240,10 @@ __global__ __launch_bounds__(kBlock) void qjl_query_kernel(const float *__restri
 // tiles 2 (w >> 1), + 1, its keys' operands built in registers from a table
 // of code pairs and one of sign nibbles.
 // 64 queries x 8,192 keys, d = 128, 3 bits: 26.7 us with a lane per key adding
-// LDS table entries (96 a score), 10.9 us now; bound by the staging and the
-// launch, the products take under 1 us.
+// LDS table entries (96 a score), 10.9 us with the matrix products and 8.3 us
+// with the row maxima of all staged rows exchanged side by side on the lanes'
+// own paths instead of one row after the other through LDS; bound by the
+// staging and the launch, the products take under 1 us.
 template <int D, int PB>
 __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restrict__ ctx, long long nq,
                                                             const uint8_t *__restrict__ polar,
@@ -306,15 +308,27 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
       for (int i = 0; i < 4; i++) xs[it][i] = p[i];
     }
   }
+  float mx[IT];  // half-row maxima, all chains of lane exchanges side by side
+#pragma unroll
+  for (int it = 0; it < IT; it++)
+    mx[it] = fmaxf(fmaxf(fabsf(xs[it][0]), fabsf(xs[it][1])), fmaxf(fabsf(xs[it][2]), fabsf(xs[it][3])));
+  auto fold = [&](auto o) {
+    if constexpr (decltype(o)::value < LPR) {
+#pragma unroll
+      for (int it = 0; it < IT; it++) mx[it] = fmaxf(mx[it], lane_xor<decltype(o)::value>(mx[it]));
+    }
+  };
+  fold(std::integral_constant<int, 1>{});
+  fold(std::integral_constant<int, 2>{});
+  fold(std::integral_constant<int, 4>{});
+  fold(std::integral_constant<int, 8>{});
+  fold(std::integral_constant<int, 16>{});
 #pragma unroll
   for (int it = 0; it < IT; it++) {
     if (it * HPS >= 2 * rows) break;  // uniform
     const int hr = it * HPS + tid / LPR, row = hr >> 1, part = hr & 1, e0 = 4 * (tid % LPR);
     const float (&x)[4] = xs[it];
-    float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-#pragma unroll
-    for (int o = 1; o < LPR; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    const int e = row_exponent(m);
+    const int e = row_exponent(mx[it]);
     const float sc = exp2i(-e);
     uint16_t hi[4], lo[4];
 #pragma unroll
