@@ -100,3 +100,21 @@ def test_bias_of_queries_in_the_cache(tq, d, hq, t, q_len, dtype, skew):
     err = np.abs(got - ref)
     tol = mag * 2.0 ** -16 + np.abs(ref) * ULP[dtype] + (2.0 ** -25 if dtype == "f16" else 0)
     assert (err <= tol).all(), float((err / tol).max())
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_bias_of_tiny_queries(tq, d):
+    """Projections times 2^-122 and f32 queries times 2^-118 give the bias times the same: their elements are rounded
+    to 2^-149 (2^-27 of them) and each output once more (2^-24), 1e-6 of the row's root mean square.  Rows on a
+    clamped scale or cut into parts below f32's normal range are off by 1e-5 and more."""
+    hk, hq, t, q_len = 2, 4, 70, 21
+    g = torch.Generator(device="cuda").manual_seed(d)
+    k, v = (torch.randn((1, hk, t, d), generator=g, device="cuda") for _ in range(2))
+    q = torch.randn((1, hq, q_len, d), generator=g, device="cuda")
+    caches = [tq.TqCache(tq.CacheConfig(bits=3, head_dim=d, num_kv_heads=hk, num_layers=1, outlier_blocks=0)) for _ in range(2)]
+    pairs = [(caches[0].prefill(0, k, v, q).logit_bias[0], caches[1].prefill(0, k, v, q * 2.0**-118).logit_bias[0], 118)]
+    rec = (*caches[0].read_qjl(0), hk, t, t)
+    pairs.append((tq.qjl_logit_bias(q[0], *rec), tq.qjl_logit_bias(q[0] * 2.0**-122, *rec), 122))
+    for ref, got, e in pairs:
+        ref, got = ref.double(), got.double() * 2.0**e
+        assert ((got - ref).abs() <= 1e-6 * ref.square().mean(-1, keepdim=True).sqrt()).all(), e

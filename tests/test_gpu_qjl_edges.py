@@ -41,6 +41,18 @@ def test_scores_at_tile_edges(tq, dim, tb, nk, nq):
     assert (np.abs(got - ref) / natural).max() <= 1e-5
 
 
+@pytest.mark.parametrize("dim,tb", [(128, 3), (64, 4), (32, 3)])
+def test_scores_of_tiny_queries(tq, dim, tb):
+    """A context times 2^-122 gives the scores times 2^-122: its elements are rounded to 2^-149, 2^-27 of them, and
+    each score once more (2^-24): 1e-6 of the row's root mean square.  Rows on a clamped scale are off by 3e-5."""
+    recs = orc.qjl_quantize_batch(tb, dim, 42, 5, orc.lcg_normal_vecs(50, dim, 50))
+    dev = [_dev(r.view(np.int16) if r.dtype == np.uint16 else r) for r in recs]
+    ctx = tq.qjl_query_context(_dev(orc.lcg_normal_vecs(7, dim, 19)), 42, 5)
+    ref = tq.qjl_scores(ctx, *dev, tb - 1, 42).double()
+    got = tq.qjl_scores(ctx * 2.0**-122, *dev, tb - 1, 42).double() * 2.0**122
+    assert ((got - ref).abs() <= 1e-6 * ref.square().mean(1, keepdim=True).sqrt()).all()
+
+
 @pytest.mark.parametrize("dim,pb,nv,nq", [(128, 2, 1, 1), (128, 3, 255, 17), (64, 3, 257, 16), (32, 2, 770, 5),
                                           (32, 3, 4100, 3), (64, 2, 4352, 33)])
 def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):

@@ -242,17 +242,18 @@ __device__ __forceinline__ int pow2_exponent(float m) {
 }
 __device__ __forceinline__ float exp2i(int e) { return u2f((uint32_t)(127 + e) << 23); }
 
-// ---- rows of an f32 matrix as two f16 parts on a power-of-two scale per row ----
-// The scale 2^-E that brings a row's largest magnitude m into [2^13, 2^14),
-// as the exponent E (m = 0 and tiny rows: clamped; an infinite m takes 114,
-// which keeps every finite element of the row finite in f16).
+// ---- rows of an f32 matrix as f16 parts on a power-of-two scale per row ----
+// The scale 2^-E that brings a row's largest magnitude m into [2^13, 2^14)
+// (a denormal m: below it, by the bits that it lacks), as the exponent E; an
+// infinite m takes 114, which keeps every finite element of the row finite in
+// f16.  2^-E can lie outside f32's range: ldexpf, not a product.
 __device__ __forceinline__ int row_exponent(float m) {
   const int e = (int)((f2u(m) >> 23) & 0xffu) - 126;
-  return min(max(e, -100), 128) - 14;
+  return min(e, 128) - 14;
 }
-// x 2^-E as two f16 parts.  An infinity is its own upper part.
-__device__ __forceinline__ void split2(float x, float sc, uint16_t &hi, uint16_t &lo) {
-  const float v = x * sc;
+// x 2^e as two f16 parts.  An infinity is its own upper part.
+__device__ __forceinline__ void split2(float x, int e, uint16_t &hi, uint16_t &lo) {
+  const float v = __builtin_amdgcn_ldexpf(x, e);
   hi = f32_to_f16(v);
   const float h = f16_to_f32(hi);
   lo = f32_to_f16(h == v ? 0.f : v - h);

@@ -253,9 +253,9 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
                                                             float *__restrict__ scores, QjlConsts k) {
   using namespace tqm;
   constexpr int NS = D / 32, QB = 64, KB = 32, RS = D + 8;
-  constexpr float kCentScale = 256.0f;
+  constexpr int kCentExp = 8;
   __shared__ __attribute__((aligned(16))) uint16_t s_q[2][2][QB * RS];  // [qt, rq][hi, lo]
-  __shared__ __attribute__((aligned(16))) float s_e[2][QB];             // their rows' scales
+  __shared__ __attribute__((aligned(16))) int s_e[2][QB];               // their rows' exponents
   __shared__ uint2 s_pair[1 << (2 * PB)];
   __shared__ uint2 s_nib[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -285,8 +285,8 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
       c1 = (tid >> PB) == i ? k.polar.cent[i] : c1;
     }
     uint16_t h0, l0, h1, l1;
-    split2(c0, kCentScale, h0, l0);
-    split2(c1, kCentScale, h1, l1);
+    split2(c0, kCentExp, h0, l0);
+    split2(c1, kCentExp, h1, l1);
     s_pair[tid] = make_uint2(pack_pair(h0, h1), pack_pair(l0, l1));
   } else if (tid >= 64 && tid < 80) {
     auto pm1 = [&](int bit) { return (((tid - 64) >> bit) & 1) ? 0x3C00u : 0xBC00u; };
@@ -329,14 +329,13 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
     const int hr = it * HPS + tid / LPR, row = hr >> 1, part = hr & 1, e0 = 4 * (tid % LPR);
     const float (&x)[4] = xs[it];
     const int e = row_exponent(mx[it]);
-    const float sc = exp2i(-e);
     uint16_t hi[4], lo[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) split2(x[i], sc, hi[i], lo[i]);
+    for (int i = 0; i < 4; i++) split2(x[i], -e, hi[i], lo[i]);
     if (row < rows) {
       *reinterpret_cast<uint2 *>(&s_q[part][0][row * RS + e0]) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
       *reinterpret_cast<uint2 *>(&s_q[part][1][row * RS + e0]) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
-      if (tid % LPR == 0) s_e[part][row] = exp2i(e) * (part ? 1.0f : 1.0f / kCentScale);
+      if (tid % LPR == 0) s_e[part][row] = e - (part ? 0 : kCentExp);
     }
   }
   __syncthreads();
@@ -374,13 +373,13 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
       base = mfma(row(0, 0, s), ch[s], base);
       corr = mfma(row(1, 0, s), sg[s], corr);
     }
-    const float4 eb = *reinterpret_cast<const float4 *>(&s_e[0][16 * rt + 4 * lg]);
-    const float4 ec = *reinterpret_cast<const float4 *>(&s_e[1][16 * rt + 4 * lg]);
-    const float b4[4] = {eb.x, eb.y, eb.z, eb.w}, c4[4] = {ec.x, ec.y, ec.z, ec.w};
+    const int4 eb = *reinterpret_cast<const int4 *>(&s_e[0][16 * rt + 4 * lg]);
+    const int4 ec = *reinterpret_cast<const int4 *>(&s_e[1][16 * rt + 4 * lg]);
+    const int b4[4] = {eb.x, eb.y, eb.z, eb.w}, c4[4] = {ec.x, ec.y, ec.z, ec.w};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int r = 16 * rt + 4 * lg + i;
-      if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * (base[i] * b4[i]) + ck * (corr[i] * c4[i]);
+      if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * __builtin_amdgcn_ldexpf(base[i], b4[i]) + ck * __builtin_amdgcn_ldexpf(corr[i], c4[i]);
     }
   }
 }

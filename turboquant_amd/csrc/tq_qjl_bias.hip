@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
   constexpr int RS = D + 8;  // halves per staged row: 16-byte chunks of 16 rows in different banks
   __shared__ uint2 s_nib[16];
   __shared__ __attribute__((aligned(16))) uint16_t s_hi[kRows * RS], s_lo[kRows * RS];
-  __shared__ __attribute__((aligned(16))) float s_scale[kRows];
+  __shared__ __attribute__((aligned(16))) int s_exp[kRows];
   __shared__ float s_max[2][kRows];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
@@ -121,13 +121,12 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
 #pragma unroll
       for (int o = 1; o < LPR; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
       const int e = row_exponent(m);
-      const float sc = exp2i(-e);
       uint16_t hi[4], lo[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) split2(x[i], sc, hi[i], lo[i]);
+      for (int i = 0; i < 4; i++) split2(x[i], -e, hi[i], lo[i]);
       *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
       *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
-      if (lane % LPR == 0) s_scale[row] = exp2i(e);
+      if (lane % LPR == 0) s_exp[row] = e;
     }
   } else {
     // Waves w and w + 4 project rows 16 w .. + 15, each for half of R's
@@ -142,29 +141,39 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
     f32x4 rq[JH];
     uint32_t rw[JH][NS];  // R's sign words of row 16 (JH jh + jt) + l16
     u32x4 q[NS][PARTS];
+    int qexp = 0;  // an f32 row's exponent: its bf16 parts are cut from q 2^-qexp
     if (live) {
 #pragma unroll
       for (int jt = 0; jt < JH; jt++)
 #pragma unroll
         for (int s = 0; s < NS; s++) rw[jt][s] = a.rbits[(16 * (JH * jh + jt) + l16) * NS + s];
+      float v[SRC == kFromF32 ? NS : 1][8];
+      if constexpr (SRC == kFromF32) {
+        float m = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(a.src) + (row0 + row) * D + 32 * s + 8 * lg);
+          const float4 none = make_float4(0.f, 0.f, 0.f, 0.f), v0 = row < nrows ? p[0] : none, v1 = row < nrows ? p[1] : none;
+          v[s][0] = v0.x; v[s][1] = v0.y; v[s][2] = v0.z; v[s][3] = v0.w;
+          v[s][4] = v1.x; v[s][5] = v1.y; v[s][6] = v1.z; v[s][7] = v1.w;
+#pragma unroll
+          for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(v[s][j]));
+        }
+        qexp = row_exponent(max_xor32(max_xor16(m)));
+      }
 #pragma unroll
       for (int s = 0; s < NS; s++) {
         const long long xi = (row0 + row) * D + 32 * s + 8 * lg;
         if constexpr (SRC == kFromF32) {
-          float v[8] = {};
-          if (row < nrows) {
-            const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(a.src) + xi);
-            const float4 v0 = p[0], v1 = p[1];
-            v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
-            v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
-          }
+#pragma unroll
+          for (int j = 0; j < 8; j++) v[s][j] = __builtin_amdgcn_ldexpf(v[s][j], -qexp);
 #pragma unroll
           for (int p = 0; p < 3; p++) {
             uint32_t cut[8];
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-              cut[j] = f2u(v[j]) & 0xffff0000u;  // the leading 8 significand bits
-              v[j] -= u2f(cut[j]);               // exact: the rest
+              cut[j] = f2u(v[s][j]) & 0xffff0000u;  // the leading 8 significand bits
+              v[s][j] -= u2f(cut[j]);               // exact: the rest
             }
             q[s][p] = u32x4{__builtin_amdgcn_perm(cut[1], cut[0], 0x07060302u),
                             __builtin_amdgcn_perm(cut[3], cut[2], 0x07060302u),
@@ -209,17 +218,16 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
     __syncthreads();
     if (live) {
       const int e = row_exponent(fmaxf(s_max[0][row], s_max[1][row]));
-      const float sc = exp2i(-e);
 #pragma unroll
       for (int jt = 0; jt < JH; jt++) {
         uint16_t hi[4], lo[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) split2(rq[jt][i], sc, hi[i], lo[i]);
+        for (int i = 0; i < 4; i++) split2(rq[jt][i], -e, hi[i], lo[i]);
         const int at = row * RS + 16 * (JH * jh + jt) + 4 * lg;
         *reinterpret_cast<uint2 *>(s_hi + at) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
         *reinterpret_cast<uint2 *>(s_lo + at) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
       }
-      if (jh == 0 && lg == 0) s_scale[row] = exp2i(e);
+      if (jh == 0 && lg == 0) s_exp[row] = e + qexp;
     }
   }
   __syncthreads();
@@ -258,14 +266,14 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
 #pragma unroll
       for (int T = 0; T < TT; T++) acc[T] = mfma(hi, b[T][s], acc[T]);
     }
-    const float4 s4 = *reinterpret_cast<const float4 *>(s_scale + 16 * rt + 4 * lg);
-    const float sc[4] = {s4.x, s4.y, s4.z, s4.w};
+    const int4 e4 = *reinterpret_cast<const int4 *>(s_exp + 16 * rt + 4 * lg);
+    const int ex[4] = {e4.x, e4.y, e4.z, e4.w};
     const int left = nrows - 16 * rt - 4 * lg;  // rows of this tile that the lane still has
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       float v[TT];
 #pragma unroll
-      for (int T = 0; T < TT; T++) v[T] = (acc[T][i] * sc[i]) * c[T];
+      for (int T = 0; T < TT; T++) v[T] = __builtin_amdgcn_ldexpf(acc[T][i], ex[i]) * c[T];
       char *p = base + i * pitch + at;
       if (i < left) {
         if (t + 4 <= a.kv_len) {
