@@ -53,6 +53,52 @@ def test_scores_of_tiny_queries(tq, dim, tb):
     assert ((got - ref).abs() <= 1e-6 * ref.square().mean(1, keepdim=True).sqrt()).all()
 
 
+def test_scores_of_infinite_and_nan_queries(tq):
+    """Rows with an infinity or a NaN are not finite, as the oracle's; the other rows of their tile keep their values,
+    huge and tiny ones too; a key whose scale overflows f16 is not finite for any query."""
+    dim, tb, nk = 64, 4, 40
+    keys, qs = orc.lcg_normal_vecs(3, dim, nk), orc.lcg_normal_vecs(4, dim, 7)
+    keys[11] *= 1e6
+    qs[1, 5], qs[2, 9] = np.inf, np.nan
+    qs[3] *= 1e30
+    qs[4] *= 1e-30
+    recs = orc.qjl_quantize_batch(tb, dim, 42, 5, keys)
+    with np.errstate(all="ignore"):
+        ref = orc.qjl_scores(tb - 1, dim, 42, 5, qs, *recs)
+    dev = [_dev(r.view(np.int16) if r.dtype == np.uint16 else r) for r in recs]
+    got = tq.qjl_scores(tq.qjl_query_context(_dev(qs), 42, 5), *dev, tb - 1, 42).cpu().numpy()
+    assert (np.isfinite(got) == np.isfinite(ref)).all()
+    assert not np.isfinite(got[1:3]).any() and not np.isfinite(got[:, 11]).any()
+    rows, cols = [0, 3, 4, 5, 6], [j for j in range(nk) if j != 11]
+    natural = np.linalg.norm(qs[rows].astype(np.float64), axis=1)[:, None] * np.linalg.norm(keys[cols], axis=1)[None, :]
+    assert (np.abs(got[np.ix_(rows, cols)] - ref[np.ix_(rows, cols)].astype(np.float64)) / natural).max() <= 1e-5
+
+
+@pytest.mark.parametrize("dim,tb", [(32, 3), (32, 4), (64, 3), (128, 3), (128, 4)])
+def test_scores_are_as_exact_as_f32_sums(tq, dim, tb):
+    """Against f64, the 2-norm of the error is no larger than that of f32 sums of pairs of products and groups of four
+    signed projections, which the split of the operands into f16 parts stands for."""
+    nk, nq, pb = 600, 40, tb - 1
+    recs = orc.qjl_quantize_batch(tb, dim, 42, 5, orc.lcg_normal_vecs(dim, dim, nk))
+    packed, sc, sg, nm = [_dev(r.view(np.int16) if r.dtype == np.uint16 else r) for r in recs]
+    ctx = tq.qjl_query_context(_dev(orc.lcg_normal_vecs(9, dim, nq)), 42, 5)
+    got = tq.qjl_scores(ctx, packed, sc, sg, nm, pb, 42).cpu().numpy().astype(np.float64)
+    unit = torch.full((nk,), 1.0, dtype=torch.float16).cuda().view(torch.int16)
+    x = tq.dequantize_rotated_batch(packed, unit, pb, dim).cpu().numpy()  # the centroids
+    qt, rq = ctx.cpu().numpy().reshape(nq, 2, dim).transpose(1, 0, 2)
+    bits = np.unpackbits(sg.cpu().numpy(), axis=-1, bitorder="little").astype(np.float32) * 2 - 1
+    scale, norm = recs[1].view(np.float16).astype(np.float32), recs[3].view(np.float16).astype(np.float32)
+
+    def sums(dt):
+        a, b = (np.asarray(z, dt) for z in (qt[:, None, :] * x.astype(dt), rq[:, None, :] * bits.astype(dt)))
+        a = a[..., ::2] + a[..., 1::2]
+        b = ((b[..., ::4] + b[..., 1::4]) + b[..., 2::4]) + b[..., 3::4]
+        ck = norm.astype(dt) * dt(1.2533141) / np.sqrt(dt(dim))
+        return scale.astype(dt) * np.cumsum(a, -1, dtype=dt)[..., -1] + ck * np.cumsum(b, -1, dtype=dt)[..., -1]
+    ref = sums(np.float64)
+    assert np.linalg.norm(got - ref) <= np.linalg.norm(sums(np.float32) - ref)
+
+
 @pytest.mark.parametrize("dim,pb,nv,nq", [(128, 2, 1, 1), (128, 3, 255, 17), (64, 3, 257, 16), (32, 2, 770, 5),
                                           (32, 3, 4100, 3), (64, 2, 4352, 33)])
 def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):

@@ -258,6 +258,20 @@ __device__ __forceinline__ void split2(float x, int e, uint16_t &hi, uint16_t &l
   const float h = f16_to_f32(hi);
   lo = f32_to_f16(h == v ? 0.f : v - h);
 }
+// A pair (x0 2^e, x1 2^e) as three f16 pairs that hold all of their bits down
+// to 2^-24 (after scaling): cut, cut of the rest, the rest.  mone: -1 that the
+// compiler does not see as a constant, as for pack_rem.  An infinity's rests
+// are NaN.
+__device__ __forceinline__ void split3(float x0, float x1, int e, float mone, uint32_t (&w)[3]) {
+  float v0 = __builtin_amdgcn_ldexpf(x0, e), v1 = __builtin_amdgcn_ldexpf(x1, e);
+#pragma unroll
+  for (int p = 0; p < 3; p++) {
+    w[p] = pack_f16(v0, v1);
+    const auto h = __builtin_bit_cast(__fp16 __attribute__((ext_vector_type(2))), w[p]);
+    v0 = __builtin_fmaf((float)h[0], mone, v0);
+    v1 = __builtin_fmaf((float)h[1], mone, v1);
+  }
+}
 __device__ __forceinline__ uint32_t pack_pair(uint16_t a, uint16_t b) { return (uint32_t)a | ((uint32_t)b << 16); }
 
 // Code pair p (codes 2p, 2p+1) of a qblock's BITS words, LSB-first: the

@@ -229,158 +229,152 @@ __global__ __launch_bounds__(kBlock) void qjl_query_kernel(const float *__restri
   }
 }
 
-// Scores of 64 queries x 32 keys per workgroup:
+// Scores, 16 queries x 16 keys per wave:
 //   est = scale_k * sum_i qt_i c[idx_i] + c_k * sum_j rq_j (2 b_j - 1),
 //   c_k = |r_k| * sqrt(pi/2) / sqrt(d)   (qjl.rs:263-265, 512-519, 585-606).
-// Both sums run on v_mfma_f32_16x16x32_f16 with every f32 operand as two f16
-// parts of 22 to 23 significant bits together (the queries' on a power-of-two
-// scale per row, the centroids' times 2^8; the signs are exact): four part
-// products for the first sum, two for the second.  The queries are staged in
-// LDS once per workgroup; wave w takes keys 16 (w & 1) .. + 15 and the query
-// tiles 2 (w >> 1), + 1, its keys' operands built in registers from a table
-// of code pairs and one of sign nibbles.
-// 64 queries x 8,192 keys, d = 128, 3 bits: 26.7 us with a lane per key adding
-// LDS table entries (96 a score), 10.9 us with the matrix products and 8.3 us
-// with the row maxima of all staged rows exchanged side by side on the lanes'
-// own paths instead of one row after the other through LDS; bound by the
-// staging and the launch, the products take under 1 us.
+// Both sums run on v_mfma_f32_16x16x32_f16 with every f32 operand as three f16
+// parts that hold all of its 24 significant bits (a query's on its row's
+// power-of-two scale, the centroids' times 2^8; the signs are exact).  Six part
+// products for the first sum (the parts below 2^-33 of it dropped), three for
+// the second.  With two parts (22 bits) scores of 32 elements were further from
+// the f64 result than f32 sums are: 1.16e-7 against 9.0e-8 (2-norm, 2-bit
+// codes); with three 6.3e-8.
+//
+// Lane (l16, lg) holds elements lg D / 4 .. + D / 4 - 1 of query l16 and of key
+// l16, 8 for each of the D / 32 slices, so a row is read in whole runs, its
+// largest magnitude needs two lane exchanges and the queries' operands stay in
+// registers.  A slice's centroids are byte permutes: 4 codes as the selector
+// bytes, tables of the parts' low and high bytes in registers.
+// 64 queries x 8,192 keys, d = 128, 3 bits: 18 us with a lane per key adding LDS
+// table entries (96 a score), 7.4 us now (7.5 with two parts and the queries
+// staged in LDS for four waves).
+constexpr int kCentExp = 8;
+struct CentroidParts {
+  uint32_t tab[3][2][2];  // [part][low, high byte][entries 0..3, 4..7]
+};
+template <int PB>
+__device__ __forceinline__ uint32_t spread_codes(uint32_t x) {  // 4 codes -> 4 bytes
+  constexpr uint32_t M = (1u << PB) - 1u;
+  x &= (1u << (4 * PB)) - 1u;
+  x = (x | x << (16 - 2 * PB)) & ((M | M << PB) * 0x00010001u);
+  return (x | x << (8 - PB)) & (M * 0x01010101u);
+}
+
 template <int D, int PB>
 __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restrict__ ctx, long long nq,
                                                             const uint8_t *__restrict__ polar,
                                                             const uint16_t *__restrict__ polar_scales,
                                                             const uint8_t *__restrict__ signs,
                                                             const uint16_t *__restrict__ residual_norms, long long nk,
-                                                            float *__restrict__ scores, QjlConsts k) {
+                                                            float *__restrict__ scores, QjlConsts k, CentroidParts cent) {
   using namespace tqm;
-  constexpr int NS = D / 32, QB = 64, KB = 32, RS = D + 8;
-  constexpr int kCentExp = 8;
-  __shared__ __attribute__((aligned(16))) uint16_t s_q[2][2][QB * RS];  // [qt, rq][hi, lo]
-  __shared__ __attribute__((aligned(16))) int s_e[2][QB];               // their rows' exponents
-  __shared__ uint2 s_pair[1 << (2 * PB)];
-  __shared__ uint2 s_nib[16];
+  constexpr int NS = D / 32, E = D / 4, CBITS = E * PB;  // slices; elements and code bits of a lane
+  constexpr int RW = D * PB / 32, NCW = D == 128 ? PB : PB - 1;  // words of a record; that hold a lane's codes
+  __shared__ __attribute__((aligned(16))) u32x4 s_sign[256];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
-  const long long q0 = (long long)blockIdx.y * QB;
-  const int nql = (int)min<long long>(QB, nq - q0);
-  // the wave's keys: 8 codes and 8 signs of every 32-element slice per lane
-  const long long key = (long long)blockIdx.x * KB + 16 * (wave & 1) + l16;
+  const long long q0 = (long long)blockIdx.y * 16;
+  const int nql = (int)min<long long>(16, nq - q0);
+  // the wave's keys: the lane's quarter of a record's codes and signs
+  const long long key = ((long long)blockIdx.x * (kBlock / 64) + wave) * 16 + l16;
   const long long kc = min(key, nk - 1);
-  uint32_t code[NS], sgn[NS];
+  uint32_t code[NCW], sgn;
+  {
+    const uint32_t *rec = reinterpret_cast<const uint32_t *>(polar + kc * (D * PB / 8));
+    const int bit = CBITS * lg, wi = bit >> 5, sh = bit & 31;
+    uint32_t raw[NCW];
 #pragma unroll
-  for (int s = 0; s < NS; s++) {
-    const uint32_t *rec = reinterpret_cast<const uint32_t *>(polar + kc * (D * PB / 8)) + PB * s;
-    const int bit = 8 * PB * lg, wi = bit >> 5, sh = bit & 31;
-    if constexpr (PB == 2) code[s] = rec[wi] >> sh;
-    else code[s] = __builtin_amdgcn_alignbit(rec[min(wi + 1, PB - 1)], rec[wi], sh);
-    sgn[s] = signs[kc * (D / 8) + 4 * s + lg];
+    for (int i = 0; i < NCW; i++) raw[i] = rec[min(wi + i, RW - 1)];
+#pragma unroll
+    for (int i = 0; i < NCW; i++) code[i] = i + 1 < NCW ? __builtin_amdgcn_alignbit(raw[i + 1], raw[i], sh) : raw[i] >> sh;
+    const uint8_t *sg = signs + kc * (D / 8) + lg * (E / 8);
+    if constexpr (E == 32) sgn = *reinterpret_cast<const uint32_t *>(sg);
+    else if constexpr (E == 16) sgn = *reinterpret_cast<const uint16_t *>(sg);
+    else sgn = *sg;
   }
   const float scale = f16_to_f32(polar_scales[kc]);
   const float ck = (f16_to_f32(residual_norms[kc]) * 1.2533141f) / k.sqrt_d;
-  // pair (c0 low, c1 high) -> (hi, hi), (lo, lo); nibble -> f16 +-1, LSB first (bit set: +1)
-  if (tid < (1 << (2 * PB))) {
-    float c0 = 0.f, c1 = 0.f;
+  // the queries' rows qt and rq
+  float x[2][E];
+  {
+    const float *row = ctx + (q0 + min(l16, nql - 1)) * 2 * D + lg * E;
 #pragma unroll
-    for (int i = 0; i < (1 << PB); i++) {
-      c0 = (tid & ((1 << PB) - 1)) == i ? k.polar.cent[i] : c0;
-      c1 = (tid >> PB) == i ? k.polar.cent[i] : c1;
-    }
-    uint16_t h0, l0, h1, l1;
-    split2(c0, kCentExp, h0, l0);
-    split2(c1, kCentExp, h1, l1);
-    s_pair[tid] = make_uint2(pack_pair(h0, h1), pack_pair(l0, l1));
-  } else if (tid >= 64 && tid < 80) {
-    auto pm1 = [&](int bit) { return (((tid - 64) >> bit) & 1) ? 0x3C00u : 0xBC00u; };
-    s_nib[tid - 64] = make_uint2(pm1(0) | (pm1(1) << 16), pm1(2) | (pm1(3) << 16));
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int e = 0; e < E; e++) x[p][e] = row[p * D + e];
   }
-  // the queries: row r's qt and rq are half-rows 2 r, 2 r + 1 of D elements, D / 4 lanes each
-  constexpr int LPR = D / 4, HPS = kBlock / LPR;
-  const int rows = min(QB, (nql + 15) & ~15);
-  constexpr int IT = 2 * QB / HPS;
-  float xs[IT][4];  // every load goes out before the first is used
-#pragma unroll
-  for (int it = 0; it < IT; it++) {
-    const int hr = it * HPS + tid / LPR, e0 = 4 * (tid % LPR);
-#pragma unroll
-    for (int i = 0; i < 4; i++) xs[it][i] = 0.f;
-    if ((hr >> 1) < nql) {
-      const float *p = ctx + (q0 * 2 + hr) * D + e0;
-#pragma unroll
-      for (int i = 0; i < 4; i++) xs[it][i] = p[i];
-    }
+  // +-1 in f16 for the eight sign bits of a byte, LSB first (bit set: +1)
+  {
+    auto pm1 = [&](int bit) { return ((tid >> bit) & 1) ? 0x3C00u : 0xBC00u; };
+    s_sign[tid] = u32x4{pm1(0) | (pm1(1) << 16), pm1(2) | (pm1(3) << 16), pm1(4) | (pm1(5) << 16), pm1(6) | (pm1(7) << 16)};
   }
-  float mx[IT];  // half-row maxima, all chains of lane exchanges side by side
+  uint32_t tab[3][2][PB - 1];
 #pragma unroll
-  for (int it = 0; it < IT; it++)
-    mx[it] = fmaxf(fmaxf(fabsf(xs[it][0]), fabsf(xs[it][1])), fmaxf(fabsf(xs[it][2]), fabsf(xs[it][3])));
-  auto fold = [&](auto o) {
-    if constexpr (decltype(o)::value < LPR) {
+  for (int p = 0; p < 3; p++)
 #pragma unroll
-      for (int it = 0; it < IT; it++) mx[it] = fmaxf(mx[it], lane_xor<decltype(o)::value>(mx[it]));
-    }
-  };
-  fold(std::integral_constant<int, 1>{});
-  fold(std::integral_constant<int, 2>{});
-  fold(std::integral_constant<int, 4>{});
-  fold(std::integral_constant<int, 8>{});
-  fold(std::integral_constant<int, 16>{});
+    for (int h = 0; h < 2; h++)
 #pragma unroll
-  for (int it = 0; it < IT; it++) {
-    if (it * HPS >= 2 * rows) break;  // uniform
-    const int hr = it * HPS + tid / LPR, row = hr >> 1, part = hr & 1, e0 = 4 * (tid % LPR);
-    const float (&x)[4] = xs[it];
-    const int e = row_exponent(mx[it]);
-    uint16_t hi[4], lo[4];
+      for (int i = 0; i < PB - 1; i++) tab[p][h][i] = cent.tab[p][h][i];
+  float mone = -1.f;
+  asm("" : "+v"(mone));
+  u32x4 q[2][NS][3];
+  int ex[2];  // row l16's exponents
 #pragma unroll
-    for (int i = 0; i < 4; i++) split2(x[i], -e, hi[i], lo[i]);
-    if (row < rows) {
-      *reinterpret_cast<uint2 *>(&s_q[part][0][row * RS + e0]) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
-      *reinterpret_cast<uint2 *>(&s_q[part][1][row * RS + e0]) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
-      if (tid % LPR == 0) s_e[part][row] = e - (part ? 0 : kCentExp);
-    }
+  for (int p = 0; p < 2; p++) {
+    float m = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; e++) m = fmaxf(m, fabsf(x[p][e]));
+    ex[p] = row_exponent(max_xor32(max_xor16(m)));
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+      for (int w = 0; w < 4; w++) {
+        uint32_t part[3];
+        split3(x[p][8 * s + 2 * w], x[p][8 * s + 2 * w + 1], -ex[p], mone, part);
+#pragma unroll
+        for (int i = 0; i < 3; i++) q[p][s][i][w] = part[i];
+      }
   }
   __syncthreads();
-  u32x4 ch[NS], cl[NS], sg[NS];
+  f32x4 base[3], corr[2];  // products of about the same size together
+#pragma unroll
+  for (int i = 0; i < 3; i++) base[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; i++) corr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < NS; s++) {
-    uint32_t h[4], l[4];
+    u32x4 c[3];
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-      const uint2 e = s_pair[(code[s] >> (2 * PB * p)) & ((1u << (2 * PB)) - 1u)];
-      h[p] = e.x;
-      l[p] = e.y;
+    for (int h = 0; h < 2; h++) {  // 4 codes each
+      const int bit = (8 * s + 4 * h) * PB, wi = bit >> 5, sh = bit & 31;
+      const uint32_t sel = spread_codes<PB>(sh + 4 * PB > 32 ? __builtin_amdgcn_alignbit(code[wi + 1], code[wi], sh) : code[wi] >> sh);
+#pragma unroll
+      for (int p = 0; p < 3; p++) {
+        const uint32_t lo = __builtin_amdgcn_perm(tab[p][0][PB - 2], tab[p][0][0], sel);
+        const uint32_t hi = __builtin_amdgcn_perm(tab[p][1][PB - 2], tab[p][1][0], sel);
+        c[p][2 * h] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+        c[p][2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+      }
     }
-    ch[s] = u32x4{h[0], h[1], h[2], h[3]};
-    cl[s] = u32x4{l[0], l[1], l[2], l[3]};
-    const uint2 n0 = s_nib[sgn[s] & 15u], n1 = s_nib[(sgn[s] >> 4) & 15u];
-    sg[s] = u32x4{n0.x, n0.y, n1.x, n1.y};
+    const u32x4 sg = s_sign[(sgn >> (8 * s)) & 0xffu];
+    const u32x4(&qt)[3] = q[0][s], (&rq)[3] = q[1][s];
+    base[2] = mfma(qt[2], c[0], base[2]);
+    corr[1] = mfma(rq[2], sg, corr[1]);
+    base[1] = mfma(qt[1], c[0], base[1]);
+    base[0] = mfma(qt[0], c[0], base[0]);
+    base[2] = mfma(qt[0], c[2], base[2]);
+    corr[1] = mfma(rq[1], sg, corr[1]);
+    base[1] = mfma(qt[0], c[1], base[1]);
+    corr[0] = mfma(rq[0], sg, corr[0]);
+    base[2] = mfma(qt[1], c[1], base[2]);
   }
-  for (int t = 0; t < 2; t++) {
-    const int rt = 2 * (wave >> 1) + t;
-    if (16 * rt >= nql) break;
-    f32x4 base = {0.f, 0.f, 0.f, 0.f}, corr = {0.f, 0.f, 0.f, 0.f};
-    const int at = (16 * rt + l16) * RS + 8 * lg;
-    auto row = [&](int part, int half, int s) { return *reinterpret_cast<const u32x4 *>(&s_q[part][half][at + 32 * s]); };
 #pragma unroll
-    for (int s = 0; s < NS; s++) {  // the small products first
-      const u32x4 qh = row(0, 0, s), ql = row(0, 1, s);
-      base = mfma(ql, cl[s], base);
-      corr = mfma(row(1, 1, s), sg[s], corr);
-      base = mfma(qh, cl[s], base);
-      base = mfma(ql, ch[s], base);
-    }
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-      base = mfma(row(0, 0, s), ch[s], base);
-      corr = mfma(row(1, 0, s), sg[s], corr);
-    }
-    const int4 eb = *reinterpret_cast<const int4 *>(&s_e[0][16 * rt + 4 * lg]);
-    const int4 ec = *reinterpret_cast<const int4 *>(&s_e[1][16 * rt + 4 * lg]);
-    const int b4[4] = {eb.x, eb.y, eb.z, eb.w}, c4[4] = {ec.x, ec.y, ec.z, ec.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int r = 16 * rt + 4 * lg + i;
-      if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * __builtin_amdgcn_ldexpf(base[i], b4[i]) + ck * __builtin_amdgcn_ldexpf(corr[i], c4[i]);
-    }
+  for (int i = 0; i < 4; i++) {
+    const int r = 4 * lg + i;
+    const int e0 = __shfl(ex[0], r, 64) - kCentExp, e1 = __shfl(ex[1], r, 64);
+    const float b = __builtin_amdgcn_ldexpf(base[0][i] + (base[1][i] + base[2][i]), e0);
+    const float c = __builtin_amdgcn_ldexpf(corr[0][i] + corr[1][i], e1);
+    if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * b + ck * c;
   }
 }
 
@@ -627,6 +621,29 @@ int qjl_consts(int polar_bits, int dim, uint64_t rot_seed, uint64_t qjl_seed, Qj
   return TQ_OK;
 }
 
+// |v| < 2^15 cut to an f16's 11 significant bits (2^-24 for values below 2^-14).
+double f16_cut(double v, uint16_t &bits) {
+  const double a = std::fabs(v);
+  const int e = a < 0x1p-14 ? -14 : std::ilogb(a);
+  const double m = std::trunc(std::ldexp(a, 10 - e));  // [0, 2^11)
+  const int field = m < 1024.0 ? 0 : e + 15;
+  bits = (uint16_t)((v < 0 ? 0x8000 : 0) | (field << 10) | ((int)m & 0x3ff));
+  return std::copysign(std::ldexp(m, e - 10), v);
+}
+CentroidParts centroid_parts(const CodecConsts &polar, int polar_bits) {
+  CentroidParts c{};
+  for (int i = 0; i < (1 << polar_bits); i++) {
+    double v = std::ldexp((double)polar.cent[i], kCentExp);
+    for (int p = 0; p < 3; p++) {
+      uint16_t h;
+      v -= f16_cut(v, h);
+      c.tab[p][0][i >> 2] |= (uint32_t)(h & 0xff) << (8 * (i & 3));
+      c.tab[p][1][i >> 2] |= (uint32_t)(h >> 8) << (8 * (i & 3));
+    }
+  }
+  return c;
+}
+
 template <typename F>
 int by_dim(int dim, F &&f) {
   switch (dim) {
@@ -698,9 +715,9 @@ extern "C" int tq_qjl_scores(const float *ctx, size_t num_queries, const uint8_t
   const long long nq = (long long)num_queries, nk = (long long)num_keys;
   return by_dim_bits(dim, polar_bits, [&](auto d, auto pb) {
     constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
-    hipLaunchKernelGGL((qjl_scores_kernel<D, PB>), dim3((unsigned)((nk + 31) / 32), (unsigned)((nq + 63) / 64)),
+    hipLaunchKernelGGL((qjl_scores_kernel<D, PB>), dim3((unsigned)((nk + 63) / 64), (unsigned)((nq + 15) / 16)),
                        dim3(kBlock), 0, stream, ctx, nq, polar_packed, polar_scales, signs, residual_norms, nk, scores,
-                       k);
+                       k, centroid_parts(k.polar, polar_bits));
     return tqh::check_launch("qjl_scores_kernel");
   });
 }
