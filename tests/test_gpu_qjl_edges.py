@@ -53,6 +53,38 @@ def test_scores_of_tiny_queries(tq, dim, tb):
     assert ((got - ref).abs() <= 1e-6 * ref.square().mean(1, keepdim=True).sqrt()).all()
 
 
+@pytest.mark.parametrize("dim,tb,nk,nq", [(32, 3, 5, 1), (32, 3, 32769, 2), (32, 3, 33000, 17), (64, 4, 49153, 1),
+                                          (128, 3, 24577, 1), (128, 4, 33007, 3)])
+def test_scores_of_many_keys(tq, dim, tb, nk, nq):
+    """Lists at which a wave walks several tiles of 16 keys, and few queries by tables: against the oracle on some
+    hundred of the keys, which are all that the list repeats."""
+    part = orc.lcg_normal_vecs(dim + nk, dim, 211)
+    recs = orc.qjl_quantize_batch(tb, dim, 42, 5, part)
+    qs = orc.lcg_normal_vecs(nq, dim, nq)
+    ref = orc.qjl_scores(tb - 1, dim, 42, 5, qs, *recs)
+    at = np.arange(nk) % len(part)
+    dev = [_dev((r.view(np.int16) if r.dtype == np.uint16 else r)[at]) for r in recs]
+    got = tq.qjl_scores(tq.qjl_query_context(_dev(qs), 42, 5), *dev, tb - 1, 42).cpu().numpy()
+    natural = np.linalg.norm(qs, axis=1)[:, None] * np.linalg.norm(part, axis=1)[None, :]
+    assert (np.abs(got - ref[:, at]) / natural[:, at]).max() <= 1e-5
+
+
+def test_scores_of_more_keys_than_a_grid_of_eight_lanes_a_key(tq):
+    """2^29 + 1 keys: a launch holds fewer than 2^32 lanes.  The last key's score is that of the key alone."""
+    nk, dim = 2**29 + 1, 32
+    if torch.cuda.mem_get_info()[0] < 16 * 2**30:
+        pytest.skip("needs 16 GiB")
+    recs = [torch.zeros((nk, 8), dtype=torch.uint8, device="cuda"), torch.zeros((nk,), dtype=torch.int16, device="cuda"),
+            torch.zeros((nk, 4), dtype=torch.uint8, device="cuda"), torch.zeros((nk,), dtype=torch.int16, device="cuda")]
+    last = [_dev(r.view(np.int16) if r.dtype == np.uint16 else r)
+            for r in orc.qjl_quantize_batch(3, dim, 42, 5, orc.lcg_normal_vecs(1, dim, 1))]
+    for r, x in zip(recs, last):
+        r[-1:] = x
+    ctx = tq.qjl_query_context(_dev(orc.lcg_normal_vecs(2, dim, 1)), 42, 5)
+    got = tq.qjl_scores(ctx, *recs, 2, 42)
+    assert torch.equal(got[0, -1:], tq.qjl_scores(ctx, *last, 2, 42)[0]) and float(got[0, 5]) == 0.0
+
+
 def test_scores_of_infinite_and_nan_queries(tq):
     """Rows with an infinity or a NaN are not finite, as the oracle's; the other rows of their tile keep their values,
     huge and tiny ones too; a key whose scale overflows f16 is not finite for any query."""

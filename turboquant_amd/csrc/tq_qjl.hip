@@ -14,6 +14,7 @@
 #include "tq_codec_dev.h"
 #include "tq_mfma.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -249,6 +250,13 @@ __global__ __launch_bounds__(kBlock) void qjl_query_kernel(const float *__restri
 // table entries (96 a score), 7.4 us now (7.5 with two parts and the queries
 // staged in LDS for four waves).
 constexpr int kCentExp = 8;
+// The workgroups of a launch: one per compute unit, whose waves then walk
+// several key tiles for one split of their queries, and two, as many as the
+// registers hold at d = 128, above 6 tiles a wave (us, one / two: 64 queries x
+// 8,192 keys 6.4 / 7.9, x 24,576 10.5 / 11.0, x 49,152 16.2 / 15.7, x 262,144
+// 57.8 / 52.7; with a tile per wave 123).
+constexpr int kScoreBlocks = 256;
+constexpr int kScoreTiles = 6;
 struct CentroidParts {
   uint32_t tab[3][2][2];  // [part][low, high byte][entries 0..3, 4..7]
 };
@@ -275,25 +283,29 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
   const int l16 = lane & 15, lg = lane >> 4;
   const long long q0 = (long long)blockIdx.y * 16;
   const int nql = (int)min<long long>(16, nq - q0);
-  // the wave's keys: the lane's quarter of a record's codes and signs
-  const long long key = ((long long)blockIdx.x * (kBlock / 64) + wave) * 16 + l16;
-  const long long kc = min(key, nk - 1);
-  uint32_t code[NCW], sgn;
-  {
+  // the wave's key tiles: the lane's quarter of a record's codes and signs
+  struct Keys {
+    uint32_t raw[NCW], sgn;
+    uint16_t scale, norm;
+  };
+  const int bit0 = CBITS * lg, wi0 = bit0 >> 5, sh0 = bit0 & 31;
+  auto load_keys = [&](long long tile) {
+    Keys r;
+    const long long kc = min(tile * 16 + l16, nk - 1);
     const uint32_t *rec = reinterpret_cast<const uint32_t *>(polar + kc * (D * PB / 8));
-    const int bit = CBITS * lg, wi = bit >> 5, sh = bit & 31;
-    uint32_t raw[NCW];
 #pragma unroll
-    for (int i = 0; i < NCW; i++) raw[i] = rec[min(wi + i, RW - 1)];
-#pragma unroll
-    for (int i = 0; i < NCW; i++) code[i] = i + 1 < NCW ? __builtin_amdgcn_alignbit(raw[i + 1], raw[i], sh) : raw[i] >> sh;
+    for (int i = 0; i < NCW; i++) r.raw[i] = rec[min(wi0 + i, RW - 1)];
     const uint8_t *sg = signs + kc * (D / 8) + lg * (E / 8);
-    if constexpr (E == 32) sgn = *reinterpret_cast<const uint32_t *>(sg);
-    else if constexpr (E == 16) sgn = *reinterpret_cast<const uint16_t *>(sg);
-    else sgn = *sg;
-  }
-  const float scale = f16_to_f32(polar_scales[kc]);
-  const float ck = (f16_to_f32(residual_norms[kc]) * 1.2533141f) / k.sqrt_d;
+    if constexpr (E == 32) r.sgn = *reinterpret_cast<const uint32_t *>(sg);
+    else if constexpr (E == 16) r.sgn = *reinterpret_cast<const uint16_t *>(sg);
+    else r.sgn = *sg;
+    r.scale = polar_scales[kc];
+    r.norm = residual_norms[kc];
+    return r;
+  };
+  const long long tiles = (nk + 15) / 16, step = (long long)gridDim.x * (kBlock / 64);
+  long long tile = (long long)blockIdx.x * (kBlock / 64) + wave;
+  Keys next = load_keys(min(tile, tiles - 1));
   // the queries' rows qt and rq
   float x[2][E];
   {
@@ -335,46 +347,145 @@ __global__ __launch_bounds__(kBlock) void qjl_scores_kernel(const float *__restr
         for (int i = 0; i < 3; i++) q[p][s][i][w] = part[i];
       }
   }
-  __syncthreads();
-  f32x4 base[3], corr[2];  // products of about the same size together
-#pragma unroll
-  for (int i = 0; i < 3; i++) base[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 2; i++) corr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < NS; s++) {
-    u32x4 c[3];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {  // 4 codes each
-      const int bit = (8 * s + 4 * h) * PB, wi = bit >> 5, sh = bit & 31;
-      const uint32_t sel = spread_codes<PB>(sh + 4 * PB > 32 ? __builtin_amdgcn_alignbit(code[wi + 1], code[wi], sh) : code[wi] >> sh);
-#pragma unroll
-      for (int p = 0; p < 3; p++) {
-        const uint32_t lo = __builtin_amdgcn_perm(tab[p][0][PB - 2], tab[p][0][0], sel);
-        const uint32_t hi = __builtin_amdgcn_perm(tab[p][1][PB - 2], tab[p][1][0], sel);
-        c[p][2 * h] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-        c[p][2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-      }
-    }
-    const u32x4 sg = s_sign[(sgn >> (8 * s)) & 0xffu];
-    const u32x4(&qt)[3] = q[0][s], (&rq)[3] = q[1][s];
-    base[2] = mfma(qt[2], c[0], base[2]);
-    corr[1] = mfma(rq[2], sg, corr[1]);
-    base[1] = mfma(qt[1], c[0], base[1]);
-    base[0] = mfma(qt[0], c[0], base[0]);
-    base[2] = mfma(qt[0], c[2], base[2]);
-    corr[1] = mfma(rq[1], sg, corr[1]);
-    base[1] = mfma(qt[0], c[1], base[1]);
-    corr[0] = mfma(rq[0], sg, corr[0]);
-    base[2] = mfma(qt[1], c[1], base[2]);
-  }
+  int e0[4], e1[4];  // the exponents of the rows 4 lg .. + 3 that the lane's sums belong to
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int r = 4 * lg + i;
-    const int e0 = __shfl(ex[0], r, 64) - kCentExp, e1 = __shfl(ex[1], r, 64);
-    const float b = __builtin_amdgcn_ldexpf(base[0][i] + (base[1][i] + base[2][i]), e0);
-    const float c = __builtin_amdgcn_ldexpf(corr[0][i] + corr[1][i], e1);
-    if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * b + ck * c;
+    e0[i] = __shfl(ex[0], 4 * lg + i, 64) - kCentExp;
+    e1[i] = __shfl(ex[1], 4 * lg + i, 64);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (; tile < tiles; tile += step) {
+    const Keys cur = next;
+    if (tile + step < tiles) next = load_keys(tile + step);  // in flight during this tile's products
+    uint32_t code[NCW];
+#pragma unroll
+    for (int i = 0; i < NCW; i++)
+      code[i] = i + 1 < NCW ? __builtin_amdgcn_alignbit(cur.raw[i + 1], cur.raw[i], sh0) : cur.raw[i] >> sh0;
+    const float scale = f16_to_f32(cur.scale);
+    const float ck = (f16_to_f32(cur.norm) * 1.2533141f) / k.sqrt_d;
+    f32x4 base[3], corr[2];  // products of about the same size together
+#pragma unroll
+    for (int i = 0; i < 3; i++) base[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 2; i++) corr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      u32x4 c[3];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {  // 4 codes each
+        const int bit = (8 * s + 4 * h) * PB, wi = bit >> 5, sh = bit & 31;
+        const uint32_t sel = spread_codes<PB>(sh + 4 * PB > 32 ? __builtin_amdgcn_alignbit(code[wi + 1], code[wi], sh) : code[wi] >> sh);
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+          const uint32_t lo = __builtin_amdgcn_perm(tab[p][0][PB - 2], tab[p][0][0], sel);
+          const uint32_t hi = __builtin_amdgcn_perm(tab[p][1][PB - 2], tab[p][1][0], sel);
+          c[p][2 * h] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+          c[p][2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+        }
+      }
+      const u32x4 sg = s_sign[(cur.sgn >> (8 * s)) & 0xffu];
+      const u32x4(&qt)[3] = q[0][s], (&rq)[3] = q[1][s];
+      base[2] = mfma(qt[2], c[0], base[2]);
+      corr[1] = mfma(rq[2], sg, corr[1]);
+      base[1] = mfma(qt[1], c[0], base[1]);
+      base[0] = mfma(qt[0], c[0], base[0]);
+      base[2] = mfma(qt[0], c[2], base[2]);
+      corr[1] = mfma(rq[1], sg, corr[1]);
+      base[1] = mfma(qt[0], c[1], base[1]);
+      corr[0] = mfma(rq[0], sg, corr[0]);
+      base[2] = mfma(qt[1], c[1], base[2]);
+    }
+    const long long key = tile * 16 + l16;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = 4 * lg + i;
+      const float b = __builtin_amdgcn_ldexpf(base[0][i] + (base[1][i] + base[2][i]), e0[i]);
+      const float c = __builtin_amdgcn_ldexpf(corr[0][i] + corr[1][i], e1[i]);
+      if (r < nql && key < nk) scores[(q0 + r) * nk + key] = scale * b + ck * c;
+    }
+  }
+}
+
+// The same scores for a few queries over many keys: lane = key, the sums of a
+// query over code pairs and sign nibbles in LDS tables, D / 2 + D / 4 entries a
+// score added in f32.  A 16-query tile's cost does not fall with its rows, a
+// table's does.  By tables / by tiles, us, 262,144 keys at 3 bits: d = 128 one
+// query 7.4 / 12.3, two 11.3 / 12.9, three 15.4 / 13.5; d = 64 one 4.2 / 8.7,
+// four 8.4 / 10.2, six 11.2 / 10.5; d = 32 one 3.4 / 6.9, six 7.3 / 8.5, eight
+// 8.8 / 8.9.  Few keys are latency, which tiles have less of: 8,192 keys, d =
+// 128, one query 4.1 / 3.9, two 6.0 / 4.0.  A 3-bit code's pair tables are four
+// times as large (4 bits in all, d = 128, one query x 49,152 keys 6.1 / 5.7,
+// 262,144 keys 8.5 / 13.1, two queries 13.5 / 13.6).
+template <int D, int PB>
+constexpr int kTableQueries = (PB == 2 ? 256 : 128) / D;
+// ... and the queries of a workgroup (their tables' LDS)
+template <int PB>
+constexpr int kTableBlockQueries = PB == 2 ? 8 : 2;
+// the keys from which one query's table is no slower, and more for each other query
+template <int D, int PB>
+constexpr int kTableKeys = PB == 2 ? (D == 32 ? 1 : D == 64 ? 8192 : 24576) : (D == 32 ? 24576 : D == 64 ? 49152 : 57344);
+template <int D>
+constexpr int kTableKeysPerQuery = D == 32 ? 24576 : 32768;
+
+template <int D, int PB>
+__global__ __launch_bounds__(kBlock) void qjl_scores_table_kernel(const float *__restrict__ ctx, long long nq,
+                                                                  const uint8_t *__restrict__ polar,
+                                                                  const uint16_t *__restrict__ polar_scales,
+                                                                  const uint32_t *__restrict__ signs,
+                                                                  const uint16_t *__restrict__ residual_norms,
+                                                                  long long nk, float *__restrict__ scores, QjlConsts k) {
+  constexpr int QB = kTableBlockQueries<PB>;
+  constexpr int PE = 1 << (2 * PB);         // entries per pair table
+  constexpr int BT = (D / 2) * PE;          // pair tables per query
+  constexpr int CT = (D / 4) * 16;          // sign-nibble tables per query
+  constexpr int SW = D / 32, NW = SW * PB;  // sign and code words of a key
+  __shared__ float s_tab[QB * (BT + CT)];
+  __shared__ float s_cent[16];
+  if (threadIdx.x < 16) s_cent[threadIdx.x] = k.polar.cent[threadIdx.x & ((1 << PB) - 1)];
+  __syncthreads();
+  const long long q0 = (long long)blockIdx.y * QB;
+  const int nql = (int)min<long long>(QB, nq - q0);
+  // pair (g, code) -> qt[2g] c[lo] + qt[2g+1] c[hi]; nibble (c, m) -> sum_b rq[4c+b] (m_b ? 1 : -1)
+  for (int e = threadIdx.x; e < nql * (BT + CT); e += kBlock) {
+    const int ql = e / (BT + CT), r = e % (BT + CT);
+    const float *cq = ctx + (q0 + ql) * 2 * D;
+    float val;
+    if (r < BT) {
+      const int g = r / PE, code = r % PE;
+      val = cq[2 * g] * s_cent[code & ((1 << PB) - 1)] + cq[2 * g + 1] * s_cent[code >> PB];
+    } else {
+      const int c = (r - BT) / 16, m = (r - BT) % 16;
+      const float *rq = cq + D + 4 * c;
+      val = -0.0f;
+#pragma unroll
+      for (int b = 0; b < 4; b++) val = val + ((m >> b) & 1 ? rq[b] : -rq[b]);
+    }
+    s_tab[e] = val;
+  }
+  __syncthreads();
+  const long long key = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (key >= nk) return;
+  uint32_t pk[NW], sg[SW];
+#pragma unroll
+  for (int i = 0; i < NW; i++) pk[i] = reinterpret_cast<const uint32_t *>(polar + key * (4 * NW))[i];
+#pragma unroll
+  for (int i = 0; i < SW; i++) sg[i] = signs[key * SW + i];
+  const float scale = f16_to_f32(polar_scales[key]);
+  const float ck = (f16_to_f32(residual_norms[key]) * 1.2533141f) / k.sqrt_d;
+  for (int ql = 0; ql < nql; ql++) {
+    const float *tb = s_tab + ql * (BT + CT);
+    float base = 0.0f, corr = 0.0f;
+#pragma unroll
+    for (int g = 0; g < D / 2; g++) {
+      const int bit = 2 * g * PB, wi = bit >> 5, sh = bit & 31;
+      uint32_t code = pk[wi] >> sh;
+      if (sh + 2 * PB > 32) code |= pk[wi + 1] << (32 - sh);
+      base += tb[g * PE + (code & (PE - 1))];
+    }
+#pragma unroll
+    for (int c = 0; c < D / 4; c++) corr += tb[BT + c * 16 + ((sg[c >> 3] >> ((c & 7) * 4)) & 15u)];
+    scores[(q0 + ql) * nk + key] = scale * base + ck * corr;
   }
 }
 
@@ -715,7 +826,17 @@ extern "C" int tq_qjl_scores(const float *ctx, size_t num_queries, const uint8_t
   const long long nq = (long long)num_queries, nk = (long long)num_keys;
   return by_dim_bits(dim, polar_bits, [&](auto d, auto pb) {
     constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
-    hipLaunchKernelGGL((qjl_scores_kernel<D, PB>), dim3((unsigned)((nk + 63) / 64), (unsigned)((nq + 15) / 16)),
+    if (nq <= kTableQueries<D, PB> && nk >= kTableKeys<D, PB> + kTableKeysPerQuery<D> * (nq - 1)) {
+      constexpr int QB = kTableBlockQueries<PB>;
+      hipLaunchKernelGGL((qjl_scores_table_kernel<D, PB>),
+                         dim3((unsigned)((nk + kBlock - 1) / kBlock), (unsigned)((nq + QB - 1) / QB)), dim3(kBlock), 0, stream, ctx, nq, polar_packed, polar_scales,
+                         reinterpret_cast<const uint32_t *>(signs), residual_norms, nk, scores, k);
+      return tqh::check_launch("qjl_scores_table_kernel");
+    }
+    const long long qblocks = (nq + 15) / 16, tiles = (nk + 15) / 16 * qblocks;
+    const long long blocks = tiles > (long long)kScoreBlocks * (kBlock / 64) * kScoreTiles ? 2 * kScoreBlocks : kScoreBlocks;
+    const long long room = std::max(1ll, blocks / qblocks);
+    hipLaunchKernelGGL((qjl_scores_kernel<D, PB>), dim3((unsigned)std::min((nk + 63) / 64, room), (unsigned)qblocks),
                        dim3(kBlock), 0, stream, ctx, nq, polar_packed, polar_scales, signs, residual_norms, nk, scores,
                        k, centroid_parts(k.polar, polar_bits));
     return tqh::check_launch("qjl_scores_kernel");
