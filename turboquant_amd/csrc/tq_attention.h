@@ -406,12 +406,24 @@ using StreamCfg64 = DecCfg<BITS, MODE, NQB, HG, 64, 8>;
 // Compute units of the current device (cached per device).
 int device_cus();
 
+// Stores a decode's token in a launch of its own.  A TQ cache's projects the
+// query with it, as rq in the reference's order, and the attention reads that
+// instead of forming R q in every workgroup.
+inline int store_token_apart(const tqh::AppendToken &t, AttnArgs &a, hipStream_t st) {
+  const int rc = tqh::store_token(t, st);
+  if (rc == TQ_OK && t.rq) {
+    a.rq = t.rq;
+    a.rmat = nullptr;
+  }
+  return rc;
+}
+
 // Launches the streaming decode (grid: chunks or ranges, head groups x KV
 // heads, batch) for BITS-bit records of cache mode MODE; a.chunk, a.cpr and
 // grid.x are set from the launched configuration.  INLINE: the last
 // workgroup of a (sequence, KV head) merges the split-K partials; else the
 // caller launches stream_merge_kernel after it.  ap: a token to store before
-// attending (INLINE, PQO and PQ only; its status in ap->rc).  Defined in the
+// attending (INLINE only; its status in ap->rc).  Defined in the
 // tq_attention_k<BITS>_<mode>.hip units.
 template <int BITS, int MODE, bool INLINE>
 void launch_stream_bm(AttnArgs &a, int nqb, int hg, dim3 grid, hipStream_t st, tqh::AppendToken *ap);

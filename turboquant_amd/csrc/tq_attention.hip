@@ -361,7 +361,7 @@ int decode_attention_ws(const void *q, int q_dtype, const uint8_t *k_indices, co
   // sketch); the workgroup that holds the last tokens starts its keys 1.5 us later
   // (2.9 with a sketch).
   if (append && (codec.norm_mode != TQ_NORM_MAXNORM || a.nr > 8)) {
-    rc = tqh::store_token(*append, stream);
+    rc = store_token_apart(*append, a, stream);
     if (rc) return rc;
     append = nullptr;
   }

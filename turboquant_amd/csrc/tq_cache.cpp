@@ -300,7 +300,8 @@ class KvCache {
       if (rc) return rc;
     }
     // a TqCache whose append did not project q (none, or one token that the
-    // decode launch stores): the decode launch projects it from the sign matrix
+    // decode stores): the decode launch projects it from the sign matrix,
+    // unless it leaves the token to a launch of its own
     const bool in_launch = mode_.qjl && !rq_ready;
     if (in_launch) {
       rc = sign_matrix(stream);
@@ -317,7 +318,8 @@ class KvCache {
   }
 
   // decode of one token per head: stored by the launch that attends, which
-  // also projects a TqCache's query
+  // then projects a TqCache's query too (a launch of the append's own does
+  // both where the attention's cannot store)
   int append_attend(int l, const void *k, const void *v, int dtype, const void *q, int q_dtype, int num_q_heads,
                     float scale, void *out, int out_dtype, hipStream_t stream) {
     const size_t old = storage_.seq_len(l);
@@ -336,9 +338,15 @@ class KvCache {
     if (mode_.qjl) {
       rc = sign_matrix(stream);
       if (rc) return rc;
+      rc = rq_scratch((size_t)num_q_heads, stream);
+      if (rc) return rc;
       t.signs = L.signs;
       t.norms = L.norms;
       t.sign_matrix = static_cast<const uint32_t *>(rmat_);
+      t.q = q;
+      t.q_dtype = q_dtype;
+      t.rq = static_cast<float *>(rq_);
+      t.num_q_rows = (size_t)num_q_heads;
     }
     t.head_stride = (long long)L.cap;
     t.offset = (long long)old;

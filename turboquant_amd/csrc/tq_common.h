@@ -61,7 +61,8 @@ int polar_codec(int bits, int norm_mode, size_t outlier_blocks, int num_blocks, 
 // One token's k and v, [num_heads][1][head_dim] of `dtype`, that a decode
 // launch stores at record h * head_stride + offset of every head before it
 // attends; the length it attends over includes it.  signs, norms and
-// sign_matrix: a TQ cache's, whose key is sketched too.
+// sign_matrix: a TQ cache's, whose key is sketched too; q and rq: its decode's
+// query rows and where a launch of the append's own leaves R q.
 struct AppendToken {
   const void *k, *v;
   int dtype, num_heads;
@@ -74,9 +75,13 @@ struct AppendToken {
   int head_dim, bits;
   size_t outlier_blocks;
   int norm_mode;
+  const void *q;
+  int q_dtype;
+  float *rq;
+  size_t num_q_rows;
   int rc;  // status of a launch of its own, where the decode took one
 };
-// The same as a launch of its own.
+// The same as a launch of its own, which projects q too.
 int store_token(const AppendToken &t, hipStream_t stream);
 
 // Fused decode attention (tq_cache_decode_attention) with the length given

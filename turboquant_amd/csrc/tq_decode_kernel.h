@@ -1374,7 +1374,7 @@ void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint, tqh::
     }
   }
   if (ap) {  // range launches: long contexts, where a launch more does not show
-    ap->rc = tqh::store_token(*ap, st);
+    ap->rc = store_token_apart(*ap, a, st);
     if (ap->rc) return;
   }
   auto go = [&](auto kernel) {

@@ -519,6 +519,10 @@ int store_token(const AppendToken &t, hipStream_t stream) {
     a.bits = t.bits;
     a.norm_mode = t.norm_mode;
     a.sign_matrix = t.sign_matrix;
+    a.q = t.q;
+    a.q_dtype = t.q_dtype;
+    a.rq = t.rq;
+    a.num_q_rows = t.num_q_rows;
     return tq_append(a, stream);
   }
   return polar_quantize_to_cache(t.k, t.v, t.dtype, t.num_heads, 1, t.k_idx, t.k_sc, t.v_idx, t.v_sc, t.head_stride,
