@@ -18,6 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("d,bits,nr,t", [
     (256, 3, 4, 255), (256, 4, 8, 256), (256, 4, 4, 257), (256, 3, 8, 513), (256, 3, 2, 511), (256, 4, 1, 1025),
     (128, 4, 4, 512), (128, 3, 4, 513), (128, 3, 8, 1024), (128, 4, 8, 1025), (64, 3, 8, 65), (64, 4, 8, 2049),
+    (256, 3, 4, 512), (256, 4, 4, 2000), (256, 3, 8, 16384), (256, 3, 4, 16385), (256, 4, 4, 16382),
 ])
 def test_workgroup_size_edges(tq, d, bits, nr, t):  # noqa: F811
     hkv = 2

@@ -1472,12 +1472,22 @@ void launch_stream_cfg(AttnArgs &a, dim3 grid, hipStream_t st, tqh::AppendToken 
   if constexpr (INLINE && C::WAVES != 4) {
     const long long wgs = (long long)((a.max_len + C::CHUNK - 1) / C::CHUNK) * grid.y * grid.z;
     if (wgs > device_cus()) return launch_stream_c<C4, INLINE>(a, grid, st, ap);
-    // sequences that 4 waves of 64 tokens hold: 4 more would only join the
-    // combine (head_dim 256, PQ 4 bits, 8 heads, 128 tokens 19.0 us against
-    // 22.0; with the QJL correction they halve the projection instead, 2
-    // heads, 81 tokens 17.5 against 15.9)
-    if constexpr (C::TPW == 64 && !C::QJL) {
-      if (a.max_len <= C4::CHUNK) return launch_stream_c<C4, INLINE>(a, grid, st, ap);
+    // 64 tokens a wave at head_dim 256: 4 waves where they hold the whole
+    // sequence (4 more would only join the combine) and from the length that
+    // 8 waves do not hold (one chunk, no merge: PQO 3 bits, 8 heads, 257
+    // tokens 21.4 us against 30.1 in two) while the 4-wave grid still fits one
+    // round, up to 64 partials a head: the setup and the combine of 8 waves'
+    // sums cost more than the merge of twice the partials.  4 / 8 waves, us,
+    // 2,500 tokens: 8 heads PQO 3 bits 30.4 / 32.7, PQ 3 bits 30.6 / 33.0, PQ 4
+    // bits 32.3 / 37.8, QJL 4 bits 39.9 / 43.6; 4 heads PQ 4 bits 19.4 / 22.0;
+    // past 64 partials, 8 heads, 18,000 tokens 41.4 / 36.4, 32,768 95 / 38.
+    // With the QJL correction at 3 bits, or up to 2 heads, 8 waves halve the
+    // projection instead (4 heads, 2,500 tokens 26.3 / 25.4, 2 heads, 81 tokens
+    // 17.5 / 15.9).
+    if constexpr (C::TPW == 64 && (C::QJL ? C::NQB == 8 && BITS == 4 && HG >= 4 : true)) {
+      const long long chunks = (a.max_len + C4::CHUNK - 1) / C4::CHUNK;
+      if (chunks <= 1 || (a.max_len > C::CHUNK && chunks <= 64 && chunks * grid.y * grid.z <= device_cus()))
+        return launch_stream_c<C4, INLINE>(a, grid, st, ap);
     }
     // a grid that leaves compute units idle: 64 tokens per wave when that
     // grid still fits one round (C3's shape up to 16,384 tokens: 2,048 and
