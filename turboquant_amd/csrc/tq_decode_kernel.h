@@ -1344,6 +1344,28 @@ __global__ __launch_bounds__(C::THREADS, TQ_DECODE_WPE) void stream_decode_kerne
 #define TQ_BAL_WGS 3  // at most this many balanced workgroups per compute unit
 #endif
 
+// A kernel as a type of its own (kernels of one signature share a pointer type).
+template <auto K>
+struct Kernel {
+  static constexpr auto value = K;
+};
+// Workgroups of K that a compute unit holds at once, up to TQ_BAL_WGS (cached
+// per kernel and device: a configuration's kernels differ in registers and LDS).
+template <auto K, int THREADS>
+int resident_workgroups() {
+  static int occ[64] = {};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  dev = dev >= 0 && dev < 64 ? dev : 0;
+  if (occ[dev] == 0) {
+    int n = 0;
+    occ[dev] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, K, THREADS, 0) == hipSuccess && n > 0
+                   ? min(n, TQ_BAL_WGS)
+                   : 2;
+  }
+  return occ[dev];
+}
+
 // 4-bit codes on the compiled-in MaxNorm codebook (evenly spaced) take the
 // grid key pass; a caller's codebook or the L2Norm tables, the pair table
 template <class C, bool INLINE, bool MULTI>
@@ -1377,33 +1399,24 @@ void launch_stream_k(AttnArgs &a, dim3 grid, hipStream_t st, int len_hint, tqh::
     ap->rc = store_token_apart(*ap, a, st);
     if (ap->rc) return;
   }
-  auto go = [&](auto kernel) {
+  auto go = [&](auto k) {
+    constexpr auto kernel = decltype(k)::value;
     if (a.bal_nwg < 0) {
-      // balanced split: as many workgroups as the compute units hold at once
-      // (this kernel's occupancy, cached per device), at most one per task
-      static int occ[64] = {};
-      int dev = 0;
-      (void)hipGetDevice(&dev);
-      dev = dev >= 0 && dev < 64 ? dev : 0;
-      if (occ[dev] == 0) {
-        int n = 0;
-        occ[dev] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, C::THREADS, 0) == hipSuccess && n > 0
-                       ? min(n, TQ_BAL_WGS)
-                       : 2;
-      }
-      a.bal_nwg = (int)min((long long)-a.bal_nwg, (long long)occ[dev] * device_cus());
+      // balanced split: as many workgroups as the compute units hold at once,
+      // at most one per task
+      a.bal_nwg = (int)min((long long)-a.bal_nwg, (long long)resident_workgroups<kernel, C::THREADS>() * device_cus());
       grid = dim3((unsigned)a.bal_nwg, 1u, 1u);
     }
     hipLaunchKernelGGL(kernel, grid, dim3(C::THREADS), 0, st, a.k_idx, a.v_idx, a.k_sc, a.v_sc, a.seq_stride,
                        a.kv_head_stride, len_hint, a, NoAppend{});
   };
   if constexpr (C::BITS == 4 && C::MODE == kModePqo) {
-    if (!a.cb_dev && !a.cb_args) return go(stream_decode_kernel<C, INLINE, true, MULTI>);
+    if (!a.cb_dev && !a.cb_args) return go(Kernel<stream_decode_kernel<C, INLINE, true, MULTI>>{});
   }
   if constexpr (C::QJL) {
-    if (!a.rq) return go(stream_decode_kernel<C, INLINE, false, MULTI, true>);
+    if (!a.rq) return go(Kernel<stream_decode_kernel<C, INLINE, false, MULTI, true>>{});
   }
-  go(stream_decode_kernel<C, INLINE, false, MULTI>);
+  go(Kernel<stream_decode_kernel<C, INLINE, false, MULTI>>{});
 }
 template <class C, bool INLINE>
 void launch_stream_c(AttnArgs &a, dim3 grid, hipStream_t st, tqh::AppendToken *ap) {
