@@ -38,6 +38,8 @@ def _bias64(rq, signs, norms, d):
 @pytest.mark.parametrize("d,heads,q_len,kv_len,dtype", [
     (128, 2, 1, 1, "f32"), (128, 4, 3, 63, "bf16"), (64, 2, 16, 64, "f16"), (64, 6, 11, 65, "f32"),
     (128, 2, 65, 511, "bf16"), (256, 2, 17, 513, "f32"), (128, 8, 16, 1030, "f16"), (256, 4, 40, 260, "bf16"),
+    (64, 4, 2, 257, "f32"), (256, 6, 1, 1025, "bf16"), (64, 64, 1, 16385, "f16"), (256, 2, 4, 16384, "f32"), (64, 2, 300, 6700, "bf16"),
+    (128, 4, 3, 129, "f32"), (256, 2, 70, 127, "f16"),
 ])
 def test_bias_of_given_projections(tq, d, heads, q_len, kv_len, dtype):
     hk = 2
@@ -77,7 +79,7 @@ def test_infinite_and_nan_projections(tq):
 
 @pytest.mark.parametrize("d,hq,t,q_len,dtype,skew", [
     (64, 4, 33, 5, "f16", 0), (128, 2, 70, 1, "f32", 0), (128, 4, 64, 33, "bf16", 0), (256, 4, 20, 18, "f32", 0),
-    (128, 4, 40, 3, "bf16", 1),
+    (128, 4, 40, 3, "bf16", 1), (256, 2, 16385, 2, "f32", 0),
 ])
 def test_bias_of_queries_in_the_cache(tq, d, hq, t, q_len, dtype, skew):
     """skew: the queries start one element past a 16-byte boundary, which takes the launch that reads rq."""

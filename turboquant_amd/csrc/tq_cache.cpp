@@ -269,7 +269,12 @@ class KvCache {
   // bias [num_q_heads][q_len][seq_len] in q's dtype
   int logit_bias(int l, const void *q, int q_dtype, int num_q_heads, int q_len, void *bias, hipStream_t stream) {
     const LayerBuffers &L = storage_.layer(l);
-    if (reinterpret_cast<uintptr_t>(q) % 16 == 0) {  // 16-byte loads of the query rows
+    // one launch, which projects its rows in every block of 512 tokens; at
+    // head_dim 256 and one or two positions over a long sequence that costs
+    // more than a launch of its own (f32, 8 heads, 32,768 tokens 28 us against
+    // 7 + 5).  The query rows by 16-byte loads.
+    const bool apart = head_dim_ == 256 && q_len <= 2 && L.seq >= 16384;
+    if (!apart && reinterpret_cast<uintptr_t>(q) % 16 == 0) {
       int rc = sign_matrix(stream);
       if (rc) return rc;
       return tqh::query_logit_bias(q, q_dtype, static_cast<const uint32_t *>(rmat_), num_q_heads, q_len, L.signs,

@@ -34,7 +34,14 @@ namespace {
 using namespace tqd;
 using namespace tqm;
 
-constexpr int kRows = 64, kThreads = 512, kTokens = kThreads;
+constexpr int kRows = 64, kThreads = 512;
+// Given rows in a grid of at most this many workgroups of 512 tokens take 128
+// tokens a workgroup instead (16 a wave): a fourth of the operands to expand
+// and four times the workgroups (us, 512 / 128 tokens, 16 query heads on 8: 8
+// rows x 1,000 tokens, d = 128 4.7 / 3.5, d = 256 7.7 / 4.7; 40 x 1,000 d = 64
+// 5.8 / 4.0; at 128 workgroups, 16 x 8,000, d = 64 4.6 / 4.3, at 256, 40 x 8,000,
+// 6.7 / 8.3).
+constexpr int kFewBlocks = 128;
 
 // Where the staged rows come from: rq as given (f32), or R q of bf16, f16 or
 // f32 query rows.
@@ -51,13 +58,13 @@ struct BiasArgs {
   long long head_stride;
   float sf;
   void *out;
-  int token_blocks;
+  int token_blocks, kv_heads, q_heads;
 };
 
 // Four values as consecutive elements of type OUT.  Rows of kv_len elements
 // start anywhere, so the store is of unaligned bytes.
 template <int OUT>
-__device__ __forceinline__ void store4(char *p, const float (&v)[4]) {
+__device__ __forceinline__ void store4(char *p, const float *v) {
   if constexpr (OUT == kF32) {
     __builtin_memcpy(p, v, 16);
   } else {
@@ -73,9 +80,9 @@ __device__ __forceinline__ void store1(char *p, float v) {
   else *reinterpret_cast<uint16_t *>(p) = OUT == kBF16 ? f32_to_bf16(v) : f32_to_f16(v);
 }
 
-template <int D, int SRC, int OUT>
-__global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_kernel(BiasArgs a) {
-  constexpr int NS = D / 32, JH = D / 32, TT = 4, OB = OUT == kF32 ? 4 : 2;
+template <int D, int SRC, int OUT, int TT>
+__global__ __launch_bounds__(kThreads, D == 256 && TT == 4 ? 2 : 4) void qjl_logit_bias_kernel(BiasArgs a) {
+  constexpr int NS = D / 32, JH = D / 32, OB = OUT == kF32 ? 4 : 2;
   constexpr int RS = D + 8;  // halves per staged row: 16-byte chunks of 16 rows in different banks
   __shared__ uint2 s_nib[16];
   __shared__ __attribute__((aligned(16))) uint16_t s_hi[kRows * RS], s_lo[kRows * RS];
@@ -88,13 +95,13 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
   const int r0 = rblk * kRows, nrows = min(kRows, a.rows - r0);
   const long long row0 = (long long)g * a.rows + r0;
 
-  // the wave's tokens: column l16 of tile T is token t0 + 4 l16 + T
-  const int t0 = tblk * kTokens + wave * 64;
+  // the wave's tokens: column l16 of tile T is token t0 + TT l16 + T
+  const int t0 = (tblk * (kThreads / 64) + wave) * (16 * TT);
   uint32_t sw[TT][NS];
   float c[TT];
 #pragma unroll
   for (int T = 0; T < TT; T++) {
-    const long long rec = (long long)g * a.head_stride + min(t0 + 4 * l16 + T, a.kv_len - 1);
+    const long long rec = (long long)g * a.head_stride + min(t0 + TT * l16 + T, a.kv_len - 1);
 #pragma unroll
     for (int s = 0; s < NS; s++) sw[T][s] = a.signs[rec * NS + s];
     c[T] = f16_to_f32(a.norms[rec]) * a.sf;
@@ -106,27 +113,47 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
   }
 
   if constexpr (SRC == kGiven) {
-    // wave w stages rows 8 w .. + 7, D / 4 lanes of 4 elements per row
-    constexpr int LPR = D / 4, RPS = 64 / LPR;
+    // wave w stages rows 8 w .. + 7, D / 4 lanes of 4 elements per row; a step
+    // past the last row stages nothing (its outputs are not stored)
+    constexpr int LPR = D / 4, RPS = 64 / LPR, STEPS = 8 / RPS;
+    const int e0 = 4 * (lane % LPR), left = nrows - 8 * wave;
+    float x[STEPS][4], m[STEPS];
 #pragma unroll
-    for (int step = 0; step < 8 / RPS; step++) {
-      const int row = 8 * wave + step * RPS + lane / LPR, e0 = 4 * (lane % LPR);
-      float x[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int step = 0; step < STEPS; step++) {  // every load goes out before the first is used
+      const int row = 8 * wave + step * RPS + lane / LPR;
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[step][i] = 0.f;
       if (row < nrows) {
         const float *p = static_cast<const float *>(a.src) + (row0 + row) * D + e0;
 #pragma unroll
-        for (int i = 0; i < 4; i++) x[i] = p[i];
+        for (int i = 0; i < 4; i++) x[step][i] = p[i];
       }
-      float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+    }
+    if (left > 0) {
 #pragma unroll
-      for (int o = 1; o < LPR; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-      const int e = row_exponent(m);
-      uint16_t hi[4], lo[4];
+      for (int step = 0; step < STEPS; step++)
+        m[step] = fmaxf(fmaxf(fabsf(x[step][0]), fabsf(x[step][1])), fmaxf(fabsf(x[step][2]), fabsf(x[step][3])));
+      auto fold = [&](auto op) {  // the steps' lane exchanges side by side
 #pragma unroll
-      for (int i = 0; i < 4; i++) split2(x[i], -e, hi[i], lo[i]);
-      *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
-      *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
-      if (lane % LPR == 0) s_exp[row] = e;
+        for (int step = 0; step < STEPS; step++) m[step] = op(m[step]);
+      };
+      fold([](float v) { return fmaxf(v, lane_xor<1>(v)); });
+      fold([](float v) { return fmaxf(v, lane_xor<2>(v)); });
+      fold([](float v) { return fmaxf(v, lane_xor<4>(v)); });
+      fold([](float v) { return fmaxf(v, lane_xor<8>(v)); });
+      if constexpr (LPR > 16) fold([](float v) { return max_xor16(v); });
+      if constexpr (LPR > 32) fold([](float v) { return max_xor32(v); });
+#pragma unroll
+      for (int step = 0; step < STEPS; step++) {
+        if (step * RPS >= left) break;  // uniform
+        const int row = 8 * wave + step * RPS + lane / LPR, e = row_exponent(m[step]);
+        uint16_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) split2(x[step][i], -e, hi[i], lo[i]);
+        *reinterpret_cast<uint2 *>(s_hi + row * RS + e0) = make_uint2(pack_pair(hi[0], hi[1]), pack_pair(hi[2], hi[3]));
+        *reinterpret_cast<uint2 *>(s_lo + row * RS + e0) = make_uint2(pack_pair(lo[0], lo[1]), pack_pair(lo[2], lo[3]));
+        if (lane % LPR == 0) s_exp[row] = e;
+      }
     }
   } else {
     // Waves w and w + 4 project rows 16 w .. + 15, each for half of R's
@@ -244,7 +271,7 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
       b[T][s] = u32x4{n0.x, n0.y, n1.x, n1.y};
     }
 
-  const int t = t0 + 4 * l16;
+  const int t = t0 + TT * l16;
   const long long pitch = (long long)a.kv_len * OB;  // bytes of an output row
   char *base = static_cast<char *>(a.out) + row0 * pitch;
   const long long at = 4 * lg * pitch + (long long)t * OB;  // the lane's first row, first token
@@ -276,7 +303,7 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
       for (int T = 0; T < TT; T++) v[T] = __builtin_amdgcn_ldexpf(acc[T][i], ex[i]) * c[T];
       char *p = base + i * pitch + at;
       if (i < left) {
-        if (t + 4 <= a.kv_len) {
+        if (TT == 4 && t + 4 <= a.kv_len) {
           store4<OUT>(p, v);
         } else {
 #pragma unroll
@@ -288,21 +315,92 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 2 : 4) void qjl_logit_bias_ker
   }
 }
 
-template <int D, int SRC, int OUT>
-int launch_one(const BiasArgs &a, dim3 grid, hipStream_t st) {
-  hipLaunchKernelGGL((qjl_logit_bias_kernel<D, SRC, OUT>), grid, dim3(kThreads), 0, st, a);
+// One or two positions of given rows: lane = token, a query's sum over sign
+// nibbles in LDS tables, D / 4 entries a value added in f32.  The products
+// above first split and exchange their rows, a chain that so few rows do not
+// repay, and at head_dim 256 a long sequence's grid runs in two rounds (us,
+// products / tables, 16 query heads on 8, one position: d = 128, 1,000 tokens
+// 3.0 / 2.8, 32,768 tokens 5.4 / 4.6; d = 256 3.8 / 3.5, 11.5 / 7.4; two
+// positions d = 256 x 32,768 13.1 / 10.7).  Every query head reads the signs
+// again, so more than 2^20 values stay with the products (32 heads, two
+// positions x 32,768, d = 128 6.6 / 9.9).
+template <int D>
+constexpr int kTablePositions = D == 256 ? 4 : 2;  // (3 and 4 from 16,384 tokens on: 8 heads x 32,768 13.1 / 9.9)
+constexpr long long kTableValues = 1 << 20;
+// At d = 256 five waves a SIMD at most: registers for more LDS reads in flight
+// (eight waves: 1,000 tokens 4.6 us against 3.5).
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 256 ? 5 : 8))) void qjl_logit_bias_table_kernel(const float *__restrict__ rq, int q_len,
+                                                                   const uint32_t *__restrict__ signs,
+                                                                   const uint16_t *__restrict__ norms, int kv_len,
+                                                                   long long head_stride, int n_rep, float sf,
+                                                                   void *__restrict__ out, int out_dtype) {
+  constexpr int CT = (D / 4) * 16;
+  __shared__ float s_tab[kTablePositions<D> * CT];
+  const int h = blockIdx.z;
+  for (int e = threadIdx.x; e < q_len * CT; e += 256) {
+    const int ql = e / CT, rr = e % CT, c = rr / 16, m = rr % 16;
+    const float *rp = rq + (((long long)h * q_len + ql) * D) + 4 * c;
+    float val = -0.0f;
+#pragma unroll
+    for (int b = 0; b < 4; b++) val = val + (((m >> b) & 1) ? rp[b] : -rp[b]);
+    s_tab[e] = val;
+  }
+  __syncthreads();
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= kv_len) return;
+  const long long rec = (long long)(h / n_rep) * head_stride + t;
+  uint32_t sgn[D / 32];
+#pragma unroll
+  for (int w = 0; w < D / 32; w++) sgn[w] = signs[rec * (D / 32) + w];
+  const float c = f16_to_f32(norms[rec]) * sf;
+  for (int ql = 0; ql < q_len; ql++) {
+    const float *tb = s_tab + ql * CT;
+    float raw = 0.0f;
+#pragma unroll
+    for (int cc = 0; cc < D / 4; cc++) raw += tb[cc * 16 + ((sgn[cc >> 3] >> ((cc & 7) * 4)) & 15u)];
+    const float val = raw * c;
+    const long long oi = ((long long)h * q_len + ql) * kv_len + t;
+    if (out_dtype == kF32) static_cast<float *>(out)[oi] = val;
+    else if (out_dtype == kBF16) static_cast<uint16_t *>(out)[oi] = f32_to_bf16(val);
+    else static_cast<uint16_t *>(out)[oi] = f32_to_f16(val);
+  }
+}
+
+template <int D, int SRC, int OUT, int TT = 4>
+int launch_one(BiasArgs &a, hipStream_t st) {
+  constexpr int TOKENS = kThreads / 64 * 16 * TT;
+  const long long tblocks = ((long long)a.kv_len + TOKENS - 1) / TOKENS, rblocks = ((long long)a.rows + kRows - 1) / kRows;
+  if (tblocks * rblocks > 0x7fffffffll)
+    return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many query rows (%d) for %d tokens", a.rows, a.kv_len);
+  a.token_blocks = (int)tblocks;
+  hipLaunchKernelGGL((qjl_logit_bias_kernel<D, SRC, OUT, TT>), dim3((unsigned)(tblocks * rblocks), 1, (unsigned)a.kv_heads),
+                     dim3(kThreads), 0, st, a);
   return tqh::check_launch("qjl_logit_bias_kernel");
 }
 
 // Query sources write their own type; rows that were given any.
 template <int D>
-int launch_bias(const BiasArgs &a, int source, int out_dtype, dim3 grid, hipStream_t st) {
-  if (source == kFromF32) return launch_one<D, kFromF32, kF32>(a, grid, st);
-  if (source == kFromBF16) return launch_one<D, kFromBF16, kBF16>(a, grid, st);
-  if (source == kFromF16) return launch_one<D, kFromF16, kF16>(a, grid, st);
-  if (out_dtype == kF32) return launch_one<D, kGiven, kF32>(a, grid, st);
-  if (out_dtype == kBF16) return launch_one<D, kGiven, kBF16>(a, grid, st);
-  return launch_one<D, kGiven, kF16>(a, grid, st);
+int launch_bias(BiasArgs &a, int source, int out_dtype, hipStream_t st) {
+  if (source == kFromF32) return launch_one<D, kFromF32, kF32>(a, st);
+  if (source == kFromBF16) return launch_one<D, kFromBF16, kBF16>(a, st);
+  if (source == kFromF16) return launch_one<D, kFromF16, kF16>(a, st);
+  const int n_rep = a.q_heads / a.kv_heads, q_len = a.rows / n_rep;
+  if (q_len <= (a.kv_len >= 16384 ? kTablePositions<D> : 2) && (long long)a.rows * a.kv_heads * a.kv_len <= kTableValues) {
+    hipLaunchKernelGGL((qjl_logit_bias_table_kernel<D>), dim3((unsigned)((a.kv_len + 255) / 256), 1, (unsigned)a.q_heads),
+                       dim3(256), 0, st, static_cast<const float *>(a.src), q_len, a.signs, a.norms, a.kv_len,
+                       a.head_stride, n_rep, a.sf, a.out, out_dtype);
+    return tqh::check_launch("qjl_logit_bias_table_kernel");
+  }
+  const long long blocks = (long long)((a.kv_len + kThreads - 1) / kThreads) * ((a.rows + kRows - 1) / kRows) * a.kv_heads;
+  if (blocks <= kFewBlocks) {
+    if (out_dtype == kF32) return launch_one<D, kGiven, kF32, 1>(a, st);
+    if (out_dtype == kBF16) return launch_one<D, kGiven, kBF16, 1>(a, st);
+    return launch_one<D, kGiven, kF16, 1>(a, st);
+  }
+  if (out_dtype == kF32) return launch_one<D, kGiven, kF32>(a, st);
+  if (out_dtype == kBF16) return launch_one<D, kGiven, kBF16>(a, st);
+  return launch_one<D, kGiven, kF16>(a, st);
 }
 
 int bias(const void *src, int source, const uint32_t *rbits, int num_q_heads, int q_len, const uint8_t *signs,
@@ -318,8 +416,7 @@ int bias(const void *src, int source, const uint32_t *rbits, int num_q_heads, in
   if (q_len == 0 || kv_len == 0) return TQ_OK;
   if (!src || !signs || !norms || !out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
   const long long rows = (long long)(num_q_heads / num_kv_heads) * q_len;
-  const long long tblocks = ((long long)kv_len + kTokens - 1) / kTokens, rblocks = (rows + kRows - 1) / kRows;
-  if (rows > 0x7fffffffll || tblocks * rblocks > 0x7fffffffll)
+  if (rows > 0x7fffffffll)
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many query rows (%lld) for %d tokens", rows, kv_len);
   BiasArgs a{};
   a.src = src;
@@ -332,11 +429,11 @@ int bias(const void *src, int source, const uint32_t *rbits, int num_q_heads, in
   a.head_stride = head_stride;
   a.sf = tq_qjl_bias_scale(head_dim);
   a.out = out;
-  a.token_blocks = (int)tblocks;
-  const dim3 grid((unsigned)(tblocks * rblocks), 1, (unsigned)num_kv_heads);
-  if (head_dim == 64) return launch_bias<64>(a, source, out_dtype, grid, stream);
-  if (head_dim == 128) return launch_bias<128>(a, source, out_dtype, grid, stream);
-  return launch_bias<256>(a, source, out_dtype, grid, stream);
+  a.kv_heads = num_kv_heads;
+  a.q_heads = num_q_heads;
+  if (head_dim == 64) return launch_bias<64>(a, source, out_dtype, stream);
+  if (head_dim == 128) return launch_bias<128>(a, source, out_dtype, stream);
+  return launch_bias<256>(a, source, out_dtype, stream);
 }
 
 }  // namespace
