@@ -142,7 +142,7 @@ def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):
     assert np.abs(got - w.astype(np.float64) @ vals).max() <= bound
 
 
-@pytest.mark.parametrize("rows,cols", [(3, 1), (2, 1023), (2, 1025), (1, 16384), (2, 16385), (1, 20000)])
+@pytest.mark.parametrize("rows,cols", [(3, 1), (2, 1023), (2, 1025), (1, 16384), (2, 16385), (1, 20000), (2, 1024), (3, 4096), (2, 4097)])
 def test_softmax_column_edges(tq, rows, cols):
     s = np.random.default_rng(cols).standard_normal((rows, cols)).astype(np.float32) * 5
     s[0, cols // 2] = -np.inf if cols > 1 else 0.0
