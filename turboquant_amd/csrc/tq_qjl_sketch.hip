@@ -84,10 +84,25 @@ template <int D>
 __device__ __forceinline__ void project_rows(const void *q, int q_dtype, float *rq, long long row0, long long nq,
                                              float inv, float *s_v, const uint32_t (&rb)[2][Geo<D>::NW], int tid,
                                              int wave, int l16, int lg) {
-  for (int i = tid; i < kVecs * D; i += Geo<D>::THREADS) {
-    const int r = i / D, e = i % D;
-    s_v[r * Geo<D>::RS + e] = row0 + r < nq ? load_elem(q, row0 * D + i, q_dtype) : 0.f;
+  // a thread's 8 elements by one or two loads, from any element boundary (one
+  // element a load, one after the other: 16 bf16 rows of d = 64 3.7 us, 2.6 now)
+  static_assert(8 * Geo<D>::THREADS == kVecs * D, "8 elements a thread");
+  const int r = 8 * tid / D, e = 8 * tid % D;
+  float x[8] = {};
+  if (row0 + r < nq) {
+    const long long i = row0 * D + 8 * tid;
+    if (q_dtype == kF32) {
+      __builtin_memcpy(x, static_cast<const float *>(q) + i, 32);
+    } else {
+      uint16_t h[8];
+      __builtin_memcpy(h, static_cast<const uint16_t *>(q) + i, 16);
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] = q_dtype == kBF16 ? bf16_to_f32(h[j]) : f16_to_f32(h[j]);
+    }
   }
+  float4 *dst = reinterpret_cast<float4 *>(s_v + r * Geo<D>::RS + e);
+  dst[0] = make_float4(x[0], x[1], x[2], x[3]);
+  dst[1] = make_float4(x[4], x[5], x[6], x[7]);
   __syncthreads();
   f32x4 acc[2];
   row_products<D>(s_v, rb, l16, lg, acc);
@@ -233,7 +248,7 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void qjl_project_kernel(const void
                                                                       const uint32_t *__restrict__ rbits,
                                                                       float *__restrict__ rq, long long nrows,
                                                                       float inv) {
-  __shared__ float s_v[kVecs * Geo<D>::RS];
+  __shared__ __attribute__((aligned(16))) float s_v[kVecs * Geo<D>::RS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint32_t rb[2][Geo<D>::NW];
   load_rows<D>(rbits, wave, lane & 15, lane >> 4, rb);
