@@ -132,7 +132,8 @@ def test_scores_are_as_exact_as_f32_sums(tq, dim, tb):
 
 
 @pytest.mark.parametrize("dim,pb,nv,nq", [(128, 2, 1, 1), (128, 3, 255, 17), (64, 3, 257, 16), (32, 2, 770, 5),
-                                          (32, 3, 4100, 3), (64, 2, 4352, 33)])
+                                          (32, 3, 4100, 3), (64, 2, 4352, 33),
+                                          (32, 3, 5, 17), (64, 3, 31, 2), (128, 3, 32, 16), (64, 2, 33, 1)])
 def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):
     packed, scales = orc.quantize_vec_batch(pb, dim, 42, orc.lcg_normal_vecs(3 + nv, dim, nv))
     w = np.random.default_rng(nv).random((nq, nv)).astype(np.float32)

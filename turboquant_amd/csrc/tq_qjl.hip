@@ -571,26 +571,30 @@ constexpr int kWvQueries = 16;
 // 64 queries x 8,192 values, d = 128, 2-bit codes, take 16.7 us with a lane
 // per element and 4 queries per workgroup, 9.5 us with each staged value
 // loaded under its own bounds check, 6.3 us with all loads in flight at once.
-template <int D, int PB>
+// CHUNK: kWvChunk, or kWvFew for lists of no more values (4 values, d = 32,
+// 16 queries: 5.6 us staging 256 places, 4.6 staging 32; a lane per element 4.7;
+// with the finish's launch).
+constexpr int kWvFew = 32;
+template <int D, int PB, int CHUNK>
 __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__restrict__ polar,
                                                                const uint16_t *__restrict__ polar_scales,
                                                                long long nv, long long nq,
                                                                const float *__restrict__ weights,
                                                                float *__restrict__ partial, QjlConsts k) {
-  constexpr int RW = D * PB / 32, THREADS = 4 * D, ST = kWvChunk / 4;  // words per value, steps
+  constexpr int RW = D * PB / 32, THREADS = 4 * D, ST = CHUNK / 4;  // words per value, steps
   constexpr int GS = ST + 4;                                           // [g] stride
   __shared__ __attribute__((aligned(16))) uint32_t s_codes[RW][4 * GS];
   __shared__ __attribute__((aligned(16))) float s_w[kWvQueries][4 * GS];
   __shared__ float s_cent[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
-  const long long t0 = (long long)blockIdx.x * kWvChunk, q0 = (long long)blockIdx.y * kWvQueries;
-  const int cnt = (int)min<long long>(kWvChunk, nv - t0);
+  const long long t0 = (long long)blockIdx.x * CHUNK, q0 = (long long)blockIdx.y * kWvQueries;
+  const int cnt = (int)min<long long>(CHUNK, nv - t0);
   if (tid < 16) s_cent[tid] = k.polar.cent[tid & ((1 << PB) - 1)];
   // every load goes out before the first is used; places past the end read
   // the last value or query and are stored as zeros
-  constexpr int NC = kWvChunk * RW / THREADS, NWT = kWvChunk * kWvQueries / THREADS;
-  static_assert(NC * THREADS == kWvChunk * RW && NWT * THREADS == kWvChunk * kWvQueries, "whole rounds");
+  constexpr int CW = CHUNK * RW, NC = (CW + THREADS - 1) / THREADS, NWT = CHUNK * kWvQueries / THREADS;
+  static_assert(NWT * THREADS == CHUNK * kWvQueries, "whole rounds");
   uint32_t cd[NC];
   float wt[NWT];
   uint16_t sc[NWT];
@@ -602,18 +606,18 @@ __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__
 #pragma unroll
   for (int j = 0; j < NWT; j++) {
     const int i = tid + j * THREADS;
-    const long long t = t0 + min(i % kWvChunk, cnt - 1);
-    wt[j] = weights[min<long long>(q0 + i / kWvChunk, nq - 1) * nv + t];
+    const long long t = t0 + min(i % CHUNK, cnt - 1);
+    wt[j] = weights[min<long long>(q0 + i / CHUNK, nq - 1) * nv + t];
     sc[j] = polar_scales[t];
   }
 #pragma unroll
   for (int j = 0; j < NC; j++) {
     const int i = tid + j * THREADS, t = i / RW;
-    s_codes[i % RW][(t & 3) * GS + (t >> 2)] = t < cnt ? cd[j] : 0u;
+    if (CW % THREADS == 0 || i < CW) s_codes[i % RW][(t & 3) * GS + (t >> 2)] = t < cnt ? cd[j] : 0u;
   }
 #pragma unroll
   for (int j = 0; j < NWT; j++) {
-    const int i = tid + j * THREADS, t = i % kWvChunk, qq = i / kWvChunk;
+    const int i = tid + j * THREADS, t = i % CHUNK, qq = i / CHUNK;
     s_w[qq][(t & 3) * GS + (t >> 2)] = t < cnt && q0 + qq < nq ? wt[j] * f16_to_f32(sc[j]) : 0.f;
   }
   __syncthreads();
@@ -885,7 +889,8 @@ extern "C" int tq_qjl_weighted_values(const uint8_t *polar_packed, const uint16_
   return by_dim_bits(dim, polar_bits, [&](auto d, auto pb) {
     constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
     if (nchunks > 0) {
-      hipLaunchKernelGGL((qjl_wv_partial_kernel<D, PB>), dim3((unsigned)nchunks, (unsigned)((nq + kWvQueries - 1) / kWvQueries)),
+      const auto kernel = nv <= kWvFew ? qjl_wv_partial_kernel<D, PB, kWvFew> : qjl_wv_partial_kernel<D, PB, kWvChunk>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nchunks, (unsigned)((nq + kWvQueries - 1) / kWvQueries)),
                          dim3(4 * D), 0, stream, polar_packed, polar_scales, nv, nq, weights, partial, k);
       int rc2 = tqh::check_launch("qjl_wv_partial_kernel");
       if (rc2) return rc2;
