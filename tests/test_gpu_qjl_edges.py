@@ -85,6 +85,26 @@ def test_scores_of_more_keys_than_a_grid_of_eight_lanes_a_key(tq):
     assert torch.equal(got[0, -1:], tq.qjl_scores(ctx, *last, 2, 42)[0]) and float(got[0, 5]) == 0.0
 
 
+def test_sketch_of_more_vectors_than_one_launch_holds(tq):
+    """2^28 + 1 vectors of 128: 512 lanes for 32 of them, and a launch holds fewer than 2^32.  The first and the last
+    one's records are those of the vector alone."""
+    n, dim = 2**28 + 1, 128
+    if torch.cuda.mem_get_info()[0] < 200 * 2**30:
+        pytest.skip("needs 200 GiB")
+    one = _dev(orc.lcg_normal_vecs(1, dim, 1))
+    x = torch.zeros((n, dim), device="cuda")
+    x[0], x[-1] = one[0], one[0]
+    ref = tq.qjl_quantize_batch(one, 3, 42, 5)
+    got = tq.qjl_quantize_batch(x, 3, 42, 5)
+    del x
+    try:
+        for r, g in zip(ref, got):
+            assert torch.equal(g[0], r[0]) and torch.equal(g[-1], r[0])
+    finally:
+        del got, g
+        torch.cuda.empty_cache()
+
+
 def test_scores_of_infinite_and_nan_queries(tq):
     """Rows with an infinity or a NaN are not finite, as the oracle's; the other rows of their tile keep their values,
     huge and tiny ones too; a key whose scale overflows f16 is not finite for any query."""
@@ -141,6 +161,13 @@ def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):
     vals = orc.dequantize_vec_batch(pb, dim, 42, packed, scales).astype(np.float64)
     bound = 1e-5 * (w.astype(np.float64) @ np.abs(vals)).max()
     assert np.abs(got - w.astype(np.float64) @ vals).max() <= bound
+
+
+def test_softmax_of_more_rows_than_one_launch_holds(tq):
+    x = torch.zeros((2**22 + 1, 3), device="cuda")
+    x[-1] = torch.tensor([0.0, 1.0, 2.0])
+    p = tq.softmax_rows(x, 1.0)
+    assert (p[:-1] == p[0]).all() and torch.allclose(p[-1].cpu(), torch.softmax(x[-1].cpu(), 0), atol=1e-6)
 
 
 @pytest.mark.parametrize("rows,cols", [(3, 1), (2, 1023), (2, 1025), (1, 16384), (2, 16385), (1, 20000), (2, 1024), (3, 4096), (2, 4097)])

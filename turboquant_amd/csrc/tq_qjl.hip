@@ -793,11 +793,18 @@ extern "C" int tq_qjl_quantize_batch(const float *data, uint8_t *polar_packed, u
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
   const long long n = (long long)num_vectors;
   return by_dim_bits(dim, total_bits - 1, [&](auto d, auto pb) {
-    hipLaunchKernelGGL((qjl_quant_kernel<decltype(d)::value, decltype(pb)::value>), dim3((unsigned)((n + 31) / 32)),
-                       dim3(4 * decltype(d)::value), 0, stream, data, polar_packed, polar_scales,
-                       reinterpret_cast<uint16_t *>(signs),
-                       residual_norms, n, k);
-    return tqh::check_launch("qjl_quant_kernel");
+    constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
+    // 32 vectors a workgroup of 4 D lanes, fewer than 2^32 lanes a launch
+    constexpr long long kMost = 32ll * ((1ll << 31) / (4 * D));
+    for (long long v = 0; v < n; v += kMost) {
+      const long long m = std::min(n - v, kMost);
+      hipLaunchKernelGGL((qjl_quant_kernel<D, PB>), dim3((unsigned)((m + 31) / 32)), dim3(4 * D), 0, stream, data + v * D,
+                         polar_packed + v * (D * PB / 8), polar_scales + v,
+                         reinterpret_cast<uint16_t *>(signs + v * (D / 8)), residual_norms + v, m, k);
+      const int rc2 = tqh::check_launch("qjl_quant_kernel");
+      if (rc2) return rc2;
+    }
+    return (int)TQ_OK;
   });
 }
 
@@ -858,9 +865,14 @@ extern "C" int tq_softmax_rows(const float *scores, float *probs, size_t rows, s
                       : keep <= 4  ? softmax_rows_kernel<4>
                       : keep <= 16 ? softmax_rows_kernel<16>
                                    : softmax_rows_kernel<0>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)rows),
-                     dim3(kSoftmaxBlock), 0, stream, scores, probs, (long long)cols, scale);
-  return tqh::check_launch("softmax_rows_kernel");
+  constexpr size_t kMost = (1ull << 31) / kSoftmaxBlock;  // rows: fewer than 2^32 lanes a launch
+  for (size_t r = 0; r < rows; r += kMost) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(rows - r, kMost)), dim3(kSoftmaxBlock), 0, stream,
+                       scores + r * cols, probs + r * cols, (long long)cols, scale);
+    const int rc = tqh::check_launch("softmax_rows_kernel");
+    if (rc) return rc;
+  }
+  return TQ_OK;
 }
 
 extern "C" size_t tq_qjl_weighted_values_workspace_size(size_t num_queries, size_t num_values, int dim) {

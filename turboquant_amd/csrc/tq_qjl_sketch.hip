@@ -310,7 +310,8 @@ int sketch_args(SketchArgs &a, tqh::PolarCodec &codec, const void *k, int k_dtyp
   if (a.nq && (!q || !rq || !tqh::valid_dtype(q_dtype)))
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "query projection needs q (f32/bf16/f16) and rq");
   const long long key_blocks = (a.nvec + kVecs - 1) / kVecs, blocks = key_blocks + (a.nq + kVecs - 1) / kVecs;
-  if (blocks > 0x7fffffffll) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many vectors in one call");
+  if (blocks * 2 * head_dim >= 1ll << 32)  // a launch holds fewer than 2^32 lanes
+    return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many vectors in one call");
   a.k = k;
   a.rbits = sign_matrix;
   a.signs = reinterpret_cast<uint32_t *>(signs);
@@ -403,6 +404,7 @@ extern "C" int tq_qjl_project(const void *q, int q_dtype, const uint32_t *sign_m
   if (num_rows == 0) return TQ_OK;
   if (!q || !sign_matrix || !rq) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
   const long long n = (long long)num_rows;
+  if ((n + kVecs - 1) / kVecs * 2 * dim >= 1ll << 32) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many rows in one call");
   return by_cache_dim(dim, [&](auto d) {
     constexpr int D = decltype(d)::value;
     hipLaunchKernelGGL((qjl_project_kernel<D>), dim3((unsigned)((n + kVecs - 1) / kVecs)), dim3(Geo<D>::THREADS), 0,
