@@ -1,8 +1,8 @@
 """Staged prefill tiles whose waves work in pairs, each pair on 32 rows and
 each wave of it on half of every tile: halves that no row sees (sequences and
 causal rows that end in a tile's first half), ragged last rows of a pair, and
-rows whose two halves hold very different maxima, against the oracle in
-double.  Tolerance 1e-3 max-abs, as for every prefill (fp32 accumulation, f16
+rows whose two halves hold very different maxima, and the shorter walks that
+waves take one group each, against the oracle in double.  Tolerance 1e-3 max-abs, as for every prefill (fp32 accumulation, f16
 two-part operands)."""
 import math
 
@@ -23,13 +23,22 @@ def _dev(a):
 
 
 @pytest.mark.parametrize("bits,outlier,hq,hkv,ql,t,causal,peak,splits", [
-    (3, orc.OUTLIER_ALL, 2, 1, 1, 768 + 20, True, None, 1),     # nothing in the last tile's second half
-    (4, orc.OUTLIER_ALL, 4, 1, 9, 704 + 32, False, None, 1),    # 12 tiles, the last one's second half is empty
-    (4, 0, 4, 1, 9, 704, False, None, 1),                       # 11 tiles: one group per wave
-    (3, 0, 2, 2, 707, 707, True, None, 1),                      # causal rows that see one half only; ragged rows
-    (4, 0, 1, 1, 130, 1601, True, None, 2),                     # two splits of 13 tiles, one row of a second workgroup
-    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 5, 1),           # the maximum in a first half
-    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 64 + 40, 1),     # and in a second half
+    # walks of at least 24 tiles: pairs
+    (3, orc.OUTLIER_ALL, 2, 1, 1, 1536 + 20, True, None, 1),    # nothing in the last tile's second half
+    (4, orc.OUTLIER_ALL, 4, 1, 9, 1472 + 32, False, None, 1),   # 24 tiles, the last one's second half is empty
+    (3, 0, 2, 2, 1475, 1475, True, None, 1),                    # causal rows that see one half only; ragged rows
+    (4, 0, 1, 1, 130, 3073, True, None, 2),                     # two splits of 25 tiles, one row of a second workgroup
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 1568, False, 5, 1),          # the maximum in a first half
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 1568, False, 64 + 40, 1),    # and in a second half
+    # shorter walks: one group per wave
+    (4, 0, 4, 1, 9, 1472, False, None, 1),                      # 23 tiles
+    (3, orc.OUTLIER_ALL, 2, 1, 1, 768 + 20, True, None, 1),
+    (4, orc.OUTLIER_ALL, 4, 1, 9, 704 + 32, False, None, 1),
+    (4, 0, 4, 1, 9, 704, False, None, 1),
+    (3, 0, 2, 2, 707, 707, True, None, 1),
+    (4, 0, 1, 1, 130, 1601, True, None, 2),
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 5, 1),
+    (3, orc.OUTLIER_ALL, 1, 1, 65, 800, False, 64 + 40, 1),
 ])
 @pytest.mark.parametrize("qdt", ["bf16", "f32"])
 def test_staged_row_pairs(monkeypatch, bits, outlier, hq, hkv, ql, t, causal, peak, splits, qdt):

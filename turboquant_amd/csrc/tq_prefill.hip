@@ -98,11 +98,15 @@ constexpr int kORow = 128 + 4;  // floats
 constexpr int kStagingMinQueryBlocks = 6;
 // Staged PQO and PQ tiles are taken by pairs of waves where the longest
 // workgroup walks at least this many: a pair saves half of a tile's LDS reads
-// and pays once for the second group's operands and the exchange of the
-// halves (one group per wave vs pairs, us: 64 tiles, 4096 x 4096 causal, 16 / 8
-// heads 198 vs 187; 32 tiles, 2048 x 2048 94.0 vs 90.7; 8 tiles, 1024 x 1024
-// 52.9 vs 53.7; 6 tiles, 768 x 768 42.8 vs 43.8)
-constexpr int kPairMinTiles = 12;
+// and pays about 1 us once for the second group's operands and the exchange
+// of the halves (one group per wave vs pairs, us, 16 heads over 8 unless
+// said: 64 tiles, 4096 x 4096 causal, 198 vs 187; 32 tiles, 2048 x 2048, 93.2
+// vs 92.3 and, 32 over 8, 1024 x 2000, 95.5 vs 93.4; 24 tiles, 1536 x 1536,
+// 74.0 vs 74.1 and, 32 over 8, 512 x 3000, 93.0 vs 91.6; 20 tiles, 1280 x
+// 1280, 64.2 vs 64.6; 16 tiles, 1024 x 2000, 71.7 vs 72.5; 12 tiles, 512 x
+// 3000, 58.7 vs 59.1; 8 tiles, 1024 x 1024, 53.5 vs 54.5; 6 tiles, 768 x 768,
+// 43.6 vs 44.5)
+constexpr int kPairMinTiles = 24;
 constexpr int kStagingMinTokens = 768;
 // A staged tile image: the tile buffer's K rows and V planes, then its
 // exponent words (the slices' K exponents, the waves' V exponents), for a TQ
