@@ -42,32 +42,15 @@ struct Geo {
   static constexpr int LPV = D / E;  // lanes per vector
 };
 
-// #{t : U[t] <= x} for the 2^BITS - 1 ascending thresholds U: a binary search
-// whose probe at each level is picked from the candidates by the decisions
-// already made (a select tree), BITS compares per element instead of
-// 2^BITS - 1.
+// #{t : U[t] <= x} for the 2^BITS - 1 ascending thresholds U (bucket_bits).
 template <int BITS>
 __device__ __forceinline__ uint32_t bucket_sorted(float x, const float (&U)[(1 << BITS) - 1]) {
-  if constexpr (BITS == 2) {
-    const bool b1 = x >= U[1];
-    const bool b0 = x >= (b1 ? U[2] : U[0]);
-    return (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
-  } else if constexpr (BITS == 3) {
-    const bool b2 = x >= U[3];
-    const bool b1 = x >= (b2 ? U[5] : U[1]);
-    const float lo = b1 ? U[2] : U[0], hi = b1 ? U[6] : U[4];
-    const bool b0 = x >= (b2 ? hi : lo);
-    return (b2 ? 4u : 0u) | (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
-  } else {
-    const bool b3 = x >= U[7];
-    const bool b2 = x >= (b3 ? U[11] : U[3]);
-    const float l1 = b2 ? U[5] : U[1], h1 = b2 ? U[13] : U[9];
-    const bool b1 = x >= (b3 ? h1 : l1);
-    const float a0 = b1 ? U[2] : U[0], a1 = b1 ? U[6] : U[4], a2 = b1 ? U[10] : U[8], a3 = b1 ? U[14] : U[12];
-    const float l0 = b2 ? a1 : a0, h0 = b2 ? a3 : a2;
-    const bool b0 = x >= (b3 ? h0 : l0);
-    return (b3 ? 8u : 0u) | (b2 ? 4u : 0u) | (b1 ? 2u : 0u) | (b0 ? 1u : 0u);
-  }
+  bool bit[BITS];
+  bucket_bits<BITS>(x, U, bit);
+  uint32_t code = 0;
+#pragma unroll
+  for (int t = 0; t < BITS; t++) code |= bit[t] ? 1u << (BITS - 1 - t) : 0u;
+  return code;
 }
 
 // Value of the lane before, inside rows of 16 (DPP row_shr:1).

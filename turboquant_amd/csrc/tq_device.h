@@ -126,4 +126,30 @@ __device__ __forceinline__ uint32_t field(const uint32_t (&w)[NW], int i) {
   return ((w[wi] >> sh) | (w[wi + 1] << (32 - sh))) & ((1u << BITS) - 1u);
 }
 
+// The code bits of x, most significant first, of #{t : U[t] <= x} for the
+// 2^BITS - 1 ascending thresholds U: a binary search whose probe at each
+// level is picked from the candidates by the decisions already made (a
+// select tree), BITS compares per element instead of 2^BITS - 1.
+template <int BITS>
+__device__ __forceinline__ void bucket_bits(float x, const float (&U)[(1 << BITS) - 1], bool (&bit)[BITS]) {
+  if constexpr (BITS == 2) {
+    bit[0] = x >= U[1];
+    bit[1] = x >= (bit[0] ? U[2] : U[0]);
+  } else if constexpr (BITS == 3) {
+    bit[0] = x >= U[3];
+    bit[1] = x >= (bit[0] ? U[5] : U[1]);
+    const float lo = bit[1] ? U[2] : U[0], hi = bit[1] ? U[6] : U[4];
+    bit[2] = x >= (bit[0] ? hi : lo);
+  } else {
+    bit[0] = x >= U[7];
+    bit[1] = x >= (bit[0] ? U[11] : U[3]);
+    const float l1 = bit[1] ? U[5] : U[1], h1 = bit[1] ? U[13] : U[9];
+    bit[2] = x >= (bit[0] ? h1 : l1);
+    const float a0 = bit[2] ? U[2] : U[0], a1 = bit[2] ? U[6] : U[4], a2 = bit[2] ? U[10] : U[8],
+                a3 = bit[2] ? U[14] : U[12];
+    const float l0 = bit[1] ? a1 : a0, h0 = bit[1] ? a3 : a2;
+    bit[3] = x >= (bit[0] ? h0 : l0);
+  }
+}
+
 }  // namespace tqd

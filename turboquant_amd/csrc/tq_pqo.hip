@@ -260,7 +260,6 @@ int launch_polar_quant(const void *x, int dt, uint8_t *packed, uint16_t *scales,
                        const tqh::PolarCodec &codec, const CacheMap &m, const Second &second, hipStream_t st) {
   auto run = [&](const tqh::PqoCodebook &cb, int cb_bits, long long b0, long long n) {
     QuantConsts k = make_quant_consts(cb, codec.outer, codec.scale_sign);
-    k.mixed_sign = codec.mixed ? 1 : 0;
     k.nb = codec.num_blocks;
     k.eo = codec.eo;
     k.blk0 = b0;
