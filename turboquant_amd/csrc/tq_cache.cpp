@@ -9,11 +9,14 @@
 // record h * capacity + t, exactly what the fused kernels read with
 // kv_head_stride = capacity; a TqCache adds signs [num_kv_heads][capacity]
 // [head_dim/8] u8 and residual norms [num_kv_heads][capacity] f16 at the
-// same records.  Appends quantize straight into their records (one launch
-// per tensor, all heads at once; a TqCache then sketches the new keys);
-// growth reallocates to needed + max(needed / 4, 128) and copies the old rows
-// (storage.rs:108-139, tq.rs:64-94).  Decode runs the single-launch fused
-// attention over the stored records.
+// same records.  An append quantizes keys and values of all heads straight
+// into their records in one launch, which sketches a TqCache's new keys too
+// (and projects the queries of a decode that follows); growth reallocates to
+// needed + max(needed / 4, 128) and fills the new buffers in one launch, old
+// rows copied and the rest zero (storage.rs:108-139, tq.rs:64-94).  Decode
+// runs the fused attention over the stored records and stores its own token
+// in the same launch, or, in the shapes where that launch cannot
+// (store_token_apart), in one launch ahead of it that forms R q as well.
 #include "tq_common.h"
 
 #include <cstring>

@@ -9,16 +9,18 @@
 //
 // What bounds it: the output (2 or 4 bytes per row and token against 128
 // useful multiply-adds), so the product has to stay below the store rate.
-// One workgroup makes 64 rows x 512 tokens: the rows are staged once in LDS
-// as two f16 parts (hi = x rounded to f16, lo = the rest rounded to f16, 22
-// to 23 significant bits together, on a power-of-two scale per row), each of
-// its 8 waves expands the sign bits of its 64 tokens once into registers
-// (f16 +-1) and keeps them for all rows.  Both part products are exact in
-// the f32 accumulator.  A lane holds 4 tokens that follow each other for
-// each of its rows, so a wave's store is 128 bytes (16-bit outputs) per row;
-// rows of a kv_len that is no multiple of 4 are stored unaligned (513 x 1537
-// 17.9 us, x 1536 13.3 us, 16 heads).  512 tokens a workgroup instead of 256
-// halve the projection's work per row: 25.2 -> 16.1 us at 16 x 1024 x 1024.
+// One workgroup makes 64 rows x 512 tokens (x 128 tokens where the grid would
+// be small; one to four positions of given rows are sums of table entries
+// instead, both below): the rows are staged once in LDS as two f16 parts (hi =
+// x rounded to f16, lo = the rest rounded to f16, 22 to 23 significant bits
+// together, on a power-of-two scale per row), each of its 8 waves expands the
+// sign bits of its 64 tokens once into registers (f16 +-1) and keeps them for
+// all rows.  Both part products are exact in the f32 accumulator.  A lane
+// holds 4 tokens that follow each other for each of its rows, so a wave's
+// store is 128 bytes (16-bit outputs) per row; rows of a kv_len that is no
+// multiple of 4 are stored unaligned (513 x 1537 17.9 us, x 1536 13.3 us, 16
+// heads).  512 tokens a workgroup instead of 256 halve the projection's work
+// per row: 25.2 -> 16.1 us at 16 x 1024 x 1024.
 //
 // Mean of 16 heads x 1024 x 1024 and 16 x 513 x 1537 over 8 KV heads, d =
 // 128, bf16: 49.2 us with one lane per token adding LDS table entries, plus
@@ -330,11 +332,10 @@ constexpr long long kTableValues = 1 << 20;
 // At d = 256 five waves a SIMD at most: registers for more LDS reads in flight
 // (eight waves: 1,000 tokens 4.6 us against 3.5).
 template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 256 ? 5 : 8))) void qjl_logit_bias_table_kernel(const float *__restrict__ rq, int q_len,
-                                                                   const uint32_t *__restrict__ signs,
-                                                                   const uint16_t *__restrict__ norms, int kv_len,
-                                                                   long long head_stride, int n_rep, float sf,
-                                                                   void *__restrict__ out, int out_dtype) {
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(1, D == 256 ? 5 : 8))) void qjl_logit_bias_table_kernel(
+    const float *__restrict__ rq, int q_len, const uint32_t *__restrict__ signs, const uint16_t *__restrict__ norms,
+    int kv_len, long long head_stride, int n_rep, float sf, void *__restrict__ out, int out_dtype) {
   constexpr int CT = (D / 4) * 16;
   __shared__ float s_tab[kTablePositions<D> * CT];
   const int h = blockIdx.z;
@@ -386,7 +387,9 @@ int launch_bias(BiasArgs &a, int source, int out_dtype, hipStream_t st) {
   if (source == kFromBF16) return launch_one<D, kFromBF16, kBF16>(a, st);
   if (source == kFromF16) return launch_one<D, kFromF16, kF16>(a, st);
   const int n_rep = a.q_heads / a.kv_heads, q_len = a.rows / n_rep;
-  if (q_len <= (a.kv_len >= 16384 ? kTablePositions<D> : 2) && (long long)a.rows * a.kv_heads * a.kv_len <= kTableValues) {
+  // (grid.z counts query heads here, KV heads in the products)
+  if (q_len <= (a.kv_len >= 16384 ? kTablePositions<D> : 2) && a.q_heads <= 65535 &&
+      (long long)a.rows * a.kv_heads * a.kv_len <= kTableValues) {
     hipLaunchKernelGGL((qjl_logit_bias_table_kernel<D>), dim3((unsigned)((a.kv_len + 255) / 256), 1, (unsigned)a.q_heads),
                        dim3(256), 0, st, static_cast<const float *>(a.src), q_len, a.signs, a.norms, a.kv_len,
                        a.head_stride, n_rep, a.sf, a.out, out_dtype);
