@@ -247,8 +247,9 @@ __global__ __launch_bounds__(kBlock) void qjl_query_kernel(const float *__restri
 // registers.  A slice's centroids are byte permutes: 4 codes as the selector
 // bytes, tables of the parts' low and high bytes in registers.
 // 64 queries x 8,192 keys, d = 128, 3 bits: 18 us with a lane per key adding LDS
-// table entries (96 a score), 7.4 us now (7.5 with two parts and the queries
-// staged in LDS for four waves).
+// table entries (96 a score), 7.5 us in two parts with the queries staged in LDS
+// for four waves, 7.4 in three parts and registers, 6.4 with a wave walking
+// several key tiles (below).
 constexpr int kCentExp = 8;
 // The workgroups of a launch: one per compute unit, whose waves then walk
 // several key tiles for one split of their queries, and two, as many as the
