@@ -184,6 +184,19 @@ def test_pack_indices(tq, bits):
         assert np.array_equal(out.cpu().numpy(), ref)
 
 
+def test_pack_indices_past_one_launch(tq):
+    """2^26 + 1 blocks of 64 bytes out, a lane a byte: a launch holds fewer than 2^32 lanes."""
+    n, bs = 2**26 + 1, 128
+    row = np.random.default_rng(15).integers(0, 16, size=bs, dtype=np.uint8)
+    idx = torch.zeros((n, bs), dtype=torch.uint8, device="cuda")
+    for i in (0, 2**25, n - 1):
+        idx[i] = _dev(row)
+    out = tq.pack_indices(idx, 4)
+    ref = orc.pack_indices(4, row)
+    for i in (0, 2**25, n - 1):
+        assert np.array_equal(out[i].cpu().numpy(), ref)
+
+
 def test_pqo_roundtrip_cosine_reference_gates(tq):
     """cache_pqo_tests.rs:151-244 gates on the reference's sin/cos K/V."""
     k, _ = sincos_kv(8, 5, 128, 5.0)

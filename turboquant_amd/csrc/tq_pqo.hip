@@ -450,10 +450,16 @@ extern "C" int tq_pack_indices(const uint8_t *indices, uint8_t *packed_out, int 
   if (bytes_per_block * 8 < block_size * bits)
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "bytes_per_block %d too small", bytes_per_block);
   if (!indices || !packed_out) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "null pointer");
-  const long long total = (long long)num_vectors * bytes_per_block;
-  hipLaunchKernelGGL(pack_indices_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, indices,
-                     packed_out, (long long)num_vectors, block_size, bits, bytes_per_block);
-  return tqh::check_launch("pack_indices_kernel");
+  // whole vectors a launch, fewer than 2^32 lanes (bytes_per_block is an int)
+  const long long most = std::max((1ll << 31) / bytes_per_block, 1ll);
+  for (long long v = 0; v < num_vectors; v += most) {
+    const long long n = std::min(num_vectors - v, most);
+    hipLaunchKernelGGL(pack_indices_kernel, dim3((unsigned)((n * bytes_per_block + 255) / 256)), dim3(256), 0, stream,
+                       indices + v * block_size, packed_out + v * bytes_per_block, n, block_size, bits, bytes_per_block);
+    const int rc = tqh::check_launch("pack_indices_kernel");
+    if (rc) return rc;
+  }
+  return TQ_OK;
 }
 
 // ---------------------------------------------------------------------------
