@@ -24,7 +24,7 @@ def _x(dim, n):
     return x
 
 
-@pytest.mark.parametrize("n", [1, 2, 7, 33, 65, 256, 257, 323])
+@pytest.mark.parametrize("n", [1, 2, 7, 16, 17, 32, 33, 64, 65, 128, 129, 256, 257, 323])
 @pytest.mark.parametrize("dim,bits", [(32, 2), (64, 3), (128, 4), (256, 3)])
 def test_core_codec_batch_edges(tq, dim, bits, n):
     x = _x(dim, n)

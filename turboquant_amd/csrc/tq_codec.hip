@@ -31,10 +31,11 @@ __global__ __launch_bounds__(kBlock) void codec_quant_kernel(const float *__rest
   if (q == 0) scales[v] = f32_to_f16(norm < kMinNorm ? 0.0f : norm);  // select_scale, quantize.rs:123-126
 }
 
-// Batches that are latency alone store from the registers: the staging would
-// only lengthen them (100 vectors of 32 2.95 us staged, 2.75 direct; 1,000 3.3
-// staged, 3.6 direct).
-constexpr long long kDirectVectors = 256;
+// Batches of up to two waves, latency alone, store from the registers: the
+// staging would only lengthen them (us, staged / direct: 100 vectors of 32 2.95
+// / 2.77, 200 3.10 / 3.30; 64 of 64 3.12 / 2.95, 100 3.32 / 3.44; 32 of 128 3.21 /
+// 3.16, 64 3.39 / 3.73; 8 of 256 3.52 / 3.38, 24 3.55 / 3.90).
+constexpr long long kDirectLanes = 128;
 
 // dequantize_vec (quantize.rs:225-240) or, ROTATE = false, dequantize_rotated
 // (quantize.rs:306-316).  A wave's 64 lanes make one run of 8 KB: staged
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(kBlock) void codec_dequant_kernel(const uint8_t *__
   }
   float w[32];
   dequant_lanes<LPV, BITS, ROTATE>(pk, sc, q, s_cent, k, w);
-  if (n <= kDirectVectors) {
+  if (n * LPV <= kDirectLanes) {
     if (v < n) {
       float4 *o = reinterpret_cast<float4 *>(out + t * 32);
 #pragma unroll
