@@ -67,6 +67,23 @@ def test_sign_matrix_and_projection_bit_exact(tq):
     assert (rq.view(np.uint32) == ref.view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("n", [1, 15, 17, 8192, 8193])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_projection_of_every_row_bit_exact(tq, d, n, dtype):
+    """One and two row tiles a wave (up to 8,192 rows and more), ragged last workgroups, rows from an odd element on."""
+    rng = np.random.default_rng(d + n)
+    pool = torch.from_numpy(rng.standard_normal((17, d)).astype(np.float32)).to(
+        {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype])
+    ref = np.stack([orc.query_projections(r, 12345) for r in pool.float().numpy()])
+    pick = np.arange(n) % 17
+    buf = torch.empty(n * d + 1, dtype=pool.dtype, device="cuda")
+    q = buf[1:].view(n, d)
+    q.copy_(pool.cuda()[torch.from_numpy(pick).cuda()])
+    rq = _host(tq.qjl_project(q, tq.qjl_sign_matrix(d, 12345)))
+    assert (rq.view(np.uint32) == ref[pick].view(np.uint32)).all()
+
+
 def _tq_cache_ref(k_np, bits):
     """Oracle codes, dequantized K and the keys' (signs, norms) for K [H, T, D]."""
     h, t, _ = k_np.shape

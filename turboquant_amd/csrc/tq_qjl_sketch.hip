@@ -15,11 +15,12 @@
 // A workgroup takes 16 vectors: lane = qblock quantizes (keys in the first
 // lanes, values in the next), the key lanes decode their codes again and
 // leave the residual in LDS, then wave w sums rows 32 w .. + 31 of R for all
-// 16 (two chains, so neither waits for its own last step).  Bound by the
-// chains: D / 4 steps of 32 cycles for two tiles each, 0.9 us at D = 128;
-// launches bound a short append (prefill, extension, a decode whose token the
-// attention launch does not store), which took three (keys, values, sketch
-// with projection: two of 3.8 us and one of 4.0 us, 16 tokens) and takes one.
+// 16 (two chains, so neither waits for its own last step; a projection of few
+// rows by itself gives each wave one).  Bound by the chains: D / 4 steps of 32
+// cycles for two tiles each, 0.9 us at D = 128; launches bound a short append
+// (prefill, extension, a decode whose token the attention launch does not
+// store), which took three (keys, values, sketch with projection: two of 3.8
+// us and one of 4.0 us, 16 tokens) and takes one.
 #include "tq_pqo_dev.h"
 
 #include <type_traits>
@@ -38,24 +39,24 @@ struct Geo {
   static constexpr int RS = D + 4;  // floats per staged row: the chain's reads hit 64 banks
 };
 
-// Sign words of R's rows 32 wave + 16 t + l16, shifted so that column
+// Sign words of R's rows 16 (T wave + t) + l16, shifted so that column
 // 4 k + lg of word w is bit 4 k.
-template <int D>
+template <int D, int T>
 __device__ __forceinline__ void load_rows(const uint32_t *__restrict__ rbits, int wave, int l16, int lg,
-                                          uint32_t (&rb)[2][Geo<D>::NW]) {
+                                          uint32_t (&rb)[T][Geo<D>::NW]) {
 #pragma unroll
-  for (int t = 0; t < 2; t++)
+  for (int t = 0; t < T; t++)
 #pragma unroll
-    for (int w = 0; w < Geo<D>::NW; w++) rb[t][w] = rbits[(32 * wave + 16 * t + l16) * Geo<D>::NW + w] >> lg;
+    for (int w = 0; w < Geo<D>::NW; w++) rb[t][w] = rbits[(16 * (T * wave + t) + l16) * Geo<D>::NW + w] >> lg;
 }
 
-// acc[t][i] = sum_c R[32 wave + 16 t + 4 lg + i][c] v[l16][c] (R = +-1), in
+// acc[t][i] = sum_c R[16 (T wave + t) + 4 lg + i][c] v[l16][c] (R = +-1), in
 // column order from -0.0, for the 16 vectors staged in LDS.
-template <int D>
-__device__ __forceinline__ void row_products(const float *s_v, const uint32_t (&rb)[2][Geo<D>::NW], int l16, int lg,
-                                             f32x4 (&acc)[2]) {
+template <int D, int T>
+__device__ __forceinline__ void row_products(const float *s_v, const uint32_t (&rb)[T][Geo<D>::NW], int l16, int lg,
+                                             f32x4 (&acc)[T]) {
 #pragma unroll
-  for (int t = 0; t < 2; t++) acc[t] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
+  for (int t = 0; t < T; t++) acc[t] = f32x4{-0.0f, -0.0f, -0.0f, -0.0f};
   const float *v = s_v + l16 * Geo<D>::RS + lg;
 #pragma unroll
   for (int w = 0; w < Geo<D>::NW; w++) {
@@ -65,7 +66,7 @@ __device__ __forceinline__ void row_products(const float *s_v, const uint32_t (&
 #pragma unroll
     for (int k = 0; k < 8; k++)
 #pragma unroll
-      for (int t = 0; t < 2; t++) {
+      for (int t = 0; t < T; t++) {
         const float a = u2f(((rb[t][w] << (31 - 4 * k)) & 0x80000000u) | 0x3f800000u);
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x[k], acc[t], 0, 0, 0);
       }
@@ -80,37 +81,37 @@ __device__ __forceinline__ float load_elem(const void *p, long long i, int dtype
 
 // rq = R q for query rows row0 .. + 15 (precompute_query_projections,
 // qjl.rs:488-492; r_q = q R^T of tq.rs:233-234).
-template <int D>
+template <int D, int T>
 __device__ __forceinline__ void project_rows(const void *q, int q_dtype, float *rq, long long row0, long long nq,
-                                             float inv, float *s_v, const uint32_t (&rb)[2][Geo<D>::NW], int tid,
+                                             float inv, float *s_v, const uint32_t (&rb)[T][Geo<D>::NW], int tid,
                                              int wave, int l16, int lg) {
-  // a thread's 8 elements by one or two loads, from any element boundary (one
-  // element a load, one after the other: 16 bf16 rows of d = 64 3.7 us, 2.6 now)
-  static_assert(8 * Geo<D>::THREADS == kVecs * D, "8 elements a thread");
-  const int r = 8 * tid / D, e = 8 * tid % D;
-  float x[8] = {};
+  // a thread's 4 T elements by one or two loads, from any element boundary (one
+  // element a load, one after the other: 16 bf16 rows of d = 64 3.7 us, 2.6 so)
+  constexpr int E = 4 * T;
+  const int r = E * tid / D, e = E * tid % D;
+  float x[E] = {};
   if (row0 + r < nq) {
-    const long long i = row0 * D + 8 * tid;
+    const long long i = row0 * D + E * tid;
     if (q_dtype == kF32) {
-      __builtin_memcpy(x, static_cast<const float *>(q) + i, 32);
+      __builtin_memcpy(x, static_cast<const float *>(q) + i, 4 * E);
     } else {
-      uint16_t h[8];
-      __builtin_memcpy(h, static_cast<const uint16_t *>(q) + i, 16);
+      uint16_t h[E];
+      __builtin_memcpy(h, static_cast<const uint16_t *>(q) + i, 2 * E);
 #pragma unroll
-      for (int j = 0; j < 8; j++) x[j] = q_dtype == kBF16 ? bf16_to_f32(h[j]) : f16_to_f32(h[j]);
+      for (int j = 0; j < E; j++) x[j] = q_dtype == kBF16 ? bf16_to_f32(h[j]) : f16_to_f32(h[j]);
     }
   }
   float4 *dst = reinterpret_cast<float4 *>(s_v + r * Geo<D>::RS + e);
-  dst[0] = make_float4(x[0], x[1], x[2], x[3]);
-  dst[1] = make_float4(x[4], x[5], x[6], x[7]);
+#pragma unroll
+  for (int j = 0; j < T; j++) dst[j] = make_float4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]);
   __syncthreads();
-  f32x4 acc[2];
+  f32x4 acc[T];
   row_products<D>(s_v, rb, l16, lg, acc);
   if (row0 + l16 >= nq) return;
 #pragma unroll
-  for (int t = 0; t < 2; t++)
+  for (int t = 0; t < T; t++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) rq[(row0 + l16) * D + 32 * wave + 16 * t + 4 * lg + i] = acc[t][i] * inv;
+    for (int i = 0; i < 4; i++) rq[(row0 + l16) * D + 16 * (T * wave + t) + 4 * lg + i] = acc[t][i] * inv;
 }
 
 struct SketchArgs {
@@ -243,14 +244,19 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void qjl_sketch_kernel(SketchArgs 
   if (lg == 0 && vec0 + l16 < a.nvec) a.signs[record(vec0 + l16) * G::NW + wave] = bits;
 }
 
-template <int D>
-__global__ __launch_bounds__(Geo<D>::THREADS) void qjl_project_kernel(const void *__restrict__ q, int q_dtype,
-                                                                      const uint32_t *__restrict__ rbits,
-                                                                      float *__restrict__ rq, long long nrows,
-                                                                      float inv) {
+// T tiles of 16 rows of R a wave.  Up to kFewRows query rows the grid is small
+// and a wave's chain is what it takes: one tile (us, two / one: d = 64, 100 rows
+// 2.86 / 2.54, 4,000 3.04 / 2.69, 16,384 4.13 / 4.10; d = 128 3.73 / 3.36, 4.10 /
+// 3.75, 8.81 / 8.66); more rows are bound by the staged vectors' reads, which two
+// tiles share (131,072 rows, f32, d = 128 45.7 / 48.7, d = 256 162.5 / 173.9).
+constexpr long long kFewRows = 8192;
+template <int D, int T>
+__global__ __launch_bounds__(4 * D / T) void qjl_project_kernel(const void *__restrict__ q, int q_dtype,
+                                                                const uint32_t *__restrict__ rbits,
+                                                                float *__restrict__ rq, long long nrows, float inv) {
   __shared__ __attribute__((aligned(16))) float s_v[kVecs * Geo<D>::RS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  uint32_t rb[2][Geo<D>::NW];
+  uint32_t rb[T][Geo<D>::NW];
   load_rows<D>(rbits, wave, lane & 15, lane >> 4, rb);
   project_rows<D>(q, q_dtype, rq, (long long)blockIdx.x * kVecs, nrows, inv, s_v, rb, tid, wave, lane & 15, lane >> 4);
 }
@@ -407,8 +413,12 @@ extern "C" int tq_qjl_project(const void *q, int q_dtype, const uint32_t *sign_m
   if ((n + kVecs - 1) / kVecs * 2 * dim >= 1ll << 32) return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many rows in one call");
   return by_cache_dim(dim, [&](auto d) {
     constexpr int D = decltype(d)::value;
-    hipLaunchKernelGGL((qjl_project_kernel<D>), dim3((unsigned)((n + kVecs - 1) / kVecs)), dim3(Geo<D>::THREADS), 0,
-                       stream, q, q_dtype, sign_matrix, rq, n, tqh::inv_sqrt_dim(dim));
+    const dim3 grid((unsigned)((n + kVecs - 1) / kVecs));
+    const float inv = tqh::inv_sqrt_dim(dim);
+    if (n <= kFewRows)
+      hipLaunchKernelGGL((qjl_project_kernel<D, 1>), grid, dim3(4 * D), 0, stream, q, q_dtype, sign_matrix, rq, n, inv);
+    else
+      hipLaunchKernelGGL((qjl_project_kernel<D, 2>), grid, dim3(2 * D), 0, stream, q, q_dtype, sign_matrix, rq, n, inv);
     return tqh::check_launch("qjl_project_kernel");
   });
 }
