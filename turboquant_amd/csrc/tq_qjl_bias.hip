@@ -44,6 +44,11 @@ constexpr int kRows = 64, kThreads = 512;
 // 5.8 / 4.0; at 128 workgroups, 16 x 8,000, d = 64 4.6 / 4.3, at 256, 40 x 8,000,
 // 6.7 / 8.3).
 constexpr int kFewBlocks = 128;
+// And 16 rows a workgroup instead of 64 while there is at most one for every
+// compute unit: a row tile a wave instead of four (us, 64 / 16 rows: 64 rows of one KV
+// head x 1,000 tokens d = 64 3.75 / 2.94, d = 256 6.76 / 4.66; in 512 workgroups of
+// 16 rows, 16 heads x 100 positions on 8 x 1,000 tokens, d = 256 7.8 / 10.2).
+constexpr int kFewRowBlocks = 256;
 
 // Where the staged rows come from: rq as given (f32), or R q of bf16, f16 or
 // f32 query rows.
@@ -60,7 +65,7 @@ struct BiasArgs {
   long long head_stride;
   float sf;
   void *out;
-  int token_blocks, kv_heads, q_heads;
+  int token_blocks, kv_heads, q_heads, block_rows;
 };
 
 // Four values as consecutive elements of type OUT.  Rows of kv_len elements
@@ -94,7 +99,7 @@ __global__ __launch_bounds__(kThreads, D == 256 && TT == 4 ? 2 : 4) void qjl_log
   const int l16 = lane & 15, lg = lane >> 4;
   const int g = blockIdx.z;
   const int rblk = (int)(blockIdx.x / (unsigned)a.token_blocks), tblk = (int)(blockIdx.x % (unsigned)a.token_blocks);
-  const int r0 = rblk * kRows, nrows = min(kRows, a.rows - r0);
+  const int block = TT == 1 ? a.block_rows : kRows, r0 = rblk * block, nrows = min(block, a.rows - r0);
   const long long row0 = (long long)g * a.rows + r0;
 
   // the wave's tokens: column l16 of tile T is token t0 + TT l16 + T
@@ -371,7 +376,7 @@ __attribute__((amdgpu_waves_per_eu(1, D == 256 ? 5 : 8))) void qjl_logit_bias_ta
 template <int D, int SRC, int OUT, int TT = 4>
 int launch_one(BiasArgs &a, hipStream_t st) {
   constexpr int TOKENS = kThreads / 64 * 16 * TT;
-  const long long tblocks = ((long long)a.kv_len + TOKENS - 1) / TOKENS, rblocks = ((long long)a.rows + kRows - 1) / kRows;
+  const long long tblocks = ((long long)a.kv_len + TOKENS - 1) / TOKENS, rblocks = ((long long)a.rows + a.block_rows - 1) / a.block_rows;
   if (tblocks * rblocks > 0x7fffffffll)
     return tqh::fail(TQ_ERR_INVALID_ARGUMENT, "too many query rows (%d) for %d tokens", a.rows, a.kv_len);
   a.token_blocks = (int)tblocks;
@@ -397,6 +402,7 @@ int launch_bias(BiasArgs &a, int source, int out_dtype, hipStream_t st) {
   }
   const long long blocks = (long long)((a.kv_len + kThreads - 1) / kThreads) * ((a.rows + kRows - 1) / kRows) * a.kv_heads;
   if (blocks <= kFewBlocks) {
+    if ((long long)((a.kv_len + 127) / 128) * ((a.rows + 15) / 16) * a.kv_heads <= kFewRowBlocks) a.block_rows = 16;
     if (out_dtype == kF32) return launch_one<D, kGiven, kF32, 1>(a, st);
     if (out_dtype == kBF16) return launch_one<D, kGiven, kBF16, 1>(a, st);
     return launch_one<D, kGiven, kF16, 1>(a, st);
@@ -434,6 +440,7 @@ int bias(const void *src, int source, const uint32_t *rbits, int num_q_heads, in
   a.out = out;
   a.kv_heads = num_kv_heads;
   a.q_heads = num_q_heads;
+  a.block_rows = kRows;
   if (head_dim == 64) return launch_bias<64>(a, source, out_dtype, stream);
   if (head_dim == 128) return launch_bias<128>(a, source, out_dtype, stream);
   return launch_bias<256>(a, source, out_dtype, stream);
