@@ -40,6 +40,7 @@ def _bias64(rq, signs, norms, d):
     (128, 2, 65, 511, "bf16"), (256, 2, 17, 513, "f32"), (128, 8, 16, 1030, "f16"), (256, 4, 40, 260, "bf16"),
     (64, 4, 2, 257, "f32"), (256, 6, 1, 1025, "bf16"), (64, 64, 1, 16385, "f16"), (256, 2, 4, 16384, "f32"), (64, 2, 300, 6700, "bf16"),
     (128, 4, 3, 129, "f32"), (256, 2, 70, 127, "f16"), (128, 2, 200, 4000, "f32"), (64, 32, 4, 1000, "f32"),
+    (64, 4, 2, 131073, "bf16"), (128, 2, 3, 131075, "f32"), (256, 8, 1, 131072, "f16"), (128, 8, 1, 131073, "f32"),
 ])
 def test_bias_of_given_projections(tq, d, heads, q_len, kv_len, dtype):
     hk = 2

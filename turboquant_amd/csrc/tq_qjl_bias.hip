@@ -330,10 +330,19 @@ __global__ __launch_bounds__(kThreads, D == 256 && TT == 4 ? 2 : 4) void qjl_log
 // 3.0 / 2.8, 32,768 tokens 5.4 / 4.6; d = 256 3.8 / 3.5, 11.5 / 7.4; two
 // positions d = 256 x 32,768 13.1 / 10.7).  Every query head reads the signs
 // again, so more than 2^20 values stay with the products (32 heads, two
-// positions x 32,768, d = 128 6.6 / 9.9).
+// positions x 32,768, d = 128 6.6 / 9.9), unless a KV head has no more than
+// kTableRows rows: a product's cost is its tokens', whatever its rows (8 heads on
+// 8, three positions x 65,536, d = 64 6.7 / 5.2, d = 128 9.1 / 7.6, d = 256 23.8 /
+// 12.9; two x 131,072 10.6 / 6.6, 14.1 / 9.5, 42.8 / 20.1).  At d = 64 and 128 not
+// with four query heads a KV head, which read the signs four times (32 heads on
+// 8 x 65,536 7.0 / 8.3, 9.5 / 11.9; d = 256 24.6 / 19.8), and at d = 128 with four
+// rows from 2^20 tokens on (8 heads, four positions x 32,768 6.0 / 6.4, x 131,072
+// 16.0 / 14.8).
 template <int D>
 constexpr int kTablePositions = D == 256 ? 4 : 2;  // (3 and 4 from 16,384 tokens on: 8 heads x 32,768 13.1 / 9.9)
 constexpr long long kTableValues = 1 << 20;
+constexpr int kTableRows = 4;
+constexpr long long kTableTokens = 1 << 18;  // of all KV heads: 512 workgroups of products
 // At d = 256 five waves a SIMD at most: registers for more LDS reads in flight
 // (eight waves: 1,000 tokens 4.6 us against 3.5).
 template <int D>
@@ -342,7 +351,7 @@ __attribute__((amdgpu_waves_per_eu(1, D == 256 ? 5 : 8))) void qjl_logit_bias_ta
     const float *__restrict__ rq, int q_len, const uint32_t *__restrict__ signs, const uint16_t *__restrict__ norms,
     int kv_len, long long head_stride, int n_rep, float sf, void *__restrict__ out, int out_dtype) {
   constexpr int CT = (D / 4) * 16;
-  __shared__ float s_tab[kTablePositions<D> * CT];
+  __shared__ float s_tab[kTableRows * CT];
   const int h = blockIdx.z;
   for (int e = threadIdx.x; e < q_len * CT; e += 256) {
     const int ql = e / CT, rr = e % CT, c = rr / 16, m = rr % 16;
@@ -392,9 +401,11 @@ int launch_bias(BiasArgs &a, int source, int out_dtype, hipStream_t st) {
   if (source == kFromBF16) return launch_one<D, kFromBF16, kBF16>(a, st);
   if (source == kFromF16) return launch_one<D, kFromF16, kF16>(a, st);
   const int n_rep = a.q_heads / a.kv_heads, q_len = a.rows / n_rep;
+  const long long tokens = (long long)a.kv_heads * a.kv_len;
+  const bool few = q_len <= (a.kv_len >= 16384 ? kTablePositions<D> : 2) && a.rows * tokens <= kTableValues;
   // (grid.z counts query heads here, KV heads in the products)
-  if (q_len <= (a.kv_len >= 16384 ? kTablePositions<D> : 2) && a.q_heads <= 65535 &&
-      (long long)a.rows * a.kv_heads * a.kv_len <= kTableValues) {
+  const int rows = D == 128 && tokens < 4 * kTableTokens ? 3 : kTableRows;
+  if (a.q_heads <= 65535 && (few || (a.rows <= rows && (n_rep <= 2 || D == 256) && tokens >= kTableTokens))) {
     hipLaunchKernelGGL((qjl_logit_bias_table_kernel<D>), dim3((unsigned)((a.kv_len + 255) / 256), 1, (unsigned)a.q_heads),
                        dim3(256), 0, st, static_cast<const float *>(a.src), q_len, a.signs, a.norms, a.kv_len,
                        a.head_stride, n_rep, a.sf, a.out, out_dtype);
