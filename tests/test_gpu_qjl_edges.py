@@ -163,6 +163,26 @@ def test_weighted_values_at_chunk_edges(tq, dim, pb, nv, nq):
     assert np.abs(got - w.astype(np.float64) @ vals).max() <= bound
 
 
+def test_weighted_values_of_more_values_than_one_launch_holds(tq):
+    """2^31 + 1 values of 128: 512 lanes for 256 of them.  All weight is on the first and the last one."""
+    nv, dim = 2**31 + 1, 128
+    if torch.cuda.mem_get_info()[0] < 120 * 2**30:
+        pytest.skip("needs 120 GiB")
+    packed, scales = orc.quantize_vec_batch(2, dim, 42, orc.lcg_normal_vecs(3, dim, 2))
+    codes = torch.zeros((nv, dim // 4), dtype=torch.uint8, device="cuda")
+    sc = torch.zeros((nv,), dtype=torch.int16, device="cuda")
+    w = torch.zeros((1, nv), device="cuda")
+    for i in (0, 1):
+        codes[-i] = _dev(packed[i])
+        sc[-i] = int(scales.view(np.int16)[i])
+        w[0, -i] = 1.0 + i
+    got = tq.qjl_weighted_values(codes, sc, w, 2, dim, 42).cpu().numpy()[0]
+    del codes, sc, w
+    torch.cuda.empty_cache()
+    vals = orc.dequantize_vec_batch(2, dim, 42, packed, scales).astype(np.float64)
+    assert np.abs(got - (vals[0] + 2 * vals[1])).max() <= 1e-5 * np.abs(vals).max()
+
+
 def test_softmax_of_more_rows_than_one_launch_holds(tq):
     x = torch.zeros((2**22 + 1, 3), device="cuda")
     x[-1] = torch.tensor([0.0, 1.0, 2.0])

@@ -581,7 +581,8 @@ __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__
                                                                const uint16_t *__restrict__ polar_scales,
                                                                long long nv, long long nq,
                                                                const float *__restrict__ weights,
-                                                               float *__restrict__ partial, QjlConsts k) {
+                                                               float *__restrict__ partial, int chunk0, int nchunks,
+                                                               QjlConsts k) {
   constexpr int RW = D * PB / 32, THREADS = 4 * D, ST = CHUNK / 4;  // words per value, steps
   constexpr int GS = ST + 4;                                           // [g] stride
   __shared__ __attribute__((aligned(16))) uint32_t s_codes[RW][4 * GS];
@@ -589,7 +590,8 @@ __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__
   __shared__ float s_cent[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
-  const long long t0 = (long long)blockIdx.x * CHUNK, q0 = (long long)blockIdx.y * kWvQueries;
+  const int chunk = chunk0 + (int)blockIdx.x;
+  const long long t0 = (long long)chunk * CHUNK, q0 = (long long)blockIdx.y * kWvQueries;
   const int cnt = (int)min<long long>(CHUNK, nv - t0);
   if (tid < 16) s_cent[tid] = k.polar.cent[tid & ((1 << PB) - 1)];
   // every load goes out before the first is used; places past the end read
@@ -648,7 +650,7 @@ __global__ __launch_bounds__(4 * D) void qjl_wv_partial_kernel(const uint8_t *__
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const long long qi = q0 + 4 * lg + i;
-    if (qi < nq) partial[(qi * gridDim.x + blockIdx.x) * D + 16 * wave + l16] = acc[i];
+    if (qi < nq) partial[(qi * nchunks + chunk) * D + 16 * wave + l16] = acc[i];
   }
 }
 
@@ -901,10 +903,11 @@ extern "C" int tq_qjl_weighted_values(const uint8_t *polar_packed, const uint16_
   float *partial = static_cast<float *>(workspace);
   return by_dim_bits(dim, polar_bits, [&](auto d, auto pb) {
     constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
-    if (nchunks > 0) {
-      const auto kernel = nv <= kWvFew ? qjl_wv_partial_kernel<D, PB, kWvFew> : qjl_wv_partial_kernel<D, PB, kWvChunk>;
-      hipLaunchKernelGGL(kernel, dim3((unsigned)nchunks, (unsigned)((nq + kWvQueries - 1) / kWvQueries)),
-                         dim3(4 * D), 0, stream, polar_packed, polar_scales, nv, nq, weights, partial, k);
+    const auto kernel = nv <= kWvFew ? qjl_wv_partial_kernel<D, PB, kWvFew> : qjl_wv_partial_kernel<D, PB, kWvChunk>;
+    constexpr int kMost = (1 << 29) / D;  // chunks: fewer than 2^32 lanes a launch
+    for (int c = 0; c < nchunks; c += kMost) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(nchunks - c, kMost), (unsigned)((nq + kWvQueries - 1) / kWvQueries)),
+                         dim3(4 * D), 0, stream, polar_packed, polar_scales, nv, nq, weights, partial, c, nchunks, k);
       int rc2 = tqh::check_launch("qjl_wv_partial_kernel");
       if (rc2) return rc2;
     }
