@@ -841,11 +841,14 @@ extern "C" int tq_qjl_scores(const float *ctx, size_t num_queries, const uint8_t
   const long long nq = (long long)num_queries, nk = (long long)num_keys;
   return by_dim_bits(dim, polar_bits, [&](auto d, auto pb) {
     constexpr int D = decltype(d)::value, PB = decltype(pb)::value;
-    if (nq <= kTableQueries<D, PB> && nk >= kTableKeys<D, PB> + kTableKeysPerQuery<D> * (nq - 1)) {
+    // (a lane a key, and a launch holds fewer than 2^32)
+    if (nq <= kTableQueries<D, PB> && nk >= kTableKeys<D, PB> + kTableKeysPerQuery<D> * (nq - 1) &&
+        nk <= (1ll << 32) - 2 * kBlock) {
       constexpr int QB = kTableBlockQueries<PB>;
       hipLaunchKernelGGL((qjl_scores_table_kernel<D, PB>),
-                         dim3((unsigned)((nk + kBlock - 1) / kBlock), (unsigned)((nq + QB - 1) / QB)), dim3(kBlock), 0, stream, ctx, nq, polar_packed, polar_scales,
-                         reinterpret_cast<const uint32_t *>(signs), residual_norms, nk, scores, k);
+                         dim3((unsigned)((nk + kBlock - 1) / kBlock), (unsigned)((nq + QB - 1) / QB)), dim3(kBlock), 0,
+                         stream, ctx, nq, polar_packed, polar_scales, reinterpret_cast<const uint32_t *>(signs),
+                         residual_norms, nk, scores, k);
       return tqh::check_launch("qjl_scores_table_kernel");
     }
     const long long qblocks = (nq + 15) / 16, tiles = (nk + 15) / 16 * qblocks;
