@@ -257,6 +257,24 @@ def test_l2norm_and_mixed_codec_bit_exact(tq, bits, outlier, norm, dtype):
     assert (_host(y).view(np.uint32) == ry.view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("d,bits,dtype,skew", [(64, 3, "bf16", 0), (64, 4, "f16", 1), (128, 4, "f16", 0),
+                                               (128, 3, "bf16", 1), (256, 3, "f32", 0), (256, 4, "bf16", 0)])
+def test_l2norm_append_stores_the_codecs_records(tq, d, bits, dtype, skew):
+    """The append's own quantizer against the codec's, keys and values; skew: they start one element past 16 bytes."""
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    h, t, norm = 3, 21, tq.QuantNormMode.L2Norm
+    g = torch.Generator(device="cuda").manual_seed(d + bits)
+    k, v = ((torch.randn((h * t * d + 1,), generator=g, device="cuda") * 3).to(dt)[skew:skew + h * t * d].view(1, h, t, d)
+            for _ in range(2))
+    cache = tq.TqCache(tq.CacheConfig(bits=bits, head_dim=d, num_kv_heads=h, num_layers=1, norm_mode=norm,
+                                      outlier_blocks=0))
+    cache.prefill(0, k, v, torch.zeros((1, h, 1, d), dtype=dt, device="cuda"))
+    ki, ks, vi, vs = cache.read_layer(0)
+    for x, p, s in ((k, ki, ks), (v, vi, vs)):
+        rp, rs = tq.polar_quantize(x.reshape(-1, d).clone(), bits, 0, norm)
+        assert torch.equal(p.reshape(rp.shape), rp) and torch.equal(s.reshape(rs.shape), rs)
+
+
 @pytest.mark.parametrize("kind,bits", [("pqo", 3), ("pq", 4), ("tq", 3), ("tq", 4)])
 def test_l2norm_caches_decode(tq, kind, bits):
     hkv, hq, t = 8, 16, 1200
